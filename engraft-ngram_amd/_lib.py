@@ -126,6 +126,19 @@ class EgGemmF32Operands(ctypes.Structure):
     ]
 
 
+class EgF16Source(ctypes.Structure):
+    """eg_f16_source"""
+
+    _fields_ = [("x", c_void_p), ("cols", c_int64), ("row_stride", c_int64), ("col_stride", c_int64)]
+
+
+class EgF16Matrix(ctypes.Structure):
+    """eg_f16_matrix"""
+
+    _fields_ = [("src", EgF16Source * 2), ("n_src", c_int32), ("rows", c_int64), ("planes", c_void_p),
+                ("exps", c_void_p)]
+
+
 # name -> (restype, argtypes); every symbol the header declares.
 SIGNATURES = {
     "eg_last_error": (c_char_p, []),
@@ -166,6 +179,11 @@ SIGNATURES = {
     "eg_gemm_bf16x6": (c_int32, [POINTER(EgGemmOperands), POINTER(EgGemmOperands), c_int32, c_int64, c_int64,
                                  c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int32, c_int32, c_void_p, c_int64,
                                  c_void_p]),
+    "eg_f16_planes_bytes": (c_int64, [c_int64, c_int64]),
+    "eg_f16_exps_count": (c_int64, [c_int64]),
+    "eg_split_f16": (c_int32, [POINTER(EgF16Matrix), c_void_p]),
+    "eg_gemm_f16x3": (c_int32, [POINTER(EgF16Matrix), POINTER(EgF16Matrix), POINTER(EgF16Matrix), c_void_p, c_int64,
+                                c_void_p, c_int64, c_void_p, c_int64, c_void_p]),
     "eg_forward_decode": (c_int32, [c_int32, POINTER(EgHashSpec), POINTER(EgTable), POINTER(EgOverlay), c_void_p,
                                     c_int64, c_int32, c_void_p, c_void_p, c_void_p, c_void_p]),
     "eg_forward_timed": (c_int32, [c_int32, POINTER(EgHashSpec), POINTER(EgTable), POINTER(EgOverlay), c_void_p,

@@ -61,6 +61,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -69,6 +70,7 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kGroupM = 8;
@@ -215,6 +217,19 @@ __device__ inline Work tile_work(const Plan& p, int logical, int64_t kv0, int64_
   return w;
 }
 
+// An output's value from its sum: the sum itself ...
+struct NoScale {
+  __device__ float operator()(float v, int, int64_t, int64_t) const { return v; }
+};
+// ... or the sum times the powers of two its operands' rows were divided by.
+struct RowScale {
+  const int32_t* a;      // exponent of A's row
+  const int32_t* b[2];   // of B's row, per column group
+  __device__ float operator()(float v, int grp, int64_t row, int64_t col) const {
+    return ldexpf(v, a[row] + b[grp][col]);
+  }
+};
+
 // Range s of the last round's (tile, K step) units: [U s / G, U (s + 1) / G).
 __device__ inline int64_t sk_start(const Plan& p, int64_t s) { return p.sk_units * s / p.sk_groups; }
 
@@ -222,10 +237,11 @@ __device__ inline int64_t sk_start(const Plan& p, int64_t s) { return p.sk_units
 // 8 (r / 4) + 4 (l / 32) + r % 4; wavefront (wm, wn) holds TI x TJ such
 // tiles, the block of 32 TI x 32 TJ outputs at (32 TI wm, 32 TJ wn) of the
 // tile.  A whole tile goes to C (bounded by m and n, added to when
-// accumulating); a piece to its BM x BN workspace slot.
-template <int BM, int BN, int TI, int TJ>
+// accumulating); a piece to its BM x BN workspace slot.  `scale` gives an
+// output its value from the sum (NoScale: the sum itself); pieces keep sums.
+template <int BM, int BN, int TI, int TJ, typename Scale>
 __device__ inline void store_acc(const Plan& p, const Work& w, const f32x16 (&acc)[TI][TJ], int wm, int wn,
-                                 int lane) {
+                                 int lane, const Scale& scale) {
   // the store addresses depend on the lane only; an opaque copy of it keeps the
   // compiler from computing them once ahead of a loop over tiles and holding
   // them (in scratch) across the K loops
@@ -256,7 +272,8 @@ __device__ inline void store_acc(const Plan& p, const Work& w, const f32x16 (&ac
         const int64_t row = w.m0 + r0 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
         if (row < p.m && col < n_grp) {
           float* q = out + row * ld + col;
-          *q = p.accumulate ? *q + acc[i][j][r] : acc[i][j][r];
+          const float v = scale(acc[i][j][r], w.grp, row, col);
+          *q = p.accumulate ? *q + v : v;
         }
       }
     }
@@ -530,7 +547,7 @@ __device__ inline void x3_tile(const GemmArgs& args, const Work& w, __bf16* lds)
     else  // PR0 4, PR1 2: segment 1 runs passes 1 and 2 of the four (lo*hi, hi*lo)
       seg_steps(s, PassSet<4, true>{}, s ? 0x6u : 0xfu);
   }
-  store_acc<BM, BN, TI, TJ>(p, w, acc, wave / WNW, wave % WNW, lane);
+  store_acc<BM, BN, TI, TJ>(p, w, acc, wave / WNW, wave % WNW, lane, NoScale{});
 }
 
 template <int BM, int BN, int WMW, int WNW, int PR>
@@ -654,7 +671,7 @@ __device__ inline void f32_tile(const F32Args& args, const Work& w, float* ldsf)
     }
     __builtin_amdgcn_s_barrier();  // the ring is refilled by the next segment or tile
   }
-  store_acc<BM, BN, 2, 2>(p, w, acc, wm, wn, lane);
+  store_acc<BM, BN, 2, 2>(p, w, acc, wm, wn, lane, NoScale{});
 }
 
 // gemm_f32 over the walk.  The stores' lane addresses are recomputed for
@@ -666,10 +683,404 @@ __global__ __launch_bounds__(BM * BN / 64) void gemm_f32_kernel(const F32Args ar
   EG_GEMM_WALK(f32_tile<BM, BN>(args, w, ldsf))
 }
 
+// gemm_h3_kernel (eg_gemm_f16x3): fp32 accuracy from three products on the
+// fp16 matrix cores; 378 us for the PLE key + value of 2,048 positions, its
+// operand's split and the marked rows' check included, against 691 us for the
+// six bf16 products (bound by the matrix cores and their operands' path
+// through LDS, as gemm_x3_kernel).  Every row of an operand is scaled by a power of two that
+// puts its largest magnitude in [2^14, 2^15) and split into hi = rne16(x) and
+// lo = rne16(x - hi): 22 significand bits where the element is at least
+// 2^-18 of the row's largest, an absolute 2^-40 of it below.  C = hi*hi +
+// hi*lo + lo*hi in fp32, scaled back when it is stored (RowScale); the dropped
+// lo*lo is at most 2^-22 of |a||b|.  Half the matrix work of the six bf16
+// products (gemm_x6_kernel) and four planes loaded in place of its eight, and
+// fewer fp32 additions: its error against float64 is no larger (2048 x 10240 x
+// 2560 of N(0, 1): 5.3e-7 in the 2-norm, against 8.3e-7 for the six products
+// and for gemm_f32_kernel).  Rows the planes do not hold (one value far above
+// the rest, an infinity, a NaN) are marked by the split and their outputs
+// computed by gemm_wide_kernel instead.
+//
+// Planes are fragment-major: 32 rows x 32 k are one 4 KB run, [k half of 16]
+// [hi, lo][lane][8 values], lane l holding row l % 32 and k 8 (l / 32) .. + 7 of
+// its half: what one MFMA operand register set takes.  A direct-to-LDS load
+// then moves 1 KB of consecutive memory (eight whole lines, where the row-major
+// planes gave sixteen half lines), a fragment read is 64 consecutive 16-byte
+// slots (no bank conflicts, no swizzle), and the load addresses are scalar
+// but for the lane's 16 bytes.
+struct H3Seg {
+  const char* a;
+  const char* b[2];       // per column group
+  int64_t a_blk;          // bytes of one 32-row block (its K steps x 4 KB), both operands
+  int64_t a_blocks, b_blocks[2];
+  int64_t ktiles;         // K / 32
+};
+
+struct H3Args {
+  H3Seg seg[1];
+  int n_seg;
+  Plan p;
+  RowScale scale;
+};
+
+constexpr int kFragBytes = 1024;  // one operand fragment, 64 lanes x 8 fp16
+constexpr int kStepBytes = 4 * kFragBytes;  // 32 rows x 32 k, both planes
+
+// The steps of x3_tile (its software pipeline and barriers) over
+// fragment-major fp16 planes.
+template <int BM, int BN, int WMW, int WNW>
+__device__ inline void h3_tile(const H3Args& args, const Work& w, char* lds) {
+  constexpr int NW = WMW * WNW, TI = BM / WMW / 32, TJ = BN / WNW / 32;
+  constexpr int AB = BM / 32, BB = BN / 32;          // 32-row blocks of a stage
+  constexpr int LPW = 4 * (AB + BB) / NW;            // 1 KB loads per wavefront per stage
+  constexpr int STAGE = (AB + BB) * kStepBytes;
+  static_assert((AB + BB) % NW == 0, "whole blocks per wavefront");
+  const Plan& p = args.p;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int uwave = __builtin_amdgcn_readfirstlane(wave);
+  const int wm = uwave / WNW, wn = uwave % WNW;
+  const H3Seg& sg = args.seg[0];
+  const int64_t lo = w.kv0, hi = w.kv1;
+
+  f32x16 acc[TI][TJ];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+  if (lo < hi) {
+    // this wavefront's loads: blocks uwave LB .. + LB - 1 of the stage (A's, then
+    // B's), four 1 KB pieces each.  Blocks past the last re-read the last: their
+    // products only reach outputs that are not stored.
+    constexpr int LB = LPW / 4;
+    const char* src[LB];
+#pragma unroll
+    for (int j = 0; j < LB; ++j) {
+      const int blk = uwave * LB + j;
+      const bool is_a = blk < AB;
+      const int64_t g = is_a ? w.m0 / 32 + blk : w.n0 / 32 + blk - AB;
+      const int64_t last = (is_a ? sg.a_blocks : sg.b_blocks[w.grp]) - 1;
+      src[j] = (is_a ? sg.a : sg.b[w.grp]) + (g < last ? g : last) * sg.a_blk;
+    }
+    const uint32_t lane16 = (uint32_t)lane * 16;
+    auto piece = [&](int64_t kt, int j, auto sub) {  // the offset advances the global and the LDS address alike
+      __builtin_amdgcn_global_load_lds(
+          (const void*)(src[j] + kt * kStepBytes + lane16),
+          (__attribute__((address_space(3))) void*)(lds + (kt & 1) * STAGE + (uwave * LB + j) * kStepBytes), 16,
+          decltype(sub)::value * kFragBytes, 0);
+    };
+    auto issue_one = [&](int64_t kt, int q) {
+      if ((q & 3) == 0) piece(kt, q >> 2, std::integral_constant<int, 0>{});
+      if ((q & 3) == 1) piece(kt, q >> 2, std::integral_constant<int, 1>{});
+      if ((q & 3) == 2) piece(kt, q >> 2, std::integral_constant<int, 2>{});
+      if ((q & 3) == 3) piece(kt, q >> 2, std::integral_constant<int, 3>{});
+    };
+    auto issue = [&](int64_t kt) {
+#pragma unroll
+      for (int j = 0; j < LPW; ++j) issue_one(kt, j);
+    };
+    f16x8 ah[2][TI], al[2][TI], bh[2][TJ], bl[2][TJ];
+    auto read = [&](int f, int64_t kt, int ks) {
+      const char* st = lds + (kt & 1) * STAGE + ks * 2 * kFragBytes + lane16;
+#pragma unroll
+      for (int i = 0; i < TI; ++i) {
+        ah[f][i] = *(const f16x8*)(st + (wm * TI + i) * kStepBytes);
+        al[f][i] = *(const f16x8*)(st + (wm * TI + i) * kStepBytes + kFragBytes);
+      }
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) {
+        bh[f][j] = *(const f16x8*)(st + (AB + wn * TJ + j) * kStepBytes);
+        bl[f][j] = *(const f16x8*)(st + (AB + wn * TJ + j) * kStepBytes + kFragBytes);
+      }
+    };
+    // pass 0: lo*hi, 1: hi*lo, 2: hi*hi
+    auto one = [&](int f, int pass, int i, int j) {
+      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(pass == 0 ? al[f][i] : ah[f][i],
+                                                          pass == 1 ? bl[f][j] : bh[f][j], acc[i][j], 0, 0, 0);
+    };
+    auto mfma = [&](int f, int pass) {
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) one(f, pass, i, j);
+    };
+    issue(lo);
+    if (lo + 1 < hi) {
+      issue(lo + 1);
+      wait_vm<LPW>();  // this wavefront's part of the first step is in LDS
+    } else {
+      wait_vm<0>();
+    }
+    __builtin_amdgcn_s_barrier();
+    read(0, lo, 0);
+    for (int64_t kt = lo; kt + 1 < hi; ++kt) {
+      mfma(0, 0);
+      __builtin_amdgcn_sched_barrier(0);  // the reads stay between the passes
+      read(1, kt, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      mfma(0, 1);
+      mfma(0, 2);
+      __builtin_amdgcn_sched_barrier(0);
+      // step kt + 1 is in LDS and step kt in registers, every wavefront's after the barrier
+      wait_vm<0>();
+      wait_lgkm0();
+      __builtin_amdgcn_s_barrier();
+      const bool ld = kt + 2 < hi;
+#pragma unroll
+      for (int t = 0; t < 3 * TI * TJ; ++t) {
+        one(1, t / (TI * TJ), (t % (TI * TJ)) / TJ, t % TJ);
+        if (t == TI * TJ - 1) {
+          __builtin_amdgcn_sched_barrier(0);
+          read(0, kt + 1, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if ((t + 1) % 2 == 0 && (t + 1) / 2 - 1 < LPW) {
+          __builtin_amdgcn_sched_barrier(0);
+          if (ld) issue_one(kt + 2, (t + 1) / 2 - 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+    mfma(0, 0);
+    read(1, hi - 1, 1);
+    mfma(0, 1);
+    mfma(0, 2);
+#pragma unroll
+    for (int pass = 0; pass < 3; ++pass) mfma(1, pass);
+    __builtin_amdgcn_s_barrier();  // the ring is refilled by the next tile
+  }
+  store_acc<BM, BN, TI, TJ>(p, w, acc, wm, wn, lane, args.scale);
+}
+
+template <int BM, int BN, int WMW, int WNW>
+__global__ __launch_bounds__(WMW * WNW * 64) void gemm_h3_kernel(const H3Args args) {
+  extern __shared__ __attribute__((aligned(16))) char ldsh[];
+  EG_GEMM_WALK((h3_tile<BM, BN, WMW, WNW>(args, w, ldsh)))
+}
+
+// The split of eg_gemm_f16x3's operands (eg_split_f16): exponents, marks and
+// fragment-major planes of a matrix given as one or two sources side by side
+// along K (each padded with zeros to a multiple of 32).
+struct F16Src {
+  const float* x;
+  int64_t cols, row_stride, col_stride;
+};
+
+struct SplitF16Args {
+  F16Src src[2];
+  int64_t chunks[2];      // 8-value chunks of each source, padding included
+  int64_t rows, blk;      // blk: bytes of a 32-row block
+  char* planes;
+  int32_t* exps;          // [rows rounded up to 32]
+  int32_t* wide;          // per 8 rows: any row marked
+};
+
+// A row is marked when more than 1 / kWideShare of its values are nonzero and
+// more than 2^24 below the largest of their source's part of the row (the
+// split's absolute 2^-40 of the row's largest is then 2^-16 of each, and such
+// values count for something: beside them, one huge value), when its largest
+// is not finite, or when that is so small (below 2^-87) that the scale would
+// leave fp32's range.  Fewer small values are left to the planes, since random
+// rows have some near zero; and so is a source far below the other, whose
+// products add less than the rounding of the other's (either rule marked rows
+// of the block's own gradients, and computing those again cost its backward
+// 0.1 to 5 ms).
+constexpr int kWideLow = 40, kWideShare = 16;
+
+// A workgroup of 64 NW threads takes ROWS rows of one 32-row block (ROWS 8:
+// rows contiguous in memory, a wavefront covers 8 rows x 8 chunks, 256 bytes a
+// row; ROWS 32 with TRANS: columns contiguous, a wavefront covers 32 rows x 2
+// chunks, 128-byte runs) and all of K.  PER > 0: a thread's PER chunks stay in
+// registers between the row maximum and the split; PER 0: they are read
+// again.  Bound by HBM: 4 bytes read and 4 written a value.
+template <int ROWS, int NW, int PER, bool TRANS>
+__global__ __launch_bounds__(64 * NW) void split_f16_kernel(const SplitF16Args a) {
+  constexpr int CPW = 64 / ROWS;  // chunks a wavefront covers
+  __shared__ uint32_t s_max[2][NW][ROWS], s_low[NW][ROWS];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane % ROWS, cl = lane / ROWS;
+  const int64_t r0 = (int64_t)blockIdx.x * ROWS, row = r0 + r;
+  const bool live = row < a.rows;
+  const int64_t n_chunks = a.chunks[0] + a.chunks[1];
+
+  auto load = [&](int64_t c, float* v) {
+    const int s = c < a.chunks[0] ? 0 : 1;
+    const F16Src& src = a.src[s];
+    const int64_t k = (s ? c - a.chunks[0] : c) * 8;
+    const float* x = src.x + row * src.row_stride + k * src.col_stride;
+    if (!live || c >= n_chunks) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = 0.0f;
+    } else if (!TRANS && k + 8 <= src.cols && (src.row_stride & 3) == 0 && ((uintptr_t)src.x & 15) == 0) {
+      const float4 p = *(const float4*)x, q = *(const float4*)(x + 4);
+      v[0] = p.x, v[1] = p.y, v[2] = p.z, v[3] = p.w;
+      v[4] = q.x, v[5] = q.y, v[6] = q.z, v[7] = q.w;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = k + e < src.cols ? x[e * src.col_stride] : 0.0f;
+    }
+  };
+  uint32_t mxs[2] = {0, 0};  // per source
+  auto see = [&](int64_t c, const float* v) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) m = max(m, __float_as_uint(v[e]) & 0x7fffffffu);
+    if (c < a.chunks[0]) mxs[0] = max(mxs[0], m);
+    else mxs[1] = max(mxs[1], m);
+  };
+  float kept[PER > 0 ? PER : 1][8];
+  if constexpr (PER > 0) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) load((int64_t)(i * NW + wave) * CPW + cl, kept[i]);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) see((int64_t)(i * NW + wave) * CPW + cl, kept[i]);
+  } else {
+    for (int64_t c = wave * CPW + cl; c < n_chunks; c += 2 * NW * CPW) {
+      float v[2][8];
+      load(c, v[0]);
+      load(c + NW * CPW, v[1]);
+      see(c, v[0]);
+      see(c + NW * CPW, v[1]);
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+#pragma unroll
+    for (int o = 32; o >= ROWS; o >>= 1) mxs[s] = max(mxs[s], (uint32_t)__shfl_xor((int)mxs[s], o));
+    if (lane < ROWS) s_max[s][wave][r] = mxs[s];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < NW; ++q) {
+    mxs[0] = max(mxs[0], s_max[0][q][r]);
+    mxs[1] = max(mxs[1], s_max[1][q][r]);
+  }
+  const uint32_t mx = max(mxs[0], mxs[1]);
+  // out of the scale's range: no planes
+  const bool out = mx != 0 && ((mx >> 23) >= 255 || (mx >> 23) < kWideLow);
+  // the row times 2^(14 - e) has its largest magnitude in [2^14, 2^15)
+  const int ex = mx == 0 || out ? 14 : (int)(mx >> 23) - 127;
+  const float scale = __uint_as_float((uint32_t)(127 + 14 - ex) << 23);
+  // the bits of 2^-24 of each source's largest
+  const uint32_t low0 = mxs[0] > (24u << 23) ? mxs[0] - (24u << 23) : 0;
+  const uint32_t low1 = mxs[1] > (24u << 23) ? mxs[1] - (24u << 23) : 0;
+  uint32_t n_low = 0;
+  auto put = [&](int64_t c, const float* v) {
+    if (c >= n_chunks) return;
+    f16x8 hi, lo;
+    const uint32_t low = c < a.chunks[0] ? low0 : low1;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      n_low += (__float_as_uint(v[e]) & 0x7fffffffu) - 1 < low;  // zero wraps to the largest
+      const float x = out ? 0.0f : v[e] * scale;
+      hi[e] = (_Float16)x;
+      lo[e] = (_Float16)(x - (float)hi[e]);
+    }
+    char* o = a.planes + (row >> 5) * a.blk + (c >> 2) * kStepBytes + ((c >> 1) & 1) * 2 * kFragBytes +
+              ((row & 31) + 32 * (c & 1)) * 16;
+    *(f16x8*)o = hi;
+    *(f16x8*)(o + kFragBytes) = lo;
+  };
+  if constexpr (PER > 0) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) put((int64_t)(i * NW + wave) * CPW + cl, kept[i]);
+  } else {
+    for (int64_t c = wave * CPW + cl; c < n_chunks; c += 2 * NW * CPW) {
+      float v[2][8];
+      load(c, v[0]);
+      load(c + NW * CPW, v[1]);
+      put(c, v[0]);
+      put(c + NW * CPW, v[1]);
+    }
+  }
+#pragma unroll
+  for (int o = 32; o >= ROWS; o >>= 1) n_low += (uint32_t)__shfl_xor((int)n_low, o);
+  if (lane < ROWS) s_low[wave][r] = n_low;
+  __syncthreads();
+  if (wave != 0) return;
+  n_low = 0;
+#pragma unroll
+  for (int q = 0; q < NW; ++q) n_low += s_low[q][r];
+  const bool wide = out || (int64_t)n_low * kWideShare > a.src[0].cols + a.src[1].cols;
+  if (lane < ROWS && live) a.exps[row] = ex - 14;
+  const uint64_t any = __ballot(wide && lane < ROWS);
+  if (lane < ROWS / 8 && r0 + 8 * lane < a.rows) a.wide[r0 / 8 + lane] = (any >> (8 * lane) & 0xff) != 0;
+}
+
+// The outputs of marked rows, in fp32: a 64 x 64 tile with a marked row of A or
+// B is computed again from the fp32 operands (any strides), its K in chunks
+// of 16 whose sums are added up.  Without a marked row a workgroup reads the
+// marks and exits.
+struct WideArgs {
+  F16Src a[2], b[2][2];    // sources of A and of B per column group
+  const int32_t* wide[3];  // marks of A, B, B2
+  int n_src;
+  int64_t m, n[2];
+  float* c[2];
+  int64_t ldc[2];
+};
+
+__global__ __launch_bounds__(256) void gemm_wide_kernel(const WideArgs g) {
+  const int tid = threadIdx.x;
+  int any = 0;
+  const int64_t lens[3] = {g.m, g.n[0], g.n[1]};
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+    for (int64_t i = tid; i < (lens[q] + 7) / 8; i += 256) any |= g.wide[q][i];
+  if (!__syncthreads_or(any)) return;
+  __shared__ float sa[16][65], sb[16][65];
+  const int64_t tm_n = (g.m + 63) / 64, tn0 = (g.n[0] + 63) / 64, tiles = tm_n * (tn0 + (g.n[1] + 63) / 64);
+  const int ty = tid >> 4, tx = tid & 15;
+  for (int64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
+    const int64_t tn = t / tm_n;
+    const int grp = tn < tn0 ? 0 : 1;
+    const int64_t m0 = (t % tm_n) * 64, n0 = (grp ? tn - tn0 : tn) * 64;
+    int mark = 0;
+    if (tid < 8 && m0 + 8 * tid < g.m) mark = g.wide[0][m0 / 8 + tid];
+    if (tid >= 8 && tid < 16 && n0 + 8 * (tid - 8) < g.n[grp]) mark = g.wide[1 + grp][n0 / 8 + tid - 8];
+    if (!__syncthreads_or(mark)) continue;
+    float sum[4][4] = {};
+    for (int s = 0; s < g.n_src; ++s) {
+      const F16Src &xa = g.a[s], &xb = g.b[grp][s];
+      for (int64_t k0 = 0; k0 < xa.cols; k0 += 16) {
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int id = tid + 256 * e, r = id >> 4, k = id & 15;
+          const bool in = k0 + k < xa.cols;
+          sa[k][r] = in && m0 + r < g.m ? xa.x[(m0 + r) * xa.row_stride + (k0 + k) * xa.col_stride] : 0.0f;
+          sb[k][r] = in && n0 + r < g.n[grp] ? xb.x[(n0 + r) * xb.row_stride + (k0 + k) * xb.col_stride] : 0.0f;
+        }
+        __syncthreads();
+        float part[4][4] = {};
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) part[i][j] = fmaf(sa[k][ty + 16 * i], sb[k][tx + 16 * j], part[i][j]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) sum[i][j] += part[i][j];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int64_t row = m0 + ty + 16 * i, col = n0 + tx + 16 * j;
+        if (row < g.m && col < g.n[grp]) g.c[grp][row * g.ldc[grp] + col] = sum[i][j];
+      }
+    __syncthreads();
+  }
+}
+
 // C (+)= the sum of a last-round tile's pieces, in K order: BM BN / 1024
 // blocks a tile, each thread four consecutive columns of one row.
-template <int BM, int BN>
-__global__ __launch_bounds__(256) void piece_sum_kernel(const Plan p) {
+template <int BM, int BN, typename Scale>
+__global__ __launch_bounds__(256) void piece_sum_kernel(const Plan p, const Scale scale) {
   constexpr int kBlocks = BM * BN / 1024;
   const int q = blockIdx.x / kBlocks;
   const int e = (blockIdx.x % kBlocks) * 256 + threadIdx.x;  // float4 of the BM x BN tile
@@ -694,7 +1105,10 @@ __global__ __launch_bounds__(256) void piece_sum_kernel(const Plan p) {
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     const int64_t col = col0 + t;
-    if (col < n_grp) out[col] = p.accumulate ? out[col] + vv[t] : vv[t];
+    if (col < n_grp) {
+      const float x = scale(vv[t], grp, row, col);
+      out[col] = p.accumulate ? out[col] + x : x;
+    }
   }
 }
 
@@ -702,8 +1116,8 @@ __global__ __launch_bounds__(256) void piece_sum_kernel(const Plan p) {
 // ranges of gemm_f32_kernel computed: the ranges meeting the tile, in
 // increasing order (a tile one range covers whole was stored directly).
 // BM BN / 1024 blocks a tile, four columns a thread.
-template <int BM, int BN>
-__global__ __launch_bounds__(256) void sk_sum_kernel(const Plan p) {
+template <int BM, int BN, typename Scale>
+__global__ __launch_bounds__(256) void sk_sum_kernel(const Plan p, const Scale scale) {
   constexpr int kBlocks = BM * BN / 1024;
   const int q = blockIdx.x / kBlocks;  // last-round tile
   const int e = (blockIdx.x % kBlocks) * 256 + threadIdx.x;
@@ -743,7 +1157,10 @@ __global__ __launch_bounds__(256) void sk_sum_kernel(const Plan p) {
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     const int64_t col = col0 + t;
-    if (col < n_grp) out[col] = p.accumulate ? out[col] + vv[t] : vv[t];
+    if (col < n_grp) {
+      const float x = scale(vv[t], grp, row, col);
+      out[col] = p.accumulate ? out[col] + x : x;
+    }
   }
 }
 
@@ -878,10 +1295,10 @@ int64_t workspace_size(const Shape& sh, int64_t m, int64_t n, int64_t n2, int64_
 
 // The part of both entry points after their operands are checked: the plan,
 // the LDS attribute, the launch and the pieces' sum.
-template <int BM, int BN, typename Args>
+template <int BM, int BN, typename Args, typename Scale = NoScale>
 int launch_gemm(const Shape& sh, void (*kernel)(const Args), const char* name, Args& g, int64_t m, int64_t n,
                 int64_t n2, float* c, int64_t ldc, float* c2, int64_t ldc2, int32_t accumulate, int32_t k_slices,
-                void* workspace, int64_t workspace_bytes, void* stream) {
+                void* workspace, int64_t workspace_bytes, void* stream, const Scale& scale = Scale{}) {
   EG_CHECK_ARG(m >= 0 && n >= 0 && n2 >= 0 && k_slices >= 0, "m=%lld n=%lld n2=%lld k_slices=%d", (long long)m,
                (long long)n, (long long)n2, k_slices);
   EG_CHECK_ARG(n == 0 || (c != nullptr && ldc >= n), "c / ldc");
@@ -889,7 +1306,8 @@ int launch_gemm(const Shape& sh, void (*kernel)(const Args), const char* name, A
   if (m == 0 || n + n2 == 0) return 0;
   Plan& p = g.p;
   p.kt0 = g.n_seg > 0 ? g.seg[0].ktiles : 0;
-  p.kt_total = p.kt0 + (g.n_seg > 1 ? g.seg[1].ktiles : 0);
+  p.kt_total = p.kt0;
+  for (int s = 1; s < g.n_seg; ++s) p.kt_total += g.seg[s].ktiles;
   int64_t tiles = 0;
   PiecePlan pp{};
   int rc = plan_for(sh, m, n, n2, p.kt_total, k_slices, &tiles, &pp);
@@ -940,10 +1358,10 @@ int launch_gemm(const Shape& sh, void (*kernel)(const Args), const char* name, A
   if (rc != 0 || pp.dp == tiles) return rc;
   const dim3 sum_grid((unsigned)((tiles - pp.dp) * (BM * BN / 1024)));
   if (pp.sk_groups > 0) {
-    hipLaunchKernelGGL((sk_sum_kernel<BM, BN>), sum_grid, dim3(256), 0, st, p);
+    hipLaunchKernelGGL((sk_sum_kernel<BM, BN, Scale>), sum_grid, dim3(256), 0, st, p, scale);
     return launch_status("sk_sum_kernel");
   }
-  hipLaunchKernelGGL((piece_sum_kernel<BM, BN>), sum_grid, dim3(256), 0, st, p);
+  hipLaunchKernelGGL((piece_sum_kernel<BM, BN, Scale>), sum_grid, dim3(256), 0, st, p, scale);
   return launch_status("piece_sum_kernel");
 }
 
@@ -1127,6 +1545,136 @@ int eg_gemm_f32(const eg_gemm_f32_operands* ops, int32_t n_seg, int64_t m, int64
   }
   return launch_gemm<kF32BM, kF32BN>(kF32Shape, gemm_f32_kernel<kF32BM, kF32BN>, "gemm_f32_kernel", g, m, n, n2,
                                      c, ldc, c2, ldc2, accumulate, k_slices, workspace, workspace_bytes, stream);
+}
+
+}  // extern "C"
+
+namespace eg {
+namespace {
+// One operand of eg_gemm_f16x3, checked: its sources' total of 32-wide K steps.
+int f16_matrix(const eg_f16_matrix* x, const char* what, int64_t* steps) {
+  EG_CHECK_ARG(x != nullptr && x->rows >= 0 && x->n_src >= 1 && x->n_src <= 2, "%s: rows / n_src", what);
+  *steps = 0;
+  for (int s = 0; s < x->n_src; ++s) {
+    const eg_f16_source& o = x->src[s];
+    EG_CHECK_ARG(o.cols >= 0 && o.row_stride >= 0 && o.col_stride >= 0, "%s: source %d", what, s);
+    EG_CHECK_ARG(o.x != nullptr || o.cols == 0 || x->rows == 0, "%s: source %d is NULL", what, s);
+    *steps += (o.cols + 31) / 32;
+  }
+  EG_CHECK_ARG(x->rows == 0 || *steps == 0 ||
+                   (x->planes != nullptr && ((uintptr_t)x->planes & 15) == 0 && x->exps != nullptr),
+               "%s: planes (16-byte aligned) and exps", what);
+  return EG_OK;
+}
+
+F16Src f16_src(const eg_f16_matrix* x, int s) {
+  return s < x->n_src ? F16Src{x->src[s].x, x->src[s].cols, x->src[s].row_stride, x->src[s].col_stride}
+                      : F16Src{nullptr, 0, 0, 0};
+}
+
+int64_t blocks32(int64_t rows) { return (rows + 31) / 32; }
+}  // namespace
+}  // namespace eg
+
+extern "C" {
+
+int64_t eg_f16_planes_bytes(int64_t rows, int64_t k) { return rows < 0 || k < 0 ? -1 : eg::blocks32(rows) * ((k + 31) / 32) * eg::kStepBytes; }
+
+int64_t eg_f16_exps_count(int64_t rows) { return rows < 0 ? -1 : eg::blocks32(rows) * 36; }
+
+int eg_split_f16(const eg_f16_matrix* x, void* stream) {
+  using namespace eg;
+  int64_t steps = 0;
+  const int rc = f16_matrix(x, "x", &steps);
+  if (rc != EG_OK) return rc;
+  if (x->rows == 0 || steps == 0) return 0;
+  SplitF16Args a{};
+  bool trans = false;
+  for (int s = 0; s < 2; ++s) {
+    a.src[s] = f16_src(x, s);
+    a.chunks[s] = (a.src[s].cols + 31) / 32 * 4;
+    trans = trans || (a.src[s].cols > 0 && a.src[s].col_stride != 1);
+  }
+  a.rows = x->rows;
+  a.blk = steps * kStepBytes;
+  a.planes = (char*)x->planes;
+  a.exps = x->exps;
+  a.wide = x->exps + blocks32(x->rows) * 32;
+  const int64_t blocks = trans ? blocks32(x->rows) : 4 * blocks32(x->rows);
+  EG_CHECK_ARG(blocks < (1LL << 31), "too many rows");
+  const int64_t chunks = 4 * steps;
+  hipStream_t st = (hipStream_t)stream;
+  const dim3 grid((unsigned)blocks);
+  // K kept in registers where it fits a thread's 80 (rows) or 48 (columns;
+  // 1,024 threads have 128 registers each, and 64 values spilled) values
+  if (trans) {
+    if (chunks <= 6 * 16 * 2)
+      hipLaunchKernelGGL((split_f16_kernel<32, 16, 6, true>), grid, dim3(1024), 0, st, a);
+    else
+      hipLaunchKernelGGL((split_f16_kernel<32, 16, 0, true>), grid, dim3(1024), 0, st, a);
+  } else {
+    if (chunks <= 10 * 4 * 8)
+      hipLaunchKernelGGL((split_f16_kernel<8, 4, 10, false>), grid, dim3(256), 0, st, a);
+    else
+      hipLaunchKernelGGL((split_f16_kernel<8, 4, 0, false>), grid, dim3(256), 0, st, a);
+  }
+  return launch_status("split_f16_kernel");
+}
+
+int eg_gemm_f16x3(const eg_f16_matrix* a, const eg_f16_matrix* b, const eg_f16_matrix* b2, float* c, int64_t ldc,
+                  float* c2, int64_t ldc2, void* workspace, int64_t workspace_bytes, void* stream) {
+  using namespace eg;
+  const eg_f16_matrix none{};
+  int64_t ka = 0, kb = 0, kb2 = 0;
+  int rc = f16_matrix(a, "a", &ka);
+  if (rc == EG_OK) rc = f16_matrix(b, "b", &kb);
+  if (rc == EG_OK && b2 != nullptr) rc = f16_matrix(b2, "b2", &kb2);
+  if (rc != EG_OK) return rc;
+  const eg_f16_matrix* second = b2 != nullptr ? b2 : &none;
+  for (int s = 0; s < 2; ++s)
+    EG_CHECK_ARG(f16_src(a, s).cols == f16_src(b, s).cols && (b2 == nullptr || f16_src(a, s).cols == f16_src(b2, s).cols),
+                 "source %d: a and b must have the same k", s);
+  const int64_t m = a->rows, n = b->rows, n2 = second->rows;
+  if (m == 0 || n + n2 == 0) return 0;
+  H3Args g{};
+  if (ka > 0) {
+    H3Seg& sg = g.seg[0];
+    sg.a = (const char*)a->planes;
+    sg.b[0] = (const char*)b->planes;
+    sg.b[1] = (const char*)second->planes;
+    sg.a_blk = ka * kStepBytes;
+    sg.a_blocks = blocks32(m);
+    sg.b_blocks[0] = blocks32(n);
+    sg.b_blocks[1] = blocks32(n2);
+    sg.ktiles = ka;
+    g.n_seg = 1;
+  }
+  g.scale = RowScale{a->exps, {b->exps, second->exps}};
+  EG_CHECK_ARG(ka > 0, "k must be positive");
+  rc = launch_gemm<kX3BM, kX3BN>(kX3Shape, gemm_h3_kernel<kX3BM, kX3BN, kX3WM, kX3WN>, "gemm_h3_kernel", g, m, n, n2,
+                                 c, ldc, c2, ldc2, 0, 0, workspace, workspace_bytes, stream, g.scale);
+  if (rc != EG_OK) return rc;
+  WideArgs w{};
+  for (int s = 0; s < 2; ++s) {
+    w.a[s] = f16_src(a, s);
+    w.b[0][s] = f16_src(b, s);
+    w.b[1][s] = f16_src(second, s);
+  }
+  w.n_src = a->n_src;
+  w.wide[0] = a->exps + blocks32(m) * 32;
+  w.wide[1] = b->exps + blocks32(n) * 32;
+  w.wide[2] = b2 != nullptr ? b2->exps + blocks32(n2) * 32 : nullptr;
+  w.m = m;
+  w.n[0] = n;
+  w.n[1] = n2;
+  w.c[0] = c;
+  w.c[1] = c2;
+  w.ldc[0] = ldc;
+  w.ldc[1] = ldc2;
+  const int64_t tiles = ((m + 63) / 64) * ((n + 63) / 64 + (n2 + 63) / 64);
+  hipLaunchKernelGGL(gemm_wide_kernel, dim3((unsigned)(tiles < 512 ? tiles : 512)), dim3(256), 0, (hipStream_t)stream,
+                     w);
+  return launch_status("gemm_wide_kernel");
 }
 
 }  // extern "C"

@@ -4,9 +4,10 @@ for ``PleWeights`` / ``ple_forward`` (``engraft/replica/layers.py:555-626``).
 Forward:
 
 * ``key = emb @ w_key^T`` and ``value = emb @ w_value^T`` in one launch: by
-  default (``gemm="bf16x6"``) on the bf16 matrix cores with fp32 accuracy
+  default (``gemm="bf16x6"``) on the 16-bit matrix cores with fp32 accuracy
   (``gemm_x6``: operands split into three bf16 planes, six products
-  accumulated in fp32), with ``gemm="fp32"`` of the ``gemm_f32`` kernel on
+  accumulated in fp32; or ``gemm_h3``: rows scaled and split into two fp16
+  planes, three products), with ``gemm="fp32"`` of the ``gemm_f32`` kernel on
   the fp32 matrix cores (fp32 products, as the reference's torch matmuls), or
   with ``gemm="bf16x3"`` of the ``gemm_x3`` kernel (hi + lo planes, three
   products: 16 mantissa bits per operand);
@@ -18,9 +19,10 @@ Forward:
 The result -- the output and the new history -- is differentiable in emb,
 hidden, the history and the weights.  The backward runs
 ``eg_ple_conv_backward`` and ``eg_ple_gate_backward`` on the forward's saved
-intermediates, then the projections' backward (one ``gemm_f32``, ``gemm_x3``
-or ``gemm_x6`` call over two K segments); when weights need gradients, also the
-two weight GEMMs (``gemm_f32`` with the positions as K) and
+intermediates, then the projections' backward (one ``gemm_f32``, ``gemm_x3``,
+``gemm_x6`` or ``gemm_h3`` call over two K segments); when weights need
+gradients, also the two weight GEMMs (``gemm_f32``, or ``gemm_h3`` under
+``"bf16x6"``, with the positions as K) and
 ``eg_ple_weight_grads`` for the norm and convolution weights.  The
 convolution takes 1..8 taps (the reference's blocks have 4; more raise
 ``ValueError``).  Only shapes beyond the HIP backward's limits (more than 4
@@ -37,6 +39,7 @@ GGUF, method for method as the reference's numpy replica.
 """
 from __future__ import annotations
 
+import ctypes
 import dataclasses
 
 import numpy as np
@@ -322,6 +325,84 @@ def gemm_x6(a, b, a2=None, b2=None, out: torch.Tensor | None = None, accumulate:
     return (out, out2) if n2 else out
 
 
+class HalfPlanes:
+    """An fp32 operand of :func:`gemm_h3` with its fp16 planes
+    (``eg_split_f16``): one matrix ``[rows, k]`` of any strides, or two with the
+    same rows taken side by side along ``k``.  ``of`` the fp32 tensors, which
+    the GEMM reads too; the planes do not keep them."""
+
+    def __init__(self, of: tuple):
+        lib = _lib.load()
+        self.shapes = tuple(tuple(x.shape) for x in of)
+        self.rows = of[0].shape[0]
+        self.kp = sum((x.shape[1] + 31) // 32 * 32 for x in of)
+        dev = of[0].device
+        self.planes = torch.empty(lib.eg_f16_planes_bytes(self.rows, self.kp), dtype=torch.uint8, device=dev)
+        self.exps = torch.empty(lib.eg_f16_exps_count(self.rows), dtype=torch.int32, device=dev)
+        _lib.call("eg_split_f16", ctypes.byref(self.operand(of)), _lib.stream_ptr(dev))
+
+    def operand(self, of: tuple) -> "_lib.EgF16Matrix":
+        m = _lib.EgF16Matrix()
+        for s, x in enumerate(of):
+            m.src[s] = _lib.EgF16Source(_lib.ptr(x), x.shape[1], x.stride(0), x.stride(1))
+        m.n_src, m.rows = len(of), self.rows
+        m.planes, m.exps = _lib.ptr(self.planes), _lib.ptr(self.exps)
+        return m
+
+
+class _HalfPlaneCache:
+    """``HalfPlanes`` of weights, kept between steps: an entry is used only for
+    the same tensor objects (weak references) with the same storage at the same
+    version counters, on the stream that filled it.  Planes made while a graph
+    is captured are not kept: they are filled when the graph replays."""
+
+    def __init__(self, size: int = 8):
+        self._entries: list = []
+        self._size = size
+
+    def get(self, ws: tuple, transposed: bool) -> HalfPlanes:
+        import weakref
+        key = (transposed, _lib.stream_ptr(ws[0].device), *((w.data_ptr(), w._version, w.shape, w.stride())
+                                                            for w in ws))
+        for refs, k, planes in self._entries:
+            if k == key and all(r() is w for r, w in zip(refs, ws)):
+                return planes
+        planes = HalfPlanes(tuple(w.T for w in ws) if transposed else ws)
+        if not torch.cuda.is_current_stream_capturing():
+            live = [e for e in self._entries if all(r() is not None for r in e[0])]
+            self._entries = live[-(self._size - 1):] + [(tuple(weakref.ref(w) for w in ws), key, planes)]
+        return planes
+
+
+_HALF = _HalfPlaneCache()
+
+
+def gemm_h3(a: tuple, b: tuple, b_n2: tuple | None = None, *, planes_b: HalfPlanes | None = None,
+            planes_b2: HalfPlanes | None = None):
+    """``sum_s a[s] @ b[s].T`` over one or two pairs of fp32 matrices (any
+    strides) with an fp32 matmul's accuracy on the fp16 matrix cores
+    (``eg_gemm_f16x3``: every row scaled by a power of two and split into two
+    fp16 planes, three products accumulated in fp32; rows beyond the planes'
+    range computed in fp32).  ``b_n2``: a second column group over the same
+    ``a``; the result is then a pair.  ``planes_b`` / ``planes_b2``: the planes
+    of ``b`` / ``b_n2`` where the caller keeps them."""
+    for name, side in (("b", b), ("b_n2", b_n2)):
+        if side is not None and [x.shape[1] for x in side] != [x.shape[1] for x in a]:
+            raise ValueError(f"gemm_h3: a and {name} must have the same k")
+    pa = HalfPlanes(a)
+    pb = planes_b if planes_b is not None else HalfPlanes(b)
+    pb2 = None if b_n2 is None else planes_b2 if planes_b2 is not None else HalfPlanes(b_n2)
+    dev = a[0].device
+    m, n, n2 = pa.rows, pb.rows, 0 if pb2 is None else pb2.rows
+    out = torch.empty((m, n), dtype=torch.float32, device=dev)
+    out2 = torch.empty((m, n2), dtype=torch.float32, device=dev) if pb2 is not None else None
+    _, ws, ws_bytes = _gemm_workspace(m, n, n2, pa.kp, None, dev, "eg_gemm_workspace_size")
+    _lib.call("eg_gemm_f16x3", ctypes.byref(pa.operand(a)), ctypes.byref(pb.operand(b)),
+              None if pb2 is None else ctypes.byref(pb2.operand(b_n2)), _lib.ptr(out), max(n, 1), _lib.ptr(out2),
+              max(n2, 1), _lib.ptr(ws), ws_bytes, _lib.stream_ptr(dev))
+    return out if pb2 is None else (out, out2)
+
+
 def _f32_operand(x: torch.Tensor, kp: int) -> torch.Tensor:
     """``x [rows, k]`` fp32 as eg_gemm_f32 reads it: unit column stride, row
     stride a multiple of 4, 16-byte aligned, ``k`` a multiple of 32; otherwise
@@ -388,25 +469,37 @@ def gemm_f32(a, b, a2=None, b2=None, out: torch.Tensor | None = None, accumulate
     return (out, out2) if n2 else out
 
 
+# gemm="bf16x6" runs gemm_h3 (no less accurate, half the matrix work) past this many
+# positions; up to here both stream the weights' planes and gemm_x6 has fewer
+# launches.  The forward of a call that is differentiated keeps gemm_x6: the
+# score's gradient goes as 1/sqrt|s|, so at a score near zero any other rounding
+# of the key moves the hidden, key and norm gradients by far more than its own
+# size (1e-4 at |s| 0.03).
+H3_MIN_ROWS = 64
+
 WGRAD_MAX_TAPS = 8  # eg_ple_weight_grads' built tap counts (1..8)
 
 
 def _weight_grad(d_y: torch.Tensor, x: torch.Tensor, w: torch.Tensor, gemm: str = "fp32") -> torch.Tensor:
     """``d_y^T x`` (``[out, T]`` x ``[T, in]``), the gradient of ``w`` in
-    ``y = x w^T``, with the positions as K (both operands transposed into
-    K-contiguous copies): on eg_gemm_f32, or with ``gemm="bf16x6"`` on
-    eg_gemm_bf16x6 (the same fp32 accuracy; bf16x3's 16-bit operands are kept
-    to the projections)."""
+    ``y = x w^T``, with the positions as K: on eg_gemm_f32 (both operands
+    transposed into K-contiguous copies), or with ``gemm="bf16x6"`` on
+    eg_gemm_f16x3 (the same fp32 accuracy, its split reading the transposes in
+    place; bf16x3's 16-bit operands are kept to the projections)."""
     if d_y.shape[0] == 0:
         return torch.zeros_like(w)
     if gemm == "bf16x6":
-        return gemm_x6(d_y.T, x.T)
+        return gemm_h3((d_y.T,), (x.T,))
     return gemm_f32(d_y.T, x.T)
 
 
-def _projection_backward(gemm: str, flat: list) -> torch.Tensor:
-    """``d_emb = sum d_i w_i`` over the (d_i, w_i^T) pairs in ``flat``, on the
+def _projection_backward(gemm: str, pairs: list) -> torch.Tensor:
+    """``d_emb = sum d_i w_i`` over the (d_i, w_i) in ``pairs``, on the
     forward's GEMM."""
+    if gemm == "bf16x6" and pairs[0][0].shape[0] > H3_MIN_ROWS:
+        ds, ws = zip(*pairs)
+        return gemm_h3(ds, tuple(w.T for w in ws), planes_b=_HALF.get(ws, True))
+    flat = [x for d, w in pairs for x in (d, _WT.get(w))]
     if gemm == "bf16x3":
         return gemm_x3(*flat, cache_b=True)
     if gemm == "bf16x6":
@@ -437,6 +530,9 @@ class _PleFn(torch.autograd.Function):
         wv32 = w_value.to(**f32)
         if gemm == "bf16x3":
             key, value = gemm_x3(SplitPlanes(emb32), wk32, cache_b=True, b_n2=wv32)
+        elif gemm == "bf16x6" and t_len > H3_MIN_ROWS and not any(ctx.needs_input_grad):
+            key, value = gemm_h3((emb32,), (wk32,), (wv32,), planes_b=_HALF.get((wk32,), False),
+                                 planes_b2=_HALF.get((wv32,), False))
         elif gemm == "bf16x6":
             key, value = gemm_x6(SplitPlanes(emb32, three=True), wk32, cache_b=True, b_n2=wv32)
         else:
@@ -553,10 +649,9 @@ class _PleFn(torch.autograd.Function):
         if need_emb:
             # the projections' backward, d_emb = d_key w_key + d_value w_value, as
             # products with the weights' transposes (kept between steps)
-            parts = [(d, _WT.get(w)) for d, w in ((d_key, wk32), (d_value, wv32)) if d is not None]
+            parts = [(d, w) for d, w in ((d_key, wk32), (d_value, wv32)) if d is not None]
             if parts:  # none: both factors detached, emb has no path to the output
-                flat = [x for part in parts for x in part]
-                d_emb = _projection_backward(ctx.gemm, flat).to(emb_dt)
+                d_emb = _projection_backward(ctx.gemm, parts).to(emb_dt)
         d_hist_in = d_full[:h0].reshape(h0, hc, n).to(hist_dt) if need_hist else None
         return (d_emb, d_hidden.to(hidden_dt) if d_hidden is not None else None, None, None, None, None, None, None,
                 d_hist_in, None, None, None, None, None)
@@ -590,10 +685,9 @@ class _PleFn(torch.autograd.Function):
                   _lib.ptr(d_key), _lib.ptr(d_value), _lib.ptr(d_hidden), _lib.ptr(d_s), st)
         d_emb = None
         if need_emb:
-            parts = [(d, _WT.get(w)) for d, w in ((d_key, wk32), (d_value, wv32)) if d is not None]
+            parts = [(d, w) for d, w in ((d_key, wk32), (d_value, wv32)) if d is not None]
             if parts:  # none: both factors detached, emb has no path to the output
-                flat = [x for part in parts for x in part]
-                d_emb = _projection_backward(ctx.gemm, flat).to(emb_dt)
+                d_emb = _projection_backward(ctx.gemm, parts).to(emb_dt)
         wdt = ctx.w_dtypes
         # the projection weights' gradients d_key^T emb and d_value^T emb on eg_gemm_f32
         # (K = the positions); a weight the detached factor cuts off keeps None
@@ -628,12 +722,13 @@ def ple_forward(emb: torch.Tensor, hidden: torch.Tensor, w: PleWeights, hist: to
     565-626``).  ``emb [T, n_embd]``, ``hidden [T, hc, n_embd]``, ``hist``
     ``[rows, hc, n_embd]`` (at most ``(K-1)*ple_ngram_size`` rows, empty at a
     sequence start); all on the device.  ``gemm`` picks the projections' GEMM:
-    ``"bf16x6"``, the default (``gemm_x6``: the bf16 matrix cores with fp32
-    accuracy, its error against float64 below both fp32 paths' and the
-    fastest of the three at that accuracy), ``"fp32"`` (``gemm_f32``: fp32
+    ``"bf16x6"``, the default (``gemm_x6`` or, past ``H3_MIN_ROWS`` positions of a
+    call without gradients and in the backward, ``gemm_h3``: the 16-bit matrix
+    cores with fp32 accuracy, both errors against float64 below the fp32
+    path's, and the fastest at that accuracy), ``"fp32"`` (``gemm_f32``: fp32
     products on the fp32 matrix cores, the reference's torch matmul
     arithmetic) or ``"bf16x3"`` (``gemm_x3``: 16 mantissa bits per operand,
-    about 1e-5 relative per projection, 1.7x faster than bf16x6)."""
+    about 1e-5 relative per projection)."""
     if gemm not in ("fp32", "bf16x3", "bf16x6"):
         raise ValueError(f"gemm must be 'fp32', 'bf16x3' or 'bf16x6', got {gemm!r}")
     hc = hparams.hc_mult

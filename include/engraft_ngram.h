@@ -36,7 +36,7 @@
  *   (+ _backward)    and the autograd of it          engraft/replica/layers.py:565-626
  *   eg_ple_rms, eg_ple_conv's other modes  PleReplica engraft/lens.py:221-385
  *   eg_split_bf16, eg_gemm_bf16x3, eg_gemm_f32 (+ _workspace_size),
- *   eg_split_bf16x6, eg_gemm_bf16x6
+ *   eg_split_bf16x6, eg_gemm_bf16x6, eg_split_f16, eg_gemm_f16x3
  *                    ple_forward's projections and their backward
  *                                                    engraft/replica/layers.py:594-606
  */
@@ -601,6 +601,50 @@ int64_t eg_gemm_f32_workspace_size(int64_t m, int64_t n, int64_t n2, int64_t k, 
 int eg_gemm_f32(const eg_gemm_f32_operands* ops, int32_t n_seg, int64_t m, int64_t n, int64_t n2, float* c,
                 int64_t ldc, float* c2, int64_t ldc2, int32_t accumulate, int32_t k_slices, void* workspace,
                 int64_t workspace_bytes, void* stream);
+
+/* Part of an operand of eg_gemm_f16x3: fp32 [rows, cols], element (r, k) at
+ * x[r * row_stride + k * col_stride] (a transposed matrix has row_stride 1). */
+typedef struct eg_f16_source {
+  const float* x;
+  int64_t cols;
+  int64_t row_stride;
+  int64_t col_stride;
+} eg_f16_source;
+
+/* An operand of eg_gemm_f16x3: one or two sources side by side along K (each
+ * padded with zeros to a multiple of 32 there), with the buffers that
+ * eg_split_f16 fills: planes (eg_f16_planes_bytes(rows, the sum of the padded
+ * cols) bytes, 16-byte aligned) and exps (eg_f16_exps_count(rows) int32).  The
+ * sources are read by eg_gemm_f16x3 too (rows beyond the planes' range). */
+typedef struct eg_f16_matrix {
+  eg_f16_source src[2];
+  int32_t n_src; /* 1 or 2 */
+  int64_t rows;
+  void* planes;
+  int32_t* exps;
+} eg_f16_matrix;
+
+int64_t eg_f16_planes_bytes(int64_t rows, int64_t k);
+int64_t eg_f16_exps_count(int64_t rows);
+
+/* Fills x's planes and exps: every row scaled by a power of two (its largest
+ * magnitude to [2^14, 2^15), the exponent kept in exps) and split into fp16
+ * planes hi = rne(x) and lo = rne(x - hi).  A row is marked when its largest
+ * magnitude is not finite or below 2^-87, or when more than 1/16 of its values
+ * are nonzero and more than 2^24 below the largest of their source's part.  No counterpart in the reference (part of its fp32
+ * matmuls). */
+int eg_split_f16(const eg_f16_matrix* x, void* stream);
+
+/* C [m, n] = A B^T and, with b2, C2 [m, n2] = A B2^T (m, n, n2 the operands'
+ * rows), with an fp32 matmul's accuracy on the fp16 matrix cores: hi*hi + hi*lo
+ * + lo*hi of the operands' eg_split_f16 planes accumulated in fp32; the
+ * outputs of marked rows in fp32 from the sources.  a and b with the same
+ * sources' cols, at least one column.  Workspace of eg_gemm_workspace_size(m, n,
+ * n2, k, 0) bytes, k the sum of the padded cols.  ple_forward's projections
+ * and their gradients past a few rows (engraft/replica/layers.py:594-606, torch
+ * fp32 matmuls). */
+int eg_gemm_f16x3(const eg_f16_matrix* a, const eg_f16_matrix* b, const eg_f16_matrix* b2, float* c, int64_t ldc,
+                  float* c2, int64_t ldc2, void* workspace, int64_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }
