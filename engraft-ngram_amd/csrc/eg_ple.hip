@@ -48,15 +48,26 @@ __device__ inline float block_sum(float x, float* red) {
 // n <= kPleThreads * kPleMaxPer values per stream.
 constexpr int kPleMaxPer = 16;
 
+// Workgroup -> (position, stream) of the gate kernels: workgroup b runs on XCD
+// b % 8, and the streams of a position, which read the same value row, are
+// consecutive workgroups of one XCD.  False for the grid's padding.
+__device__ inline bool position_stream(int hc, int64_t T, int64_t& t, int& j) {
+  const unsigned k = blockIdx.x / 8;
+  j = (int)(k % (unsigned)hc);
+  t = (int64_t)(k / (unsigned)hc) * 8 + blockIdx.x % 8;
+  return t < T;
+}
+
 __global__ __launch_bounds__(kPleThreads) void ple_gate_kernel(
     const float* __restrict__ key, const float* __restrict__ value, const float* __restrict__ hidden,
     const float* __restrict__ norm_key, const float* __restrict__ norm_query, const float* __restrict__ norm_conv,
-    int hc, int n, float eps, float inv_sqrt_n, float* __restrict__ normed, float* __restrict__ s_out,
+    int64_t T, int hc, int n, float eps, float inv_sqrt_n, float* __restrict__ normed, float* __restrict__ s_out,
     float* __restrict__ gate_out, float* __restrict__ rstd_out) {
 #pragma clang fp contract(off)
   __shared__ float red[kPleThreads / 64];
-  const int64_t t = blockIdx.x / hc;
-  const int j = (int)(blockIdx.x - t * hc);
+  int64_t t;
+  int j;
+  if (!position_stream(hc, T, t, j)) return;
   const int tid = threadIdx.x;
   const int per = (n + kPleThreads - 1) / kPleThreads;
   // Every load of the workgroup is issued before the first reduction (indices
@@ -107,7 +118,7 @@ __global__ __launch_bounds__(kPleThreads) void ple_gate_kernel(
 #pragma unroll
   for (int m = 0; m < kPleMaxPer; ++m) {
     const int i = tid + m * kPleThreads;
-    if (m < per && i < n) normed[row + i] = ((v[m] * gate) * rg) * norm_conv[j * n + i];
+    if (normed != nullptr && m < per && i < n) normed[row + i] = ((v[m] * gate) * rg) * norm_conv[j * n + i];
   }
   if (tid == 0) {
     s_out[t * hc + j] = s;
@@ -255,6 +266,131 @@ __global__ __launch_bounds__(256) void ple_conv_win_kernel(const float* __restri
   }
 }
 
+// ple_conv_win_kernel over [history; normed] with the normed rows computed
+// here from value, gate and the gated row's RMS factor, ((value gate) r_g)
+// norm_conv as the gate kernel writes them (the same values), so that they are
+// neither written nor read: hidden and out, and value (a quarter of them) once
+// an XCD, are what the kernel moves, and HBM bounds it.  Workgroup: 256
+// channels of one stream (n a multiple of 256) x RUN positions, four channels
+// a lane; its value rows (and the history's before the first position) sit in
+// LDS, a wavefront's hidden rows in registers before the barrier.  The
+// workgroups of one channel block's streams are consecutive on one XCD (they
+// read the same value columns).  The last positions' workgroups write the new
+// history, the last new_rows rows.  2,048 positions of 4 x 2560: 48 us
+// (190 MB at 4.0 TB/s; 88 us with ple_gate_kernel), against 62 us with the
+// normed rows in memory (119 us with their write); 32 positions a thread with
+// one channel each, the window in registers (two wavefronts a SIMD): 75 us.
+constexpr int kGatedRun = 16;
+
+typedef float fvec4 __attribute__((ext_vector_type(4)));
+
+__device__ inline void f4(const float* p, float* o) {
+  const float4 v = *(const float4*)p;
+  o[0] = v.x;
+  o[1] = v.y;
+  o[2] = v.z;
+  o[3] = v.w;
+}
+
+// Rows read or written once go past the caches' reuse.
+__device__ inline float4 nt_load4(const float* p) {
+  const fvec4 v = __builtin_nontemporal_load((const fvec4*)p);
+  return make_float4(v.x, v.y, v.z, v.w);
+}
+__device__ inline void nt_store4(float* p, const float* x) {
+  __builtin_nontemporal_store((fvec4){x[0], x[1], x[2], x[3]}, (fvec4*)p);
+}
+
+template <int TAPS, int DIL>
+__global__ __launch_bounds__(256) void ple_conv_gated_kernel(
+    const float* __restrict__ hist, int64_t hist_rows, int64_t T, int hc, int n, const float* __restrict__ value,
+    const float* __restrict__ gate, const float* __restrict__ rstd, const float* __restrict__ norm_conv,
+    const float* __restrict__ conv_w, const float* __restrict__ hidden, float* __restrict__ out,
+    float* __restrict__ pre, float* __restrict__ new_hist, int64_t new_rows) {
+#pragma clang fp contract(off)
+  constexpr int H = (TAPS - 1) * DIL, RUN = kGatedRun, ROWS = RUN + H, PW = RUN / 4;
+  __shared__ float s_gate[ROWS], s_rg[ROWS];
+  __shared__ float4 s_row[ROWS][64];
+  const int C = hc * n;
+  const int n_iblk = n / 256;
+  const unsigned q8 = blockIdx.x / 8;
+  const int j = (int)(q8 % (unsigned)hc);
+  const int64_t unit = (int64_t)(q8 / (unsigned)hc) * 8 + blockIdx.x % 8;  // (run, channel block)
+  const int64_t t0 = unit / n_iblk * RUN;
+  if (t0 >= T) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int i = (int)(unit % n_iblk) * 256 + 4 * lane;
+  const int c = j * n + i;
+  // row q is position t0 - H + q: its value, or, before the first position, the
+  // history's row (none: zeros whose taps are dropped)
+  float4 row[(ROWS + 3) / 4], hv[PW];
+#pragma unroll
+  for (int k = 0; k < (ROWS + 3) / 4; ++k) {
+    const int q = min(wave + 4 * k, ROWS - 1);
+    const int64_t t = t0 - H + q, r = hist_rows + t;
+    if (t >= 0) row[k] = *(const float4*)(value + min(t, T - 1) * n + i);
+    else row[k] = r >= 0 ? *(const float4*)(hist + r * C + c) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  }
+#pragma unroll
+  for (int b = 0; b < PW; ++b) hv[b] = nt_load4(hidden + min(t0 + wave * PW + b, T - 1) * C + c);
+  if (threadIdx.x < ROWS) {
+    const int64_t t = t0 - H + threadIdx.x;
+    const int64_t pj = (t < 0 ? 0 : min(t, T - 1)) * hc + j;
+    s_gate[threadIdx.x] = gate[pj];
+    s_rg[threadIdx.x] = rstd[pj * 3 + 2];
+  }
+  float w[4][TAPS], nc[4];
+  static_assert(TAPS == 4, "a channel's taps are one float4");
+#pragma unroll
+  for (int e = 0; e < 4; ++e) f4(conv_w + (int64_t)(c + e) * TAPS, w[e]);
+  f4(norm_conv + c, nc);
+#pragma unroll
+  for (int k = 0; k < (ROWS + 3) / 4; ++k)
+    if (wave + 4 * k < ROWS) s_row[wave + 4 * k][lane] = row[k];
+  __syncthreads();
+  // [history; normed] at row q
+  auto normed = [&](int q, float* x) {
+    const float4 v = s_row[q][lane];
+    x[0] = v.x, x[1] = v.y, x[2] = v.z, x[3] = v.w;
+    if (t0 - H + q < 0) return;
+    const float g = s_gate[q], rg = s_rg[q];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = ((x[e] * g) * rg) * nc[e];
+  };
+#pragma unroll
+  for (int b = 0; b < PW; ++b) {
+    const int p = wave * PW + b;
+    const int64_t t = t0 + p;
+    if (t >= T) break;
+    float acc[4] = {};
+#pragma unroll
+    for (int k = 0; k < TAPS; ++k) {
+      float x[4];
+      normed(p + k * DIL, x);
+      if (hist_rows + t - H + k * DIL >= 0) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] += x[e] * w[e][k];
+      }
+    }
+    const float4 v = s_row[p + H][lane];
+    const float vv[4] = {v.x, v.y, v.z, v.w}, h[4] = {hv[b].x, hv[b].y, hv[b].z, hv[b].w}, g = s_gate[p + H];
+    float o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (h[e] + vv[e] * g) + acc[e] / (1.0f + expf(-acc[e]));
+    if (pre != nullptr) nt_store4(pre + t * C + c, acc);
+    nt_store4(out + t * C + c, o);
+  }
+  if (t0 + RUN >= T) {
+    for (int q = wave; q < ROWS; q += 4) {
+      const int64_t t = t0 - H + q, r = t - (T - new_rows);
+      if (t >= T || r < 0) continue;
+      float x[4];
+      normed(q, x);
+      *(float4*)(new_hist + r * C + c) = make_float4(x[0], x[1], x[2], x[3]);
+    }
+  }
+}
+
 // The per-stream RMS norm, with the reductions of ple_gate_kernel (same thread
 // layout and tree), so it reproduces that kernel's normed values bit for bit.
 __global__ __launch_bounds__(kPleThreads) void ple_rms_kernel(const float* __restrict__ x, int hc, int n, float eps,
@@ -303,24 +439,17 @@ __device__ inline float block_sum_2w(float x, float* red) {
   return red[0] + red[1];
 }
 
-__device__ inline void f4(const float* p, float* o) {
-  const float4 v = *(const float4*)p;
-  o[0] = v.x;
-  o[1] = v.y;
-  o[2] = v.z;
-  o[3] = v.w;
-}
-
 template <int P>
 __global__ __launch_bounds__(kVecThreads) void ple_gate_vec_kernel(
     const float* __restrict__ key, const float* __restrict__ value, const float* __restrict__ hidden,
     const float* __restrict__ norm_key, const float* __restrict__ norm_query, const float* __restrict__ norm_conv,
-    int hc, int n, float eps, float inv_sqrt_n, float* __restrict__ normed, float* __restrict__ s_out,
+    int64_t T, int hc, int n, float eps, float inv_sqrt_n, float* __restrict__ normed, float* __restrict__ s_out,
     float* __restrict__ gate_out, float* __restrict__ rstd_out) {
 #pragma clang fp contract(off)
   __shared__ float red[2];
-  const int64_t t = blockIdx.x / hc;
-  const int j = (int)(blockIdx.x - t * hc);
+  int64_t t;
+  int j;
+  if (!position_stream(hc, T, t, j)) return;
   const int64_t row = (t * hc + j) * n;
   float v[P][4], k[P][4], h[P][4], wk[P][4], wq[P][4];
 #pragma unroll
@@ -364,14 +493,16 @@ __global__ __launch_bounds__(kVecThreads) void ple_gate_vec_kernel(
         sq += g * g;
       }
   const float rg = 1.0f / sqrtf(block_sum_2w(sq, red) / (float)n + eps);
+  if (normed != nullptr) {
 #pragma unroll
-  for (int p = 0; p < P; ++p) {
-    const int i = 4 * threadIdx.x + p * 4 * kVecThreads;
-    float wc[4], o[4];
-    f4(norm_conv + (int64_t)j * n + i, wc);
+    for (int p = 0; p < P; ++p) {
+      const int i = 4 * threadIdx.x + p * 4 * kVecThreads;
+      float wc[4], o[4];
+      f4(norm_conv + (int64_t)j * n + i, wc);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = ((v[p][e] * gate) * rg) * wc[e];
-    *(float4*)(normed + row + i) = make_float4(o[0], o[1], o[2], o[3]);
+      for (int e = 0; e < 4; ++e) o[e] = ((v[p][e] * gate) * rg) * wc[e];
+      *(float4*)(normed + row + i) = make_float4(o[0], o[1], o[2], o[3]);
+    }
   }
   if (threadIdx.x == 0) {
     s_out[t * hc + j] = s;
@@ -938,22 +1069,23 @@ int eg_ple_gate(const float* key, const float* value, const float* hidden, const
   EG_CHECK_ARG(n_pos >= 0 && n_pos * hc < (1LL << 31), "n_pos=%lld", (long long)n_pos);
   EG_CHECK_ARG(hc >= 1 && hc <= 64 && n_embd >= 1 && n_embd <= kPleThreads * kPleMaxPer,
                "hc=%d n_embd=%d (n_embd <= %d)", hc, n_embd, kPleThreads * kPleMaxPer);
-  EG_CHECK_ARG(n_pos == 0 || (key && value && hidden && norm_key && norm_query && norm_conv && normed && s_out &&
-                              gate_out),
+  EG_CHECK_ARG(n_pos == 0 || (key && value && hidden && norm_key && norm_query && (norm_conv || !normed) && s_out &&
+                              gate_out && (normed || rstd_out)),
                "NULL argument");
   if (n_pos == 0) return EG_OK;
+  EG_CHECK_ARG((n_pos + 7) / 8 * 8 * hc < (1LL << 31), "n_pos=%lld", (long long)n_pos);
+  const dim3 grid((unsigned)((n_pos + 7) / 8 * 8 * hc));
   const bool vec = n_embd % (4 * kVecThreads) == 0 &&
                    ((uintptr_t)key | (uintptr_t)value | (uintptr_t)hidden | (uintptr_t)norm_key |
                     (uintptr_t)norm_query | (uintptr_t)norm_conv | (uintptr_t)normed) % 16 == 0;
   if (vec)
     launch_vec_p(n_embd / (4 * kVecThreads), [&](auto pc) {
-      hipLaunchKernelGGL(ple_gate_vec_kernel<decltype(pc)::value>, dim3((unsigned)(n_pos * hc)), dim3(kVecThreads), 0,
-                         (hipStream_t)stream, key, value, hidden, norm_key, norm_query, norm_conv, hc, n_embd, eps,
-                         (float)(1.0 / sqrt((double)n_embd)), normed, s_out, gate_out, rstd_out);
+      hipLaunchKernelGGL(ple_gate_vec_kernel<decltype(pc)::value>, grid, dim3(kVecThreads), 0, (hipStream_t)stream, key,
+                         value, hidden, norm_key, norm_query, norm_conv, n_pos, hc, n_embd, eps, (float)(1.0 / sqrt((double)n_embd)), normed, s_out, gate_out, rstd_out);
     });
   else
-    hipLaunchKernelGGL(ple_gate_kernel, dim3((unsigned)(n_pos * hc)), dim3(kPleThreads), 0, (hipStream_t)stream, key,
-                       value, hidden, norm_key, norm_query, norm_conv, hc, n_embd, eps,
+    hipLaunchKernelGGL(ple_gate_kernel, grid, dim3(kPleThreads), 0, (hipStream_t)stream, key, value, hidden, norm_key,
+                       norm_query, norm_conv, n_pos, hc, n_embd, eps,
                        (float)(1.0 / sqrt((double)n_embd)), normed, s_out, gate_out, rstd_out);
   return launch_status("ple_gate_kernel");
 }
@@ -982,6 +1114,34 @@ int eg_ple_conv(const float* full, int64_t hist_rows, int64_t n_pos, int32_t hc,
   else sh ? EG_CONV(2, true) : EG_CONV(2, false);
 #undef EG_CONV
   return launch_status("ple_conv_kernel");
+}
+
+int eg_ple_conv_gated(const float* hist, int64_t hist_rows, int64_t n_pos, int32_t hc, int32_t n_embd,
+                      const float* value, const float* gate, const float* rstd, const float* norm_conv,
+                      const float* conv_w, int32_t taps, int32_t dilation, const float* hidden, float* out, float* pre,
+                      float* new_hist, void* stream) {
+  EG_CHECK_ARG(n_pos >= 0 && hist_rows >= 0 && hc >= 1 && n_embd >= 1, "n_pos=%lld hist_rows=%lld hc=%d n_embd=%d",
+               (long long)n_pos, (long long)hist_rows, hc, n_embd);
+  if (taps != 4 || dilation != 3 || n_embd % 256 != 0)
+    return set_error(EG_ERR_UNSUPPORTED, "gated convolution of %d taps, dilation %d, n_embd %d (built: 4 taps, "
+                     "dilation 3, n_embd a multiple of 256)", taps, dilation, n_embd);
+  EG_CHECK_ARG(n_pos < (1LL << 31) && (int64_t)hc * n_embd < (1LL << 31), "too many elements");
+  EG_CHECK_ARG(n_pos == 0 || (value && gate && rstd && norm_conv && conv_w && hidden && out && new_hist &&
+                              (hist || hist_rows == 0)),
+               "NULL argument");
+  if (n_pos == 0) return EG_OK;
+  const int64_t new_rows = hist_rows + n_pos < 9 ? hist_rows + n_pos : 9;
+  // float4 rows: every pointer on 16 bytes
+  EG_CHECK_ARG((((uintptr_t)hist | (uintptr_t)value | (uintptr_t)hidden | (uintptr_t)out | (uintptr_t)pre |
+                 (uintptr_t)new_hist | (uintptr_t)conv_w | (uintptr_t)norm_conv) & 15) == 0,
+               "pointers must be 16-byte aligned");
+  const int64_t units = (n_pos + kGatedRun - 1) / kGatedRun * (n_embd / 256);
+  const int64_t blocks = (units + 7) / 8 * 8 * hc;
+  EG_CHECK_ARG(blocks < (1LL << 31), "too many elements");
+  hipLaunchKernelGGL((ple_conv_gated_kernel<4, 3>), dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, hist,
+                     hist_rows, n_pos, hc, n_embd, value, gate, rstd, norm_conv, conv_w, hidden, out, pre, new_hist,
+                     new_rows);
+  return launch_status("ple_conv_gated_kernel");
 }
 
 int eg_ple_rms(const float* x, int64_t n_rows, int32_t hc, int32_t n_embd, const float* weight, float eps, float* out,
@@ -1016,7 +1176,7 @@ int eg_ple_conv_backward(const float* full, int64_t hist_rows, int64_t n_pos, in
   EG_CHECK_ARG(tail_rows >= 0 && tail_rows <= hist_rows + n_pos, "tail_rows=%lld", (long long)tail_rows);
   EG_CHECK_ARG(n_pos < (1LL << 31) && (int64_t)hc * n_embd < (1LL << 31), "too many elements");
   const int64_t rows = hist_rows + n_pos;
-  EG_CHECK_ARG(rows == 0 || (full && conv_w && d_full && (n_pos == 0 || d_out)), "NULL argument");
+  EG_CHECK_ARG(rows == 0 || ((full || pre) && conv_w && d_full && (n_pos == 0 || d_out)), "NULL argument");
   EG_CHECK_ARG(tail_rows == 0 || d_tail != nullptr, "d_tail is NULL");
   if (rows == 0) return EG_OK;
   const int64_t blocks = (int64_t)((hc * n_embd + 255) / 256) * ((rows + kConvBwdRun - 1) / kConvBwdRun);

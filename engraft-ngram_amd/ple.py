@@ -539,9 +539,6 @@ class _PleFn(torch.autograd.Function):
             key, value = gemm_f32(emb32, wk32, b_n2=wv32)
         hidden32 = hidden.to(**f32).contiguous()
         h0 = hist.shape[0]
-        full = torch.empty((h0 + t_len, hc * n), **f32)
-        if h0:
-            full[:h0] = hist.reshape(h0, hc * n)
         s = torch.empty((t_len, hc), **f32)
         gate = torch.empty((t_len, hc), **f32)
         st = _lib.stream_ptr(dev)
@@ -550,17 +547,35 @@ class _PleFn(torch.autograd.Function):
         taps = conv32.shape[1]
         native = any(ctx.needs_input_grad) and _native_backward_ok(hc, n, taps, int(dil),
                                                                    weights=any(ctx.needs_input_grad[2:8]))
-        rstd = torch.empty((t_len, hc, 3), **f32) if native else None
+        # without the normed rows in memory where the gated convolution is built and no
+        # weight's gradient reads them
+        gated = (taps == 4 and int(dil) == 3 and n % 256 == 0 and not any(ctx.needs_input_grad[2:8])
+                 and not (hidden32.data_ptr() | hist.data_ptr() | nc32.data_ptr() | conv32.data_ptr()) % 16)
+        rstd = torch.empty((t_len, hc, 3), **f32) if native or gated else None
+        full = None if gated else torch.empty((h0 + t_len, hc * n), **f32)
         _lib.call("eg_ple_gate", _lib.ptr(key), _lib.ptr(value), _lib.ptr(hidden32), _lib.ptr(nk32), _lib.ptr(nq32),
-                  _lib.ptr(nc32), t_len, hc, n, float(eps), _lib.ptr(full[h0:]), _lib.ptr(s), _lib.ptr(gate),
-                  _lib.ptr(rstd), st)
+                  _lib.ptr(nc32), t_len, hc, n, float(eps), None if gated else _lib.ptr(full[h0:]), _lib.ptr(s),
+                  _lib.ptr(gate), _lib.ptr(rstd), st)
         out = torch.empty((t_len, hc, n), **f32)
         pre = torch.empty((t_len, hc * n), **f32) if native else None  # kept for the backward's SiLU derivative
-        _lib.call("eg_ple_conv", _lib.ptr(full), h0, t_len, hc, n, _lib.ptr(conv32), taps, int(dil), 0,
-                  _lib.ptr(hidden32), _lib.ptr(value), _lib.ptr(gate), _lib.ptr(out), _lib.ptr(pre), st)
-        hist_len = (taps - 1) * int(dil)
-        new_hist = (full[-hist_len:] if hist_len > 0 else full[:0]).reshape(-1, hc, n).to(hidden.dtype).clone()
+        if gated:
+            hist32 = hist.to(**f32).contiguous()
+            new_hist = torch.empty((min(9, h0 + t_len), hc, n), **f32)
+            if t_len == 0:
+                new_hist.copy_(hist32[h0 - new_hist.shape[0]:])
+            _lib.call("eg_ple_conv_gated", _lib.ptr(hist32), h0, t_len, hc, n, _lib.ptr(value), _lib.ptr(gate),
+                      _lib.ptr(rstd), _lib.ptr(nc32), _lib.ptr(conv32), taps, int(dil), _lib.ptr(hidden32),
+                      _lib.ptr(out), _lib.ptr(pre), _lib.ptr(new_hist), st)
+            new_hist = new_hist.to(hidden.dtype)
+        else:
+            if h0:
+                full[:h0] = hist.reshape(h0, hc * n)
+            _lib.call("eg_ple_conv", _lib.ptr(full), h0, t_len, hc, n, _lib.ptr(conv32), taps, int(dil), 0,
+                      _lib.ptr(hidden32), _lib.ptr(value), _lib.ptr(gate), _lib.ptr(out), _lib.ptr(pre), st)
+            hist_len = (taps - 1) * int(dil)
+            new_hist = (full[-hist_len:] if hist_len > 0 else full[:0]).reshape(-1, hc, n).to(hidden.dtype).clone()
         ctx.native = native
+        ctx.hist_rows = h0
         if native:
             # emb for the projection weights' gradients
             emb_w = emb32 if any(ctx.needs_input_grad[2:4]) else None
@@ -603,8 +618,8 @@ class _PleFn(torch.autograd.Function):
         emb_dt, hidden_dt, hist_dt = ctx.dtypes
         t_len, hc, n = hidden32.shape
         c_dim = hc * n
-        h0 = full.shape[0] - t_len
-        dev = full.device
+        h0 = ctx.hist_rows
+        dev = hidden32.device
         f32 = dict(dtype=torch.float32, device=dev)
         st = _lib.stream_ptr(dev)
         need_emb, need_hidden, need_hist = ctx.needs_input_grad[0], ctx.needs_input_grad[1], ctx.needs_input_grad[8]

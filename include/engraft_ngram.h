@@ -32,7 +32,7 @@
  *   (= eg_descent_plan + eg_descent_apply)           engraft/descend_corpus.py:785-790,921-947
  *   eg_forward_decode  the per-token gather of a decode step with the overlay
  *                                                    engraft/replica/model.py:473-495
- *   eg_ple_gate, eg_ple_conv  ple_forward after its two projections
+ *   eg_ple_gate, eg_ple_conv(_gated)  ple_forward after its two projections
  *   (+ _backward)    and the autograd of it          engraft/replica/layers.py:565-626
  *   eg_ple_rms, eg_ple_conv's other modes  PleReplica engraft/lens.py:221-385
  *   eg_split_bf16, eg_gemm_bf16x3, eg_gemm_f32 (+ _workspace_size),
@@ -413,7 +413,8 @@ int eg_synth_table(const eg_table* table, uint64_t seed, const float* qtable,
  * gated_j = value * gate, normed_j = rmsnorm(gated_j) * norm_conv.
  * normed f32 [n_pos, hc*n_embd]; s_out, gate_out f32 [n_pos, hc]; rstd_out
  * (optional, f32 [n_pos, hc, 3]) the RMS factors 1/sqrt(mean(x^2) + eps) of
- * key, hidden and gated, which eg_ple_gate_backward takes. */
+ * key, hidden and gated, which eg_ple_gate_backward takes.  normed may be NULL
+ * where rstd_out is given: eg_ple_conv_gated computes it from the factors. */
 int eg_ple_gate(const float* key, const float* value, const float* hidden, const float* norm_key,
                 const float* norm_query, const float* norm_conv, int64_t n_pos, int32_t hc,
                 int32_t n_embd, float eps, float* normed, float* s_out, float* gate_out,
@@ -435,13 +436,25 @@ int eg_ple_conv(const float* full, int64_t hist_rows, int64_t n_pos, int32_t hc,
                 const float* hidden, const float* value, const float* gate, float* out, float* pre,
                 void* stream);
 
+/* eg_ple_conv (hidden, value and gate given, own history) from eg_ple_gate's
+ * gate and rstd in place of its normed rows, which it computes as
+ * ((value * gate) * rstd[.., 2]) * norm_conv (the same values; they are
+ * neither written nor read), over the history hist f32 [hist_rows,
+ * hc*n_embd].  new_hist receives the last min(9, hist_rows + n_pos) rows of
+ * [history; normed].  Built for 4 taps at dilation 3 and n_embd a multiple of
+ * 256 (EG_ERR_UNSUPPORTED otherwise); the rows' pointers 16-byte aligned. */
+int eg_ple_conv_gated(const float* hist, int64_t hist_rows, int64_t n_pos, int32_t hc, int32_t n_embd,
+                      const float* value, const float* gate, const float* rstd, const float* norm_conv,
+                      const float* conv_w, int32_t taps, int32_t dilation, const float* hidden,
+                      float* out, float* pre, float* new_hist, void* stream);
+
 /* Backward of eg_ple_conv (mode 0, own history): d_full f32 [hist_rows + n_pos,
  * hc*n_embd] = the gradient of [history; normed] given d_out f32 [n_pos,
  * hc*n_embd] (the block's output gradient) and d_tail (optional, f32
  * [tail_rows, hc*n_embd]: the gradient of the last tail_rows rows of full, the
  * history the forward returned).  full and conv_w as the forward's; pre
  * (optional) the forward's pre-activation, read in place of recomputing the
- * convolution.  The convolution weights' gradient is not computed.
+ * convolution (full is then not read and may be NULL).  The convolution weights' gradient is not computed.
  * (taps-1)*dilation <= 32.  Replaces the autograd of causal_depthwise_conv +
  * silu (engraft/replica/layers.py:257-293, 614-626). */
 int eg_ple_conv_backward(const float* full, int64_t hist_rows, int64_t n_pos, int32_t hc, int32_t n_embd,
