@@ -1113,53 +1113,65 @@ __global__ __launch_bounds__(256) void piece_sum_kernel(const Plan p, const Scal
 }
 
 // C (+)= the sum, in K order, of the parts of a last-round tile that the
-// ranges of gemm_f32_kernel computed: the ranges meeting the tile, in
-// increasing order (a tile one range covers whole was stored directly).
-// BM BN / 1024 blocks a tile, four columns a thread.
+// ranges computed: the ranges meeting the tile, in increasing order (a tile
+// one range covers whole was stored directly).  A range holds at least 8
+// units, so the tile's parts are those of the consecutive ranges s0 .. s1, and
+// only s0 can have begun in an earlier tile.  A thread sums kSumRows float4,
+// one row of four apart, all their loads of a part in flight, and stores four
+// columns at once where C allows it: bound by HBM (the parts and C).  On the
+// PLE key + value of 2,048 positions (100 MB of parts, 38 MB of C) 24 us,
+// 41 us with one float4 and the ranges' 64-bit divisions a thread.
+constexpr int kSumRows = 4;
+
 template <int BM, int BN, typename Scale>
 __global__ __launch_bounds__(256) void sk_sum_kernel(const Plan p, const Scale scale) {
-  constexpr int kBlocks = BM * BN / 1024;
-  const int q = blockIdx.x / kBlocks;  // last-round tile
-  const int e = (blockIdx.x % kBlocks) * 256 + threadIdx.x;
-  const int lr = e / (BN / 4), lc = (e % (BN / 4)) * 4;
+  constexpr int kBlocks = BM * BN / 1024 / kSumRows;
+  constexpr int kRowsApart = 1024 / BN;  // rows of the tile 256 threads of float4 cover
+  const int q = blockIdx.x / kBlocks;    // last-round tile
+  const int lr0 = (int)(blockIdx.x % kBlocks) * kSumRows * kRowsApart + (int)threadIdx.x / (BN / 4);
+  const int lc = ((int)threadIdx.x % (BN / 4)) * 4;
   const int64_t kt = p.kt_total, x0 = (int64_t)q * kt, x1 = x0 + kt;
-  // the range holding unit x0: the last s with start(s) <= x0 (skips empty ranges)
-  int64_t s = x0 * p.sk_groups / p.sk_units;
-  while (s > 0 && sk_start(p, s) > x0) --s;
-  while (s + 1 < p.sk_groups && sk_start(p, s + 1) <= x0) ++s;
-  if (sk_start(p, s + 1) >= x1) return;  // one range covers the tile: stored directly
+  // the last s with start(s) <= x: floor(U s / G) <= x  <=>  U s < (x + 1) G
+  const int64_t s0 = ((x0 + 1) * p.sk_groups - 1) / p.sk_units, s1 = (x1 * p.sk_groups - 1) / p.sk_units;
+  if (s0 == s1) return;  // one range covers the tile: stored directly
   int tm, tn;
   grouped(p.dp_tiles + q, p.tiles_m, p.tiles_n, tm, tn);
   const int grp = tn < p.tiles_n0 ? 0 : 1;
-  const int64_t row = (int64_t)tm * BM + lr;
-  if (row >= p.m) return;
-  float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  bool first = true;
-  for (; s < p.sk_groups; ++s) {
-    const int64_t a = sk_start(p, s);
-    if (a >= x1) break;
-    if (a == sk_start(p, s + 1)) continue;  // empty range
-    const int slot = 2 * (int)s + (int)(q - a / kt);
-    const float4 u = *((const float4*)(p.ws + (int64_t)slot * (BM * BN)) + e);
-    if (first) {
-      v = u;
-      first = false;
-    } else {
-      v.x += u.x;
-      v.y += u.y;
-      v.z += u.z;
-      v.w += u.w;
+  const float* ws = p.ws + lr0 * BN + lc;
+  const int64_t first = 2 * s0 + (sk_start(p, s0) < x0 ? 1 : 0);
+  float4 v[kSumRows];
+#pragma unroll
+  for (int r = 0; r < kSumRows; ++r) v[r] = *(const float4*)(ws + first * (BM * BN) + r * kRowsApart * BN);
+  for (int64_t s = s0 + 1; s <= s1; ++s) {
+#pragma unroll
+    for (int r = 0; r < kSumRows; ++r) {
+      const float4 u = *(const float4*)(ws + 2 * s * (BM * BN) + r * kRowsApart * BN);
+      v[r].x += u.x;
+      v[r].y += u.y;
+      v[r].z += u.z;
+      v[r].w += u.w;
     }
   }
-  const int64_t n_grp = p.n[grp], col0 = (int64_t)(grp ? tn - p.tiles_n0 : tn) * BN + lc;
-  float* out = p.c[grp] + row * p.ldc[grp];
-  const float vv[4] = {v.x, v.y, v.z, v.w};
+  const int64_t n_grp = p.n[grp], col0 = (int64_t)(grp ? tn - p.tiles_n0 : tn) * BN + lc, ld = p.ldc[grp];
+  const bool whole = col0 + 4 <= n_grp && (ld & 3) == 0 && ((uintptr_t)p.c[grp] & 15) == 0 && !p.accumulate;
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int64_t col = col0 + t;
-    if (col < n_grp) {
-      const float x = scale(vv[t], grp, row, col);
-      out[col] = p.accumulate ? out[col] + x : x;
+  for (int r = 0; r < kSumRows; ++r) {
+    const int64_t row = (int64_t)tm * BM + lr0 + r * kRowsApart;
+    if (row >= p.m) return;
+    float* out = p.c[grp] + row * ld;
+    const float vv[4] = {v[r].x, v[r].y, v[r].z, v[r].w};
+    if (whole) {
+      *(float4*)(out + col0) = make_float4(scale(vv[0], grp, row, col0), scale(vv[1], grp, row, col0 + 1),
+                                           scale(vv[2], grp, row, col0 + 2), scale(vv[3], grp, row, col0 + 3));
+      continue;
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int64_t col = col0 + t;
+      if (col < n_grp) {
+        const float x = scale(vv[t], grp, row, col);
+        out[col] = p.accumulate ? out[col] + x : x;
+      }
     }
   }
 }
@@ -1358,7 +1370,7 @@ int launch_gemm(const Shape& sh, void (*kernel)(const Args), const char* name, A
   if (rc != 0 || pp.dp == tiles) return rc;
   const dim3 sum_grid((unsigned)((tiles - pp.dp) * (BM * BN / 1024)));
   if (pp.sk_groups > 0) {
-    hipLaunchKernelGGL((sk_sum_kernel<BM, BN, Scale>), sum_grid, dim3(256), 0, st, p, scale);
+    hipLaunchKernelGGL((sk_sum_kernel<BM, BN, Scale>), dim3(sum_grid.x / kSumRows), dim3(256), 0, st, p, scale);
     return launch_status("sk_sum_kernel");
   }
   hipLaunchKernelGGL((piece_sum_kernel<BM, BN, Scale>), sum_grid, dim3(256), 0, st, p, scale);
