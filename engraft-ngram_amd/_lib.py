@@ -182,6 +182,8 @@ SIGNATURES = {
     "eg_gemm_bf16x6": (c_int32, [POINTER(EgGemmOperands), POINTER(EgGemmOperands), c_int32, c_int64, c_int64,
                                  c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int32, c_int32, c_void_p, c_int64,
                                  c_void_p]),
+    "eg_gemm_f32_rows": (c_int32, [POINTER(EgGemmF32Operands), c_int32, c_int64, c_int64, c_int64, c_void_p, c_int64,
+                                   c_void_p, c_int64, c_int32, c_void_p]),
     "eg_f16_planes_bytes": (c_int64, [c_int64, c_int64]),
     "eg_f16_exps_count": (c_int64, [c_int64]),
     "eg_split_f16": (c_int32, [POINTER(EgF16Matrix), c_void_p]),

@@ -72,6 +72,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kGroupM = 8;
 constexpr int kXcds = 8;
@@ -681,6 +682,213 @@ template <int BM, int BN>
 __global__ __launch_bounds__(BM * BN / 64) void gemm_f32_kernel(const F32Args args) {
   extern __shared__ __attribute__((aligned(16))) float ldsf[];
   EG_GEMM_WALK(f32_tile<BM, BN>(args, w, ldsf))
+}
+
+// eg_gemm_f32_rows: at most 32 rows of A (a decoded token's projections): reading B
+// once from HBM is all such a product costs, so nothing is split over
+// workgroups.  A workgroup takes 32 columns; its NW wavefronts take every
+// NW-th K step (together 128 NW consecutive bytes of a row), and their sums
+// are added in wavefront order.  A wavefront loads a step's 32 rows of B (and
+// MR of A) eight lanes to a row's 128 bytes, SETS steps ahead, and turns them
+// into fragments (f32_tile's) through 4 + MR / 8 KB of LDS of its own, without
+// a barrier: fragments loaded straight from global memory, a lane to a row,
+// cost the address path a request a lane (42 us).  131 MB of the PLE key and
+// value weights, 5 to 8 rows: 36 us, 32 rows: 44 us; 115 us for gemm_x6_kernel's 256-row tiles
+// (196 MB of planes, its parts' sum included).
+constexpr int kFewRows = 32;  // SETS: 2 or 3
+
+template <int NW, int MR, int SETS>
+__global__ __launch_bounds__(64 * NW, 4) void gemm_f32_rows_kernel(const F32Args args) {
+  constexpr int MA = MR / 8;  // loads of A a step
+  // the steps' staging, then the wavefronts' sums
+  __shared__ f32x4 lds[NW * 256 > NW * (32 + MR) * 8 ? NW * 256 : NW * (32 + MR) * 8];
+  const Plan& p = args.p;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t blocks0 = (p.n[0] + 31) / 32;
+  const int grp = (int64_t)blockIdx.x < blocks0 ? 0 : 1;
+  const int64_t n0 = 32 * ((int64_t)blockIdx.x - (grp ? blocks0 : 0)), n_grp = p.n[grp];
+  f32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+  f32x4* mine = lds + wave * (32 + MR) * 8;  // B's 32 rows of 8 chunks, then A's MR
+  const int lr = lane >> 3, lc = lane & 7;
+  int64_t seg0 = 0;
+  for (int s = 0; s < args.n_seg; ++s) {
+    const F32Seg& sg = args.seg[s];
+    // rows past m or n re-read the last one: not stored
+    const float *a[MA], *b[4];
+#pragma unroll
+    for (int i = 0; i < MA; ++i) a[i] = sg.a + min((int64_t)(lr + 8 * i), p.m - 1) * sg.lda + 4 * lc;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) b[i] = sg.b[grp] + min(n0 + lr + 8 * i, n_grp - 1) * sg.ldb[grp] + 4 * lc;
+    const int64_t first = (wave - seg0 % NW + NW) % NW, last = sg.ktiles - 1;
+    f32x4 fa[SETS][MA], fb[SETS][4];  // sets are named at compile time: registers
+    auto load = [&](auto set, int64_t kt) {
+      constexpr int f = decltype(set)::value;
+      const int64_t k = (kt < last ? kt : last) * kBK;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) fb[f][i] = *(const f32x4*)(b[i] + k);
+#pragma unroll
+      for (int i = 0; i < MA; ++i) fa[f][i] = *(const f32x4*)(a[i] + k);
+    };
+    auto mul = [&](auto set) {
+      constexpr int f = decltype(set)::value;
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mine[(lr + 8 * i) * 8 + swz8(lr + 8 * i, lc)] = fb[f][i];
+#pragma unroll
+      for (int i = 0; i < MA; ++i) mine[(32 + lr + 8 * i) * 8 + swz8(lr + 8 * i, lc)] = fa[f][i];
+      __builtin_amdgcn_wave_barrier();  // a wavefront's LDS accesses run in order
+      const int rb = lane & 31, ra = lane & (MR - 1);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int chunk = 4 * (lane >> 5) + c;
+        const f32x4 x = mine[(32 + ra) * 8 + swz8(ra, chunk)], y = mine[rb * 8 + swz8(rb, chunk)];
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x.x, y.x, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x.y, y.y, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x.z, y.z, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x.w, y.w, acc, 0, 0, 0);
+      }
+    };
+    if (first <= last) {
+      constexpr std::integral_constant<int, 0> s0{};
+      constexpr std::integral_constant<int, 1> s1{};
+      constexpr std::integral_constant<int, SETS - 1> s2{};  // SETS 2: s1 again, unused
+      int64_t kt = first;
+      auto turn = [&](auto set, int d) {
+        mul(set);
+        load(set, kt + (d + SETS) * NW);
+        __builtin_amdgcn_sched_barrier(0);  // the loads go out here, SETS steps ahead
+      };
+      load(s0, kt);
+      load(s1, kt + NW);
+      if constexpr (SETS > 2) load(s2, kt + 2 * NW);
+      for (; kt + (SETS - 1) * NW <= last; kt += SETS * NW) {
+        turn(s0, 0);
+        turn(s1, 1);
+        if constexpr (SETS > 2) turn(s2, 2);
+      }
+      if (kt <= last) mul(s0);
+      if (SETS > 2 && kt + NW <= last) mul(s1);
+    }
+    seg0 += sg.ktiles;
+  }
+  __syncthreads();
+  float* red = (float*)lds;  // [NW][16][64]
+#pragma unroll
+  for (int r = 0; r < 16; ++r) red[(wave * 16 + r) * 64 + lane] = acc[r];
+  __syncthreads();
+  float* out = p.c[grp];
+  const int64_t ld = p.ldc[grp];
+#pragma unroll
+  for (int e = threadIdx.x; e < 1024; e += 64 * NW) {
+    const int r = e >> 6, l = e & 63;
+    float v = red[r * 64 + l];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) v += red[(w * 16 + r) * 64 + l];
+    const int64_t row = 8 * (r >> 2) + 4 * (l >> 5) + (r & 3), col = n0 + (l & 31);
+    if (row < p.m && col < n_grp) {
+      float* q = out + row * ld + col;
+      *q = p.accumulate ? *q + v : v;
+    }
+  }
+}
+
+// At most 4 rows of A: on the vector units, where a row of A costs 1 us of
+// multiply-adds over those weights (the 32-row MFMA tile costs 16 to 20 us
+// whatever it holds).  A wavefront takes 4 columns, 256 k of each at a time
+// (a KB of consecutive memory a column), two such steps in flight, and adds
+// its lanes' sums at the end; KS 4: the workgroup's wavefronts share 4 columns
+// and take every fourth step, for fewer columns than keep the chip's
+// wavefronts busy.  One row: 23 us (5.8 TB/s), four: 32 us; 36 us on the
+// MFMA kernel.
+constexpr int kVecRows = 4, kVecCols = 4;
+
+template <int M, int KS>
+__global__ __launch_bounds__(256) void gemm_f32_vec_kernel(const F32Args args) {
+  __shared__ float red[4][kVecCols * M];
+  const Plan& p = args.p;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t groups0 = (p.n[0] + kVecCols - 1) / kVecCols;
+  const int64_t g = KS == 1 ? (int64_t)blockIdx.x * 4 + wave : (int64_t)blockIdx.x;  // column group
+  const int grp = g < groups0 ? 0 : 1;
+  const int64_t n0 = (g - (grp ? groups0 : 0)) * kVecCols, n_grp = p.n[grp];
+  if (n0 >= n_grp) return;  // past the last group (KS 1: no barrier follows)
+  float acc[kVecCols][M];
+#pragma unroll
+  for (int c = 0; c < kVecCols; ++c)
+#pragma unroll
+    for (int m = 0; m < M; ++m) acc[c][m] = 0.0f;
+  for (int s = 0; s < args.n_seg; ++s) {
+    const F32Seg& sg = args.seg[s];
+    const int64_t k_len = sg.ktiles * kBK;
+    const float* b[kVecCols];
+#pragma unroll
+    for (int c = 0; c < kVecCols; ++c) b[c] = sg.b[grp] + min(n0 + c, n_grp - 1) * sg.ldb[grp];
+    f32x4 fa[2][M], fb[2][kVecCols];
+    auto load = [&](auto set, int64_t k) {  // a lane past the end multiplies zeros
+      constexpr int f = decltype(set)::value;
+      const bool in = k < k_len;
+      const int64_t kk = in ? k : 0;
+#pragma unroll
+      for (int c = 0; c < kVecCols; ++c) fb[f][c] = *(const f32x4*)(b[c] + kk);
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        fa[f][m] = *(const f32x4*)(sg.a + (m < p.m ? m : 0) * sg.lda + kk);
+        if (!in) fa[f][m] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+      }
+      if (!in) {
+#pragma unroll
+        for (int c = 0; c < kVecCols; ++c) fb[f][c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+      }
+    };
+    auto mul = [&](auto set) {
+      constexpr int f = decltype(set)::value;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int c = 0; c < kVecCols; ++c)
+#pragma unroll
+          for (int m = 0; m < M; ++m) acc[c][m] = fmaf(fa[f][m][e], fb[f][c][e], acc[c][m]);
+    };
+    constexpr std::integral_constant<int, 0> s0{};
+    constexpr std::integral_constant<int, 1> s1{};
+    constexpr int STEP = 256 * KS;
+    const int64_t base = KS == 1 ? 0 : 256 * wave;  // uniform: the wavefront's first step
+    int64_t k = base;
+    if (k < k_len) load(s0, k + 4 * lane);
+    for (; k + STEP < k_len; k += 2 * STEP) {
+      load(s1, k + STEP + 4 * lane);
+      mul(s0);
+      load(s0, k + 2 * STEP + 4 * lane);
+      mul(s1);
+    }
+    if (k < k_len) mul(s0);
+  }
+#pragma unroll
+  for (int c = 0; c < kVecCols; ++c)
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+#pragma unroll
+      for (int o = 32; o >= 1; o >>= 1) acc[c][m] += __shfl_xor(acc[c][m], o);
+      if (lane == 0) red[wave][c * M + m] = acc[c][m];
+    }
+  int e = lane;
+  if constexpr (KS > 1) {
+    __syncthreads();
+    e = threadIdx.x;
+  } else {
+    __builtin_amdgcn_wave_barrier();  // a wavefront reads its own sums
+  }
+  if (e >= kVecCols * M) return;
+  float v = red[KS == 1 ? wave : 0][e];
+#pragma unroll
+  for (int w = 1; w < KS; ++w) v += red[w][e];
+  const int64_t row = e % M, col = n0 + e / M;
+  if (row < p.m && col < n_grp) {
+    float* q = p.c[grp] + row * p.ldc[grp] + col;
+    *q = p.accumulate ? *q + v : v;
+  }
 }
 
 // gemm_h3_kernel (eg_gemm_f16x3): fp32 accuracy from three products on the
@@ -1526,12 +1734,13 @@ int eg_gemm_bf16x6(const eg_gemm_operands* hi_mid, const eg_gemm_operands* hi_lo
                                    m, n, n2, c, ldc, c2, ldc2, 1, k_slices, workspace, workspace_bytes, stream);
 }
 
-int eg_gemm_f32(const eg_gemm_f32_operands* ops, int32_t n_seg, int64_t m, int64_t n, int64_t n2, float* c,
-                int64_t ldc, float* c2, int64_t ldc2, int32_t accumulate, int32_t k_slices, void* workspace,
-                int64_t workspace_bytes, void* stream) {
-  using namespace eg;
+}  // extern "C"
+
+namespace eg {
+namespace {
+// The kernel arguments of eg_gemm_f32(_rows) operands, checked.
+int f32_operands(const eg_gemm_f32_operands* ops, int32_t n_seg, int64_t n2, F32Args& g) {
   EG_CHECK_ARG(ops != nullptr && n_seg >= 0 && n_seg <= 2, "n_seg=%d", n_seg);
-  F32Args g{};
   for (int s = 0; s < n_seg; ++s) {
     const eg_gemm_f32_operands& o = ops[s];
     EG_CHECK_ARG(o.k >= 0 && o.k % 32 == 0, "segment %d: k must be a multiple of 32 (k=%lld)", s, (long long)o.k);
@@ -1555,8 +1764,75 @@ int eg_gemm_f32(const eg_gemm_f32_operands* ops, int32_t n_seg, int64_t m, int64
     sg.ktiles = o.k / 32;
     ++g.n_seg;
   }
+  return EG_OK;
+}
+}  // namespace
+}  // namespace eg
+
+extern "C" {
+
+int eg_gemm_f32(const eg_gemm_f32_operands* ops, int32_t n_seg, int64_t m, int64_t n, int64_t n2, float* c,
+                int64_t ldc, float* c2, int64_t ldc2, int32_t accumulate, int32_t k_slices, void* workspace,
+                int64_t workspace_bytes, void* stream) {
+  using namespace eg;
+  F32Args g{};
+  const int rc = f32_operands(ops, n_seg, n2, g);
+  if (rc != EG_OK) return rc;
   return launch_gemm<kF32BM, kF32BN>(kF32Shape, gemm_f32_kernel<kF32BM, kF32BN>, "gemm_f32_kernel", g, m, n, n2,
                                      c, ldc, c2, ldc2, accumulate, k_slices, workspace, workspace_bytes, stream);
+}
+
+int eg_gemm_f32_rows(const eg_gemm_f32_operands* ops, int32_t n_seg, int64_t m, int64_t n, int64_t n2, float* c,
+                     int64_t ldc, float* c2, int64_t ldc2, int32_t accumulate, void* stream) {
+  using namespace eg;
+  F32Args g{};
+  const int rc = f32_operands(ops, n_seg, n2, g);
+  if (rc != EG_OK) return rc;
+  EG_CHECK_ARG(m >= 0 && n >= 0 && n2 >= 0, "m=%lld n=%lld n2=%lld", (long long)m, (long long)n, (long long)n2);
+  if (m > kFewRows)
+    return set_error(EG_ERR_UNSUPPORTED, "eg_gemm_f32_rows of %lld rows (built: up to %d)", (long long)m, kFewRows);
+  if (m == 0 || n + n2 == 0) return EG_OK;
+  EG_CHECK_ARG(n == 0 || (c != nullptr && ldc >= n), "c / ldc");
+  EG_CHECK_ARG(n2 == 0 || (c2 != nullptr && ldc2 >= n2), "c2 / ldc2");
+  Plan& p = g.p;
+  p.c[0] = c;
+  p.c[1] = c2;
+  p.ldc[0] = ldc;
+  p.ldc[1] = ldc2;
+  p.m = m;
+  p.n[0] = n;
+  p.n[1] = n2;
+  p.accumulate = accumulate ? 1 : 0;
+  const int64_t blocks = (n + 31) / 32 + (n2 + 31) / 32;
+  EG_CHECK_ARG(blocks < (1LL << 31), "too many columns");
+  // sixteen wavefronts a workgroup where the columns are fewer than the CUs
+  const dim3 grid((unsigned)blocks);
+  hipStream_t st = (hipStream_t)stream;
+  if (m <= kVecRows) {
+    // one group of 4 columns a wavefront fills the 256 CUs with ten or more each from about
+    // 10,000 columns on; below, four wavefronts share a group
+    const int64_t groups = (n + kVecCols - 1) / kVecCols + (n2 + kVecCols - 1) / kVecCols;
+    const bool split = groups < 2560;
+    const dim3 vgrid((unsigned)(split ? groups : (groups + 3) / 4));
+    auto go = [&](auto rows) {
+      constexpr int M = decltype(rows)::value;
+      if (split) hipLaunchKernelGGL((gemm_f32_vec_kernel<M, 4>), vgrid, dim3(256), 0, st, g);
+      else hipLaunchKernelGGL((gemm_f32_vec_kernel<M, 1>), vgrid, dim3(256), 0, st, g);
+    };
+    if (m == 1) go(std::integral_constant<int, 1>{});
+    else if (m == 2) go(std::integral_constant<int, 2>{});
+    else go(std::integral_constant<int, 4>{});
+    return launch_status("gemm_f32_vec_kernel");
+  }
+  if (blocks <= 256 && m <= 8)
+    hipLaunchKernelGGL((gemm_f32_rows_kernel<16, 8, 3>), grid, dim3(1024), 0, st, g);
+  else if (blocks <= 256)
+    hipLaunchKernelGGL((gemm_f32_rows_kernel<16, 32, 2>), grid, dim3(1024), 0, st, g);
+  else if (m <= 8)
+    hipLaunchKernelGGL((gemm_f32_rows_kernel<8, 8, 3>), grid, dim3(512), 0, st, g);
+  else
+    hipLaunchKernelGGL((gemm_f32_rows_kernel<8, 32, 2>), grid, dim3(512), 0, st, g);
+  return launch_status("gemm_f32_rows_kernel");
 }
 
 }  // extern "C"

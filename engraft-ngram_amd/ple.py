@@ -419,13 +419,16 @@ def _f32_operand(x: torch.Tensor, kp: int) -> torch.Tensor:
 
 
 def gemm_f32(a, b, a2=None, b2=None, out: torch.Tensor | None = None, accumulate: bool = False,
-             b_n2=None, b2_n2=None, out2: torch.Tensor | None = None, k_slices: int | None = None):
+             b_n2=None, b2_n2=None, out2: torch.Tensor | None = None, k_slices: int | None = None,
+             few_rows: bool = False):
     """``a @ b.T (+ a2 @ b2.T)`` in fp32 arithmetic on the fp32 matrix cores
     (``eg_gemm_f32``): the products of an fp32 matmul, accumulated in fp32.
     Operands and the column groups, K segments and K slices as
     :func:`gemm_x3`, every operand an fp32 tensor (a ``k`` not a multiple of
-    32 is zero-padded in a copy).  Returns ``out``, or ``(out, out2)`` with a
-    second column group."""
+    32 is zero-padded in a copy).  ``few_rows``: the kernels for at most
+    ``FEW_ROWS`` rows of ``a`` (``eg_gemm_f32_rows``; a row's sums are then taken
+    in an order that depends on ``m``).  Returns ``out``, or ``(out, out2)`` with
+    a second column group."""
     raw = [(a, b, b_n2)] + ([(a2, b2, b2_n2)] if a2 is not None else [])
     m, n = a.shape[0], b.shape[0]
     n2 = 0 if b_n2 is None else b_n2.shape[0]
@@ -462,6 +465,10 @@ def gemm_f32(a, b, a2=None, b2=None, out: torch.Tensor | None = None, accumulate
 
     out = _out(out, m, n, "out")
     out2 = _out(out2, m, n2, "out2") if n2 else None
+    if few_rows:
+        _lib.call("eg_gemm_f32_rows", ops, len(raw), m, n, n2, _lib.ptr(out), max(out.stride(0), n), _lib.ptr(out2),
+                  max(out2.stride(0), n2) if n2 else 0, int(accumulate), _lib.stream_ptr(dev))
+        return (out, out2) if n2 else out
     slices, ws, ws_bytes = _gemm_workspace(m, n, n2, 32 * k_tiles, k_slices, dev, "eg_gemm_f32_workspace_size")
     _lib.call("eg_gemm_f32", ops, len(raw), m, n, n2, _lib.ptr(out), max(out.stride(0), n),
               _lib.ptr(out2), max(out2.stride(0), n2) if n2 else 0, int(accumulate), slices, _lib.ptr(ws),
@@ -476,6 +483,19 @@ def gemm_f32(a, b, a2=None, b2=None, out: torch.Tensor | None = None, accumulate
 # of the key moves the hidden, key and norm gradients by far more than its own
 # size (1e-4 at |s| 0.03).
 H3_MIN_ROWS = 64
+
+# Up to this many positions every gemm= runs eg_gemm_f32_rows: reading the weights
+# bounds such a product, it reads them once as they are (4 bytes a weight against 4 to
+# 6 of planes; one position 23 us, 32 positions 44 us, against 115 us for gemm_x6 and 147 us
+# for gemm_f32), and its arithmetic is the most precise of the three
+FEW_ROWS = 32
+
+
+def _f32_in_place(*ws: torch.Tensor) -> bool:
+    """eg_gemm_f32 reads these fp32 matrices where they are (``_f32_operand`` makes no copy)."""
+    return all(w.shape[1] % 32 == 0 and w.stride(1) == 1 and w.stride(0) % 4 == 0 and w.data_ptr() % 16 == 0
+               for w in ws)
+
 
 WGRAD_MAX_TAPS = 8  # eg_ple_weight_grads' built tap counts (1..8)
 
@@ -500,6 +520,8 @@ def _projection_backward(gemm: str, pairs: list) -> torch.Tensor:
         ds, ws = zip(*pairs)
         return gemm_h3(ds, tuple(w.T for w in ws), planes_b=_HALF.get(ws, True))
     flat = [x for d, w in pairs for x in (d, _WT.get(w))]
+    if pairs[0][0].shape[0] <= FEW_ROWS and _f32_in_place(*flat[1::2]):
+        return gemm_f32(*flat, few_rows=True)
     if gemm == "bf16x3":
         return gemm_x3(*flat, cache_b=True)
     if gemm == "bf16x6":
@@ -528,7 +550,9 @@ class _PleFn(torch.autograd.Function):
         emb32 = emb.to(**f32).contiguous()
         wk32 = w_key.to(**f32)
         wv32 = w_value.to(**f32)
-        if gemm == "bf16x3":
+        if t_len <= FEW_ROWS and _f32_in_place(wk32, wv32):
+            key, value = gemm_f32(emb32, wk32, b_n2=wv32, few_rows=True)
+        elif gemm == "bf16x3":
             key, value = gemm_x3(SplitPlanes(emb32), wk32, cache_b=True, b_n2=wv32)
         elif gemm == "bf16x6" and t_len > H3_MIN_ROWS and not any(ctx.needs_input_grad):
             key, value = gemm_h3((emb32,), (wk32,), (wv32,), planes_b=_HALF.get((wk32,), False),

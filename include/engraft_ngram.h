@@ -35,7 +35,7 @@
  *   eg_ple_gate, eg_ple_conv(_gated)  ple_forward after its two projections
  *   (+ _backward)    and the autograd of it          engraft/replica/layers.py:565-626
  *   eg_ple_rms, eg_ple_conv's other modes  PleReplica engraft/lens.py:221-385
- *   eg_split_bf16, eg_gemm_bf16x3, eg_gemm_f32 (+ _workspace_size),
+ *   eg_split_bf16, eg_gemm_bf16x3, eg_gemm_f32 (+ _rows, _workspace_size),
  *   eg_split_bf16x6, eg_gemm_bf16x6, eg_split_f16, eg_gemm_f16x3
  *                    ple_forward's projections and their backward
  *                                                    engraft/replica/layers.py:594-606
@@ -614,6 +614,12 @@ int64_t eg_gemm_f32_workspace_size(int64_t m, int64_t n, int64_t n2, int64_t k, 
 int eg_gemm_f32(const eg_gemm_f32_operands* ops, int32_t n_seg, int64_t m, int64_t n, int64_t n2, float* c,
                 int64_t ldc, float* c2, int64_t ldc2, int32_t accumulate, int32_t k_slices, void* workspace,
                 int64_t workspace_bytes, void* stream);
+
+/* eg_gemm_f32 of at most 32 rows (EG_ERR_UNSUPPORTED past them), bound by
+ * reading B once: no workspace.  Its sums are taken in another order than
+ * eg_gemm_f32's, one that depends on m (deterministic for one m). */
+int eg_gemm_f32_rows(const eg_gemm_f32_operands* ops, int32_t n_seg, int64_t m, int64_t n, int64_t n2, float* c,
+                     int64_t ldc, float* c2, int64_t ldc2, int32_t accumulate, void* stream);
 
 /* Part of an operand of eg_gemm_f16x3: fp32 [rows, cols], element (r, k) at
  * x[r * row_stride + k * col_stride] (a transposed matrix has row_stride 1). */
