@@ -165,6 +165,11 @@ SIGNATURES = {
     "eg_ple_weight_grads_workspace_size": (ctypes.c_size_t, [c_int64, c_int32, c_int32, c_int32]),
     "eg_ple_weight_grads": (c_int32, [c_void_p] * 11 + [c_int64, c_void_p, c_int64, c_int32, c_int32, c_int32,
                                                         c_int32] + [c_void_p] * 5 + [ctypes.c_size_t, c_void_p]),
+    "eg_ple_weight_sums_workspace_size": (ctypes.c_size_t, [c_int64, c_int64, c_int32, c_int32]),
+    "eg_ple_conv_backward_sums": (c_int32, [c_void_p, c_int64, c_int64, c_int32, c_int32] + [c_void_p] * 8 +
+                                  [c_int64, c_void_p, c_void_p, ctypes.c_size_t, c_void_p]),
+    "eg_ple_weight_sums": (c_int32, [c_void_p] * 6 + [c_int64, c_int64, c_int32, c_int32] + [c_void_p] * 5 +
+                           [ctypes.c_size_t, c_void_p]),
     "eg_ple_conv": (c_int32, [c_void_p, c_int64, c_int64, c_int32, c_int32, c_void_p, c_int32, c_int32, c_int32,
                               c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "eg_ple_conv_gated": (c_int32, [c_void_p, c_int64, c_int64, c_int32, c_int32, c_void_p, c_void_p, c_void_p,

@@ -636,6 +636,196 @@ __global__ __launch_bounds__(256) void ple_conv_bwd_kernel(const float* __restri
   }
 }
 
+// ple_conv_bwd_kernel with the forward's pre-activation, for 4 taps at
+// dilation 3 (the model's): a thread walks kBwdRows rows of its channel, nine at
+// a time, the d_acc of the nine rows at hand and of the next nine in
+// registers, so that pre and d_out are read once (and nine rows twice, 14 %)
+// and nothing passes through LDS: bound by HBM.  SUMS (workgroups of one
+// stream: n a multiple of 256): the chunk's partial sums of the normed rows'
+// weight and of the taps as well (ple_wgrad_part_kernel's), from value, gate
+// and the factor r_g, which give the normed rows the taps met, and from the
+// d_normed just formed: one pass over pre, d_out and value in place of two
+// over them, the normed rows and d_normed.  1,531 positions of 4 x 2560:
+// 68 us and 35 us for ple_norm_grads_part_kernel, against 83 us and 166 us for
+// ple_conv_bwd_kernel and ple_wgrad_part_kernel.
+constexpr int kBwdRows = 63;  // a multiple of the nine rows of a turn
+
+template <bool SUMS>
+__global__ __launch_bounds__(256) void ple_conv_bwd_run_kernel(
+    const float* __restrict__ hist, int64_t hist_rows, int64_t T, int hc, int n, const float* __restrict__ value,
+    const float* __restrict__ gate, const float* __restrict__ rstd, const float* __restrict__ norm_conv,
+    const float* __restrict__ conv_w, const float* __restrict__ pre, const float* __restrict__ d_out,
+    const float* __restrict__ d_tail, int64_t tail_rows, float* __restrict__ d_full, float* __restrict__ part) {
+#pragma clang fp contract(off)
+  constexpr int TAPS = 4, DIL = 3, H = (TAPS - 1) * DIL;
+  __shared__ float s_gate[kBwdRows + H], s_rg[kBwdRows + H];
+  const int C = hc * n;
+  const int c = blockIdx.x * 256 + threadIdx.x;
+  const int64_t R = hist_rows + T, r0 = (int64_t)blockIdx.y * kBwdRows, r1 = min(r0 + kBwdRows, R);
+  const int64_t t0 = r0 - hist_rows;  // row r is position r - hist_rows
+  const int j = c / n, i = c - j * n;
+  if constexpr (SUMS) {
+    if (threadIdx.x < kBwdRows + H) {
+      const int64_t t = t0 - H + threadIdx.x;
+      const int64_t pj = (t < 0 ? 0 : min(t, T - 1)) * hc + j;
+      s_gate[threadIdx.x] = gate[pj];
+      s_rg[threadIdx.x] = rstd[pj * 3 + 2];
+    }
+    __syncthreads();
+  }
+  if (c >= C) return;
+  float w[TAPS];
+#pragma unroll
+  for (int k = 0; k < TAPS; ++k) w[k] = conv_w[(int64_t)c * TAPS + k];
+  const float nc = SUMS ? norm_conv[c] : 0.0f;
+  // nine positions' loads, and their d_acc (zero outside [0, T))
+  float pa[H], dv[H], vv[H];
+  auto load = [&](int64_t t) {
+#pragma unroll
+    for (int b = 0; b < H; ++b) {
+      const int64_t tt = min(max(t + b, (int64_t)0), T - 1);
+      pa[b] = pre[tt * C + c];
+      dv[b] = d_out[tt * C + c];
+    }
+  };
+  auto form = [&](int64_t t, float* da) {
+#pragma unroll
+    for (int b = 0; b < H; ++b) {
+      const float sg = 1.0f / (1.0f + expf(-pa[b]));
+      da[b] = t + b >= 0 && t + b < T ? dv[b] * (sg * (1.0f + pa[b] * (1.0f - sg))) : 0.0f;
+    }
+  };
+  // nine rows of [history; normed] and, of the positions among them, gated * r_g
+  auto load_value = [&](int64_t t) {
+#pragma unroll
+    for (int b = 0; b < H; ++b) {
+      const int64_t tb = t + b, r = hist_rows + tb;
+      if (tb >= 0) vv[b] = value[min(tb, T - 1) * n + i];
+      else vv[b] = r >= 0 ? hist[r * C + c] : 0.0f;
+    }
+  };
+  auto rows = [&](int64_t t, float* x, float* y) {
+#pragma unroll
+    for (int b = 0; b < H; ++b) {
+      const int q = (int)(t + b - t0) + H;  // past the table only past the chunk: not used
+      const float z = (vv[b] * s_gate[min(q, kBwdRows + H - 1)]) * s_rg[min(q, kBwdRows + H - 1)];
+      x[b] = t + b >= 0 ? z * nc : vv[b];
+      y[b] = z;
+    }
+  };
+  float cur[H], next[H], before[H], now[H], z[H];
+  float a_nc = 0.0f, a_w[TAPS] = {};
+  load(t0);
+  if constexpr (SUMS) load_value(t0 - H);
+  form(t0, cur);
+  load(t0 + H);
+  if constexpr (SUMS) {
+    rows(t0 - H, before, z);
+    load_value(t0);
+  }
+  for (int64_t r = r0; r < r1; r += H) {
+    const int64_t t = r - hist_rows;
+    form(t + H, next);
+    if constexpr (SUMS) rows(t, now, z);
+    if (r + H < r1) {
+      load(t + 2 * H);
+      if constexpr (SUMS) load_value(t + H);
+    }
+#pragma unroll
+    for (int b = 0; b < H; ++b) {
+      if (r + b >= r1) break;
+      float g = 0.0f;
+#pragma unroll
+      for (int k = 0; k < TAPS; ++k) {
+        const int d = (TAPS - 1 - k) * DIL;  // the tap at distance d read this row for position t + b + d
+        if (t + b + d >= 0 && t + b + d < T) g += w[k] * (b + d < H ? cur[b + d] : next[b + d - H]);
+      }
+      if (d_tail != nullptr && r + b >= R - tail_rows) g += d_tail[(r + b - (R - tail_rows)) * C + c];
+      d_full[(r + b) * C + c] = g;
+      if constexpr (SUMS) {
+        if (t + b >= 0) {
+          a_nc += g * z[b];
+#pragma unroll
+          for (int k = 0; k < TAPS; ++k) {
+            const int d = (TAPS - 1 - k) * DIL;
+            if (r + b - d >= 0) a_w[k] += cur[b] * (b - d >= 0 ? now[b - d] : before[b - d + H]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < H; ++b) {
+      cur[b] = next[b];
+      before[b] = now[b];
+    }
+  }
+  if constexpr (SUMS) {
+    float* o = part + ((int64_t)blockIdx.y * (3 + TAPS) + 2) * C + c;
+    o[0] = a_nc;
+#pragma unroll
+    for (int k = 0; k < TAPS; ++k) o[(1 + (int64_t)k) * C] = a_w[k];
+  }
+}
+
+// The key and query norms' weights' partial sums over the same chunks of rows:
+// key and hidden read once, eight positions' loads at a time.
+__global__ __launch_bounds__(256) void ple_norm_grads_part_kernel(
+    const float* __restrict__ key, const float* __restrict__ hidden, const float* __restrict__ rstd,
+    const float* __restrict__ d_s, const float* __restrict__ norm_key, const float* __restrict__ norm_query,
+    int64_t hist_rows, int64_t T, int hc, int n, int Q, float inv_sqrt_n, float* __restrict__ part) {
+#pragma clang fp contract(off)
+  __shared__ float s_rk[kBwdRows], s_rq[kBwdRows], s_ds[kBwdRows];
+  constexpr int B = 8;
+  const int C = hc * n;
+  const int c = blockIdx.x * 256 + threadIdx.x;  // n a multiple of 256: one stream, whole wavefronts
+  const int j = c / n;
+  const int64_t r0 = (int64_t)blockIdx.y * kBwdRows;
+  const int64_t t0 = max(r0 - hist_rows, (int64_t)0), t1 = min(r0 + kBwdRows - hist_rows, T);
+  if (t0 + threadIdx.x < t1) {
+    const int64_t pj = (t0 + threadIdx.x) * hc + j;
+    s_rk[threadIdx.x] = rstd[pj * 3 + 0];
+    s_rq[threadIdx.x] = rstd[pj * 3 + 1];
+    s_ds[threadIdx.x] = d_s[pj] * inv_sqrt_n;
+  }
+  __syncthreads();
+  const float nk = norm_key[c], nq = norm_query[c];
+  float a_nk = 0.0f, a_nq = 0.0f, k[2][B], h[2][B];
+  auto load = [&](auto set, int64_t t) {
+    constexpr int f = decltype(set)::value;
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const int64_t e = min(t + b, T - 1) * C + c;
+      k[f][b] = key[e];
+      h[f][b] = hidden[e];
+    }
+  };
+  auto add = [&](auto set, int64_t t) {
+    constexpr int f = decltype(set)::value;
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      if (t + b >= t1) break;
+      const int q = (int)(t + b - t0);
+      const float kr = k[f][b] * s_rk[q], hr = h[f][b] * s_rq[q], dsn = s_ds[q];
+      a_nk += (dsn * (hr * nq)) * kr;
+      a_nq += (dsn * (kr * nk)) * hr;
+    }
+  };
+  constexpr std::integral_constant<int, 0> s0{};
+  constexpr std::integral_constant<int, 1> s1{};
+  if (t0 < t1) {
+    load(s0, t0);
+    for (int64_t t = t0; t < t1; t += 2 * B) {
+      load(s1, t + B);
+      add(s0, t);
+      load(s0, t + 2 * B);
+      add(s1, t + B);
+    }
+  }
+  float* o = part + (int64_t)blockIdx.y * Q * C + c;
+  o[0] = a_nk;
+  o[C] = a_nq;
+}
+
 // ple_gate_bwd_kernel: one workgroup of 1024 threads per position, every
 // stream (hc <= 4, n <= 4096).  With x = value * gate_j (gated), y = normed,
 // dy = d_normed, r = the forward's RMS factors:
@@ -1182,7 +1372,12 @@ int eg_ple_conv_backward(const float* full, int64_t hist_rows, int64_t n_pos, in
   const int64_t blocks = (int64_t)((hc * n_embd + 255) / 256) * ((rows + kConvBwdRun - 1) / kConvBwdRun);
   EG_CHECK_ARG(blocks < (1LL << 32), "too many elements");
   const size_t lds = (size_t)(kConvBwdRun + (taps - 1) * dilation) * 256 * sizeof(float);
-  if (pre != nullptr)
+  const int64_t runs = (rows + kBwdRows - 1) / kBwdRows;
+  if (pre != nullptr && taps == 4 && dilation == 3 && n_pos > 0 && runs < 65536)
+    hipLaunchKernelGGL(ple_conv_bwd_run_kernel<false>, dim3((unsigned)((hc * n_embd + 255) / 256), (unsigned)runs),
+                       dim3(256), 0, (hipStream_t)stream, nullptr, hist_rows, n_pos, hc, n_embd, nullptr, nullptr,
+                       nullptr, nullptr, conv_w, pre, d_out, tail_rows ? d_tail : nullptr, tail_rows, d_full, nullptr);
+  else if (pre != nullptr)
     hipLaunchKernelGGL(ple_conv_bwd_kernel<true>, dim3((unsigned)blocks), dim3(256), lds, (hipStream_t)stream, full,
                        hist_rows, n_pos, hc, n_embd, conv_w, taps, dilation, pre, d_out, tail_rows ? d_tail : nullptr,
                        tail_rows, d_full);
@@ -1251,6 +1446,62 @@ int eg_ple_gate_backward_planes(const float* key, const float* value, const floa
                      detach_gate ? nullptr : (float*)d_key_hi, detach_value ? nullptr : (float*)d_value_hi, d_hidden,
                      (__bf16*)d_key_lo, (__bf16*)d_value_lo, d_s);
   return launch_status("ple_gate_bwd_vec_kernel");
+}
+
+size_t eg_ple_weight_sums_workspace_size(int64_t hist_rows, int64_t n_pos, int32_t hc, int32_t n_embd) {
+  if (n_pos <= 0 || hist_rows < 0 || hc < 1 || n_embd < 1) return 0;
+  return (size_t)((hist_rows + n_pos + kBwdRows - 1) / kBwdRows) * 7 * (size_t)hc * (size_t)n_embd * 4;
+}
+
+static int weight_sums_shape(int64_t hist_rows, int64_t n_pos, int32_t hc, int32_t n_embd, const void* workspace,
+                             size_t workspace_bytes) {
+  EG_CHECK_ARG(n_pos >= 1 && n_pos < (1LL << 31) && hist_rows >= 0 && hc >= 1 && n_embd >= 1,
+               "n_pos=%lld hist_rows=%lld hc=%d n_embd=%d", (long long)n_pos, (long long)hist_rows, hc, n_embd);
+  if (n_embd % 256 != 0 || hist_rows + n_pos > 65535LL * kBwdRows)
+    return set_error(EG_ERR_UNSUPPORTED, "weight sums for n_embd=%d, %lld rows (built: n_embd a multiple of 256, up to "
+                     "%lld rows)", n_embd, (long long)(hist_rows + n_pos), 65535LL * kBwdRows);
+  EG_CHECK_ARG((int64_t)hc * n_embd < (1LL << 31), "too many columns");
+  const size_t need = eg_ple_weight_sums_workspace_size(hist_rows, n_pos, hc, n_embd);
+  if (workspace_bytes < need)
+    return set_error(EG_ERR_WORKSPACE, "workspace of %zu bytes < %zu needed", workspace_bytes, need);
+  EG_CHECK_ARG(workspace != nullptr, "workspace is NULL");
+  return EG_OK;
+}
+
+int eg_ple_conv_backward_sums(const float* hist, int64_t hist_rows, int64_t n_pos, int32_t hc, int32_t n_embd,
+                              const float* value, const float* gate, const float* rstd, const float* norm_conv,
+                              const float* conv_w, const float* pre, const float* d_out, const float* d_tail,
+                              int64_t tail_rows, float* d_full, void* workspace, size_t workspace_bytes,
+                              void* stream) {
+  const int rc = weight_sums_shape(hist_rows, n_pos, hc, n_embd, workspace, workspace_bytes);
+  if (rc != EG_OK) return rc;
+  EG_CHECK_ARG((hist || hist_rows == 0) && value && gate && rstd && norm_conv && conv_w && pre && d_out && d_full,
+               "NULL argument");
+  EG_CHECK_ARG(tail_rows >= 0 && tail_rows <= hist_rows + n_pos && (tail_rows == 0 || d_tail != nullptr),
+               "tail_rows=%lld", (long long)tail_rows);
+  const int64_t runs = (hist_rows + n_pos + kBwdRows - 1) / kBwdRows;
+  hipLaunchKernelGGL(ple_conv_bwd_run_kernel<true>, dim3((unsigned)(hc * n_embd / 256), (unsigned)runs), dim3(256), 0,
+                     (hipStream_t)stream, hist, hist_rows, n_pos, hc, n_embd, value, gate, rstd, norm_conv, conv_w, pre,
+                     d_out, tail_rows ? d_tail : nullptr, tail_rows, d_full, (float*)workspace);
+  return launch_status("ple_conv_bwd_run_kernel");
+}
+
+int eg_ple_weight_sums(const float* key, const float* hidden, const float* rstd, const float* d_s,
+                       const float* norm_key, const float* norm_query, int64_t hist_rows, int64_t n_pos, int32_t hc,
+                       int32_t n_embd, float* d_norm_key, float* d_norm_query, float* d_norm_conv, float* d_conv_w,
+                       void* workspace, size_t workspace_bytes, void* stream) {
+  const int rc = weight_sums_shape(hist_rows, n_pos, hc, n_embd, workspace, workspace_bytes);
+  if (rc != EG_OK) return rc;
+  EG_CHECK_ARG(key && hidden && rstd && d_s && norm_key && norm_query, "NULL argument");
+  const int C = hc * n_embd, Q = 7;
+  const int64_t runs = (hist_rows + n_pos + kBwdRows - 1) / kBwdRows, total = (int64_t)Q * C;
+  hipStream_t st = (hipStream_t)stream;
+  hipLaunchKernelGGL(ple_norm_grads_part_kernel, dim3((unsigned)(C / 256), (unsigned)runs), dim3(256), 0, st, key,
+                     hidden, rstd, d_s, norm_key, norm_query, hist_rows, n_pos, hc, n_embd, Q,
+                     (float)(1.0 / sqrt((double)n_embd)), (float*)workspace);
+  hipLaunchKernelGGL(ple_wgrad_sum_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
+                     (const float*)workspace, runs, Q, C, 4, d_norm_key, d_norm_query, d_norm_conv, d_conv_w);
+  return launch_status("ple_norm_grads kernels");
 }
 
 size_t eg_ple_weight_grads_workspace_size(int64_t n_pos, int32_t hc, int32_t n_embd, int32_t taps) {

@@ -571,9 +571,8 @@ class _PleFn(torch.autograd.Function):
         taps = conv32.shape[1]
         native = any(ctx.needs_input_grad) and _native_backward_ok(hc, n, taps, int(dil),
                                                                    weights=any(ctx.needs_input_grad[2:8]))
-        # without the normed rows in memory where the gated convolution is built and no
-        # weight's gradient reads them
-        gated = (taps == 4 and int(dil) == 3 and n % 256 == 0 and not any(ctx.needs_input_grad[2:8])
+        # without the normed rows in memory where the gated convolution is built
+        gated = (taps == 4 and int(dil) == 3 and n % 256 == 0 and t_len > 0
                  and not (hidden32.data_ptr() | hist.data_ptr() | nc32.data_ptr() | conv32.data_ptr()) % 16)
         rstd = torch.empty((t_len, hc, 3), **f32) if native or gated else None
         full = None if gated else torch.empty((h0 + t_len, hc * n), **f32)
@@ -585,8 +584,6 @@ class _PleFn(torch.autograd.Function):
         if gated:
             hist32 = hist.to(**f32).contiguous()
             new_hist = torch.empty((min(9, h0 + t_len), hc, n), **f32)
-            if t_len == 0:
-                new_hist.copy_(hist32[h0 - new_hist.shape[0]:])
             _lib.call("eg_ple_conv_gated", _lib.ptr(hist32), h0, t_len, hc, n, _lib.ptr(value), _lib.ptr(gate),
                       _lib.ptr(rstd), _lib.ptr(nc32), _lib.ptr(conv32), taps, int(dil), _lib.ptr(hidden32),
                       _lib.ptr(out), _lib.ptr(pre), _lib.ptr(new_hist), st)
@@ -598,13 +595,17 @@ class _PleFn(torch.autograd.Function):
                       _lib.ptr(hidden32), _lib.ptr(value), _lib.ptr(gate), _lib.ptr(out), _lib.ptr(pre), st)
             hist_len = (taps - 1) * int(dil)
             new_hist = (full[-hist_len:] if hist_len > 0 else full[:0]).reshape(-1, hc, n).to(hidden.dtype).clone()
+        ctx.set_materialize_grads(False)  # s, gate and value get no gradient: none is filled for them
         ctx.native = native
         ctx.hist_rows = h0
         if native:
             # emb for the projection weights' gradients
             emb_w = emb32 if any(ctx.needs_input_grad[2:4]) else None
-            ctx.save_for_backward(key, value, hidden32, full, s, gate, rstd, nk32, nq32, nc32, conv32, wk32, wv32, pre,
+            # the rows the taps' gradients meet: all of them, or the history alone
+            rows = hist32 if gated else full
+            ctx.save_for_backward(key, value, hidden32, rows, s, gate, rstd, nk32, nq32, nc32, conv32, wk32, wv32, pre,
                                   emb_w)
+            ctx.gated = gated
             ctx.dtypes = (emb.dtype, hidden.dtype, hist.dtype)
             ctx.w_dtypes = tuple(x.dtype for x in (w_key, w_value, nk, nq, nc, conv))
             ctx.tail_rows = new_hist.shape[0]
@@ -617,6 +618,9 @@ class _PleFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, d_out, d_hist, _d_s, _d_gate, _d_value):
+        if d_out is None:  # the loss reaches the new history alone
+            like = ctx.saved_tensors[2] if ctx.native else ctx.saved_tensors[1]  # hidden
+            d_out = torch.zeros_like(like)
         if ctx.native:
             return _PleFn._backward_native(ctx, d_out, d_hist)
         inputs = ctx.saved_tensors
@@ -651,12 +655,21 @@ class _PleFn(torch.autograd.Function):
         tail = ctx.tail_rows if (d_hist is not None and ctx.tail_rows > 0) else 0
         d_tail = d_hist.to(**f32).reshape(tail, c_dim).contiguous() if tail else None
         d_full = torch.empty((h0 + t_len, c_dim), **f32)
-        _lib.call("eg_ple_conv_backward", _lib.ptr(full), h0, t_len, hc, n, _lib.ptr(conv32), conv32.shape[1],
-                  int(dil), _lib.ptr(pre), _lib.ptr(d_out32), _lib.ptr(d_tail), tail, _lib.ptr(d_full), st)
-        d_hidden = torch.empty((t_len, hc, n), **f32) if need_hidden else None
         need_w = ctx.needs_input_grad[2:8]
+        sums = None  # the weight sums' workspace, from the convolution's backward on
+        if ctx.gated and any(need_w[2:]):
+            ws_bytes = int(_lib.load().eg_ple_weight_sums_workspace_size(h0, t_len, hc, n))
+            sums = torch.empty(ws_bytes // 4, **f32)
+            _lib.call("eg_ple_conv_backward_sums", _lib.ptr(full), h0, t_len, hc, n, _lib.ptr(value), _lib.ptr(gate),
+                      _lib.ptr(rstd), _lib.ptr(nc32), _lib.ptr(conv32), _lib.ptr(pre), _lib.ptr(d_out32),
+                      _lib.ptr(d_tail), tail, _lib.ptr(d_full), _lib.ptr(sums), ws_bytes, st)
+        else:
+            _lib.call("eg_ple_conv_backward", None if ctx.gated else _lib.ptr(full), h0, t_len, hc, n,
+                      _lib.ptr(conv32), conv32.shape[1], int(dil), _lib.ptr(pre), _lib.ptr(d_out32),
+                      _lib.ptr(d_tail), tail, _lib.ptr(d_full), st)
+        d_hidden = torch.empty((t_len, hc, n), **f32) if need_hidden else None
         if any(need_w):
-            return _PleFn._backward_with_weights(ctx, d_out32, d_full, d_hidden)
+            return _PleFn._backward_with_weights(ctx, d_out32, d_full, d_hidden, sums)
         if ctx.gemm == "bf16x3" and n % 256 == 0:
             # d_key and d_value straight into the bf16 planes gemm_x3 takes
             pk = _empty_planes(t_len, c_dim, dev) if (need_emb and not detach_gate) else None
@@ -697,19 +710,21 @@ class _PleFn(torch.autograd.Function):
 
 
     @staticmethod
-    def _backward_with_weights(ctx, d_out32, d_full, d_hidden):
+    def _backward_with_weights(ctx, d_out32, d_full, d_hidden, sums):
         """The HIP backward with the weights' gradients too: the gate backward
         in fp32 (its d_key / d_value also feed the projection weights'
         gradients, and its score gradient d_s the norm weights'), the two
         weight GEMMs ``d_w_key = d_key^T emb`` and ``d_w_value = d_value^T emb``,
-        and ``eg_ple_weight_grads`` for the norms and the convolution."""
+        and ``eg_ple_weight_grads`` for the norms and the convolution
+        (``eg_ple_weight_sums`` on the partial sums ``sums`` that the convolution's
+        backward began)."""
         key, value, hidden32, full, s, gate, rstd, nk32, nq32, nc32, conv32, wk32, wv32, pre, emb32 = ctx.saved_tensors
         _eps, dil, detach_value, detach_gate = ctx.cfg
         emb_dt, hidden_dt, hist_dt = ctx.dtypes
         t_len, hc, n = hidden32.shape
         c_dim = hc * n
-        h0 = full.shape[0] - t_len
-        dev = full.device
+        h0 = ctx.hist_rows
+        dev = hidden32.device
         f32 = dict(dtype=torch.float32, device=dev)
         st = _lib.stream_ptr(dev)
         need = ctx.needs_input_grad
@@ -737,8 +752,14 @@ class _PleFn(torch.autograd.Function):
         d_nk = d_nq = d_nc = d_cv = None
         if need_nk or need_nq or need_nc or need_cv:
             taps = conv32.shape[1]
-            outs = [torch.zeros(c_dim, **f32) for _ in range(3)] + [torch.zeros((c_dim, taps), **f32)]
-            if t_len > 0:
+            if sums is not None:
+                outs = [torch.empty(c_dim, **f32) for _ in range(3)] + [torch.empty((c_dim, taps), **f32)]
+                _lib.call("eg_ple_weight_sums", _lib.ptr(key), _lib.ptr(hidden32), _lib.ptr(rstd), _lib.ptr(d_s),
+                          _lib.ptr(nk32), _lib.ptr(nq32), h0, t_len, hc, n, *[_lib.ptr(o) for o in outs],
+                          _lib.ptr(sums), sums.numel() * 4, st)
+            else:
+                outs = [torch.zeros(c_dim, **f32) for _ in range(3)] + [torch.zeros((c_dim, taps), **f32)]
+            if t_len > 0 and sums is None:
                 ws_bytes = int(_lib.load().eg_ple_weight_grads_workspace_size(t_len, hc, n, taps))
                 ws = torch.empty(max(ws_bytes // 4, 1), **f32)
                 _lib.call("eg_ple_weight_grads", _lib.ptr(key), _lib.ptr(value), _lib.ptr(hidden32), _lib.ptr(gate),

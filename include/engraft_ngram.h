@@ -508,6 +508,26 @@ int eg_ple_weight_grads(const float* key, const float* value, const float* hidde
                         float* d_norm_key, float* d_norm_query, float* d_norm_conv,
                         float* d_conv_w, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same gradients in two calls around eg_ple_gate_backward, for 4 taps at
+ * dilation 3 and n_embd a multiple of 256 (EG_ERR_UNSUPPORTED otherwise):
+ * eg_ple_conv_backward_sums is eg_ple_conv_backward (hist the history rows; the
+ * normed rows are formed from value, gate, rstd and norm_conv) and leaves the
+ * norm_conv and conv1d gradients' partial sums in the workspace, which
+ * eg_ple_weight_sums completes with those of norm_key and norm_query and adds
+ * up in chunk order (any output may be NULL).  The same hist_rows, n_pos >= 1
+ * and workspace (eg_ple_weight_sums_workspace_size bytes) in both. */
+size_t eg_ple_weight_sums_workspace_size(int64_t hist_rows, int64_t n_pos, int32_t hc, int32_t n_embd);
+int eg_ple_conv_backward_sums(const float* hist, int64_t hist_rows, int64_t n_pos, int32_t hc, int32_t n_embd,
+                              const float* value, const float* gate, const float* rstd,
+                              const float* norm_conv, const float* conv_w, const float* pre,
+                              const float* d_out, const float* d_tail, int64_t tail_rows, float* d_full,
+                              void* workspace, size_t workspace_bytes, void* stream);
+int eg_ple_weight_sums(const float* key, const float* hidden, const float* rstd, const float* d_s,
+                       const float* norm_key, const float* norm_query, int64_t hist_rows, int64_t n_pos,
+                       int32_t hc, int32_t n_embd, float* d_norm_key, float* d_norm_query,
+                       float* d_norm_conv, float* d_conv_w, void* workspace, size_t workspace_bytes,
+                       void* stream);
+
 /* Per-stream RMS norm: out[r, j, :] = x[r, j, :] / sqrt(mean(x[r, j, :]^2) + eps)
  * * weight[j, :], x and out f32 [n_rows, hc, n_embd], weight f32 [hc, n_embd]
  * (PleReplica._rmsnorm_per_stream, engraft/lens.py:282-287; the reductions of

@@ -44,3 +44,70 @@ def test_conv_gated_is_the_convolution_of_the_normed_rows(cuda, t, h0, hc, n):
         res.append((out, pre, new, s, gate, rstd))
     for a, b in zip(*res):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("t,h0,hc,n", [(1, 0, 1, 256), (9, 2, 2, 256), (54, 9, 4, 512), (63, 0, 3, 256),
+                                       (64, 12, 2, 512), (135, 9, 4, 256)])
+@pytest.mark.parametrize("tail", [False, True])
+def test_conv_backward_sums_against_the_separate_kernels(cuda, t, h0, hc, n, tail):
+    """eg_ple_conv_backward_sums + eg_ple_weight_sums against eg_ple_conv_backward
+    without the forward's pre-activation (its general kernel) and
+    eg_ple_weight_grads, at the edges of the 63-row chunks and nine-row turns:
+    d_full bit for bit, the sums over t positions within t 2^-23 of the sum of
+    the terms' magnitudes (two fp32 sums of the same terms)."""
+    from engraft_ngram_amd import _lib
+    print(f"[gpu-test] conv_backward_sums t={t} h0={h0} hc={hc} n={n} tail={tail}", file=sys.stderr, flush=True)
+    g = torch.Generator(device=cuda).manual_seed(t + h0 + n)
+    rnd = lambda *s: torch.randn(s, generator=g, device=cuda)
+    C = hc * n
+    key, hidden, d_out, value, hist, conv = rnd(t, C), rnd(t, C), rnd(t, C), rnd(t, n), rnd(h0, C), rnd(C, 4)
+    nk, nq, nc = (1 + 0.1 * rnd(C) for _ in range(3))
+    tail_rows = min(9, h0 + t) if tail else 0
+    d_tail = rnd(tail_rows, C) if tail else None
+    d_s = rnd(t, hc)
+    full, out, pre = torch.cat([hist, torch.empty((t, C), device=cuda)]), rnd(t, C), rnd(t, C)
+    s, gate, rstd = rnd(t, hc), rnd(t, hc), rnd(t, hc, 3)
+    st, p = _lib.stream_ptr(cuda), _lib.ptr
+    _lib.call("eg_ple_gate", p(key), p(value), p(hidden), p(nk), p(nq), p(nc), t, hc, n, 1e-6, p(full[h0:]), p(s),
+              p(gate), p(rstd), st)
+    _lib.call("eg_ple_conv", p(full), h0, t, hc, n, p(conv), 4, 3, 0, p(hidden), p(value), p(gate), p(out), p(pre), st)
+    want, got = (torch.full((h0 + t, C), 7.0, device=cuda) for _ in range(2))
+    _lib.call("eg_ple_conv_backward", p(full), h0, t, hc, n, p(conv), 4, 3, None, p(d_out), p(d_tail), tail_rows,
+              p(want), st)
+    size = int(_lib.load().eg_ple_weight_sums_workspace_size(h0, t, hc, n))
+    ws = torch.full((size // 4,), float("nan"), device=cuda)
+    _lib.call("eg_ple_conv_backward_sums", p(hist), h0, t, hc, n, p(value), p(gate), p(rstd), p(nc), p(conv), p(pre),
+              p(d_out), p(d_tail), tail_rows, p(got), p(ws), size, st)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    # the run kernel without the sums, from the pre-activation
+    again = torch.full((h0 + t, C), 7.0, device=cuda)
+    _lib.call("eg_ple_conv_backward", None, h0, t, hc, n, p(conv), 4, 3, p(pre), p(d_out), p(d_tail), tail_rows,
+              p(again), st)
+    assert torch.equal(again, want)
+
+    def outs():
+        return [torch.empty(C, device=cuda) for _ in range(3)] + [torch.empty((C, 4), device=cuda)]
+    a, b = outs(), outs()
+    _lib.call("eg_ple_weight_sums", p(key), p(hidden), p(rstd), p(d_s), p(nk), p(nq), h0, t, hc, n, *map(p, a), p(ws),
+              size, st)
+    size = int(_lib.load().eg_ple_weight_grads_workspace_size(t, hc, n, 4))
+    ws = torch.empty(size // 4, device=cuda)
+
+    def grads(key, hidden, d_s, d_out, d_normed, full, into):
+        _lib.call("eg_ple_weight_grads", p(key), p(value), p(hidden), p(gate), p(rstd), p(d_s), p(nk), p(nq), p(d_out),
+                  p(d_normed), p(full), h0, p(pre), t, hc, n, 4, 3, *map(p, into), p(ws), size, st)
+    grads(key, hidden, d_s, d_out, want[h0:].contiguous(), full, b)
+    torch.cuda.synchronize()
+    x = pre.double()
+    da = (d_out.double() * torch.sigmoid(x) * (1 + x * (1 - torch.sigmoid(x)))).abs()
+    kr, hr = (y.double().view(t, hc, n) * rstd[..., i:i + 1].double() for i, y in ((0, key), (1, hidden)))
+    ds = d_s.double().unsqueeze(-1) / n ** 0.5
+    z = (value.double().unsqueeze(1) * gate.double().unsqueeze(-1) * rstd[..., 2:].double()).reshape(t, C)
+    mags = [(ds * hr * nq.double().view(hc, n) * kr).abs().sum(0).reshape(-1),
+            (ds * kr * nk.double().view(hc, n) * hr).abs().sum(0).reshape(-1),
+            (want[h0:].double() * z).abs().sum(0)]
+    pad = torch.cat([torch.zeros((9, C), device=cuda), full]).double().abs()[h0:]
+    mags.append(torch.stack([(da * pad[3 * k:3 * k + t]).sum(0) for k in range(4)], dim=1))
+    for u, v, m in zip(a, b, mags):
+        assert bool(((u.double() - v.double()).abs() <= (t + 8) * 2.0 ** -23 * m + 1e-30).all())
