@@ -341,8 +341,11 @@ __global__ __launch_bounds__(256) void forward_kernel(const FwdArgs a) {
   //    go out before the overlay lookup: the lookup's dependent probes then
   //    overlap the row's own latency, and a row the overlay replaces (rare)
   //    costs one wasted load.
+  //    LATE (more chunks than registers for every replacement): a replacement
+  //    is loaded where it is decoded, by the wavefronts that have one.
+  constexpr bool LATE = OVL && NCH > 2;
   RawChunk tr[MAXL][NCH];
-  RawChunk orow[OVL ? MAXL : 1][OVL ? NCH : 1];
+  RawChunk orow[OVL && !LATE ? MAXL : 1][OVL && !LATE ? NCH : 1];
   int32_t ovk_keep[OVL ? MAXL : 1];
   uint32_t src[MAXL][NCH];  // 0: base table, 1: overlay, 2: invalid id
 #pragma unroll
@@ -377,7 +380,7 @@ __global__ __launch_bounds__(256) void forward_kernel(const FwdArgs a) {
         if (e0 < W && k >= 0) {
           src[l][c] = 2;
           if (k < ov.rows.n_rows) {
-            orow[l][c] = load_raw_rt(ov.rows, k, e0 - h * dim);
+            if constexpr (!LATE) orow[l][c] = load_raw_rt(ov.rows, k, e0 - h * dim);
             src[l][c] = 1;
           }
         }
@@ -417,8 +420,17 @@ __global__ __launch_bounds__(256) void forward_kernel(const FwdArgs a) {
       const int e0 = cb + (lane + 64 * c) * 8;
       const int off = e0 - (min(e0, W - 8) / dim) * dim;
       float v[8];
-      if (OVL && src[l][c] == 1) {
-        decode_rt(a.ov[l].rows.fmt, orow[OVL ? l : 0][OVL ? c : 0], off, v);
+      if constexpr (LATE) {
+        decode<FMT>(tr[l][c], src[l][c] == 0 ? off : 0, v);
+        const int32_t k = __shfl(ovk_keep[l], min(e0, W - 8) / dim - h_lo);  // by every lane
+        if (src[l][c] == 1) {
+          decode_rt(a.ov[l].rows.fmt, load_raw_rt(a.ov[l].rows, k, off), off, v);
+        } else if (src[l][c] != 0) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) v[i] = __uint_as_float(0x7fc00000u);
+        }
+      } else if (OVL && src[l][c] == 1) {
+        decode_rt(a.ov[l].rows.fmt, orow[OVL && !LATE ? l : 0][OVL && !LATE ? c : 0], off, v);
       } else {
         decode<FMT>(tr[l][c], src[l][c] == 0 ? off : 0, v);
         if (src[l][c] != 0) {
@@ -516,12 +528,19 @@ static bool launch_special_f32(const FwdArgs& a, hipStream_t st) {
 }
 
 // The reference's real table shape (16 heads of 160 values, W = 2560, one
-// layer, no overlay): five 512-column chunks per position.
+// layer): five 512-column chunks per position.  Under an overlay the rare
+// replacements are loaded where they are decoded (LATE): 8,193 positions under
+// 14,032 fp32 rows, half of them read, 30 us against 41 us on the generic
+// kernel (three parts a position, each searching its heads; runtime dim), and
+// 20 us without an overlay.  Measured there and dropped: every replacement's
+// chunk in registers (186 of them, two wavefronts a SIMD); the ids searched by
+// the wavefront together, 64 pivots a round and key: 40 us.
 constexpr int kRealNch = 5;
 template <int FMT, bool ROWS>
 static bool launch_real(const FwdArgs& a, bool ovl, hipStream_t st) {
-  if (a.dim != 160 || a.heads * a.dim != 2560 || a.n_layers != 1 || ovl) return false;
-  launch_nch<FMT, 160, kRealNch, 1, false, false, 5 / kRealNch, ROWS>(a, st);
+  if (a.dim != 160 || a.heads * a.dim != 2560 || a.n_layers != 1) return false;
+  if (ovl) launch_nch<FMT, 160, kRealNch, 1, false, true, 5 / kRealNch, ROWS>(a, st);
+  else launch_nch<FMT, 160, kRealNch, 1, false, false, 5 / kRealNch, ROWS>(a, st);
   return true;
 }
 
