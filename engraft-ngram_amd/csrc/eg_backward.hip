@@ -781,10 +781,10 @@ __device__ void adam_apply(const SegArgs& a, int64_t k, int sub, const float g[V
 // The sum g of variable k is final: optimizer step, or accumulation into grad_out.
 template <int VPL, bool CONSEC, bool ADAM>
 __device__ inline void finish(const SegArgs& a, int64_t k, int sub, const float g[VPL], float p[VPL], float m[VPL],
-                              float v[VPL]) {
+                              float v[VPL], bool hit = true) {
   if constexpr (ADAM) {
     adam_apply<VPL, CONSEC>(a, k, sub, g, p, m, v);
-    if (a.dense && sub == 0) a.stamp[k] = (int32_t)a.step;
+    if (a.dense && hit && sub == 0) a.stamp[k] = (int32_t)a.step;
   } else {
     float* dst = a.grad_out + k * a.dim;
     if (a.overwrite) {
@@ -848,12 +848,15 @@ __global__ __launch_bounds__(256) void reduce_kernel(const SegArgs a, int64_t n_
     const int64_t hi = a.end[key];
     const int64_t len = hi - lo;
     float p[VPL], m[VPL], v[VPL];
-    if (ADAM && grp == 0) {  // independent of the gradient: fetched first
+    auto load_state = [&] {
       const int64_t off = (int64_t)key * a.stride;
       load_f32<VPL, CONSEC>(a.master + off, sub, p);
       load_f32<VPL, CONSEC>(a.m + off, sub, m);
       load_f32<VPL, CONSEC>(a.v + off, sub, v);
-    }
+    };
+    // independent of the gradient: fetched first (beside f32 gradients after
+    // them, so that eight slots' loads keep the registers of the short ranges)
+    if (ADAM && !F32 && grp == 0) load_state();
     const bool in_lds = len <= kLongLds;
     uint32_t* gseg = (uint32_t*)a.slots + lo;
     if (in_lds) {
@@ -872,12 +875,11 @@ __global__ __launch_bounds__(256) void reduce_kernel(const SegArgs a, int64_t n_
       float P[VPL];
 #pragma unroll
       for (int t = 0; t < VPL; ++t) P[t] = 0.0f;
-      // eight slots' loads in flight at a time (four with both the optimizer's
-      // state and f32 gradients held: eight would cost occupancy there)
-      sum_piece<VPL, CONSEC, (ADAM && F32) ? 4 : 8, F32>(a, vl, gbase, cnt, sub, P);
+      sum_piece<VPL, CONSEC, 8, F32>(a, vl, gbase, cnt, sub, P);  // eight slots' loads in flight at a time
 #pragma unroll
       for (int t = 0; t < VPL; ++t) G[t] = G[t] + P[t];
     }
+    if (ADAM && F32 && grp == 0) load_state();
     __syncthreads();  // every slot id has been read: the buffer takes the group sums
 #pragma unroll
     for (int t = 0; t < VPL; ++t) part[grp * 512 + col_of<VPL, CONSEC>(sub, t)] = G[t];
@@ -905,7 +907,8 @@ __global__ __launch_bounds__(256) void reduce_kernel(const SegArgs a, int64_t n_
     store_f32<VPL, CONSEC>(a.grad_out + k * a.dim, sub, z);
     return;
   }
-  if (len == 0 || len > kPiece) return;  // not hit, or a long range (its own workgroup)
+  // not hit (a dense step takes a zero gradient), or a long range (its own workgroup)
+  if ((len == 0 && !(ADAM && a.dense)) || len > kPiece) return;
   float p[VPL], m[VPL], v[VPL];
   if constexpr (ADAM) {  // the state rows do not depend on the gradient: fetch them first
     const int64_t off = k * a.stride;
@@ -914,7 +917,7 @@ __global__ __launch_bounds__(256) void reduce_kernel(const SegArgs a, int64_t n_
     load_f32<VPL, CONSEC>(a.v + off, sub, v);
   }
   const int cnt = (int)len;
-  const uint32_t sl = a.slots[lo + min(sub, cnt - 1)];  // every lane loads (no divergent load)
+  const uint32_t sl = a.slots[cnt > 0 ? lo + min(sub, cnt - 1) : 0];  // every lane loads (no divergent load)
   // the network only as wide as the longest of the wavefront's two ranges needs
   // (most ranges hold one or two slots); lanes past a range hold 0xffffffff
   // (the other group's count is read from its lanes; a group that has already
@@ -931,17 +934,20 @@ __global__ __launch_bounds__(256) void reduce_kernel(const SegArgs a, int64_t n_
   const int cw = __builtin_amdgcn_readfirstlane(cmax);
   if (cw == 1) sum_piece<VPL, CONSEC, 1, F32>(a, vl, gbase, cnt, sub, g);
   else if (cw == 2) sum_piece<VPL, CONSEC, 2, F32>(a, vl, gbase, cnt, sub, g);
-  else sum_piece<VPL, CONSEC, 4, F32>(a, vl, gbase, cnt, sub, g);
-  finish<VPL, CONSEC, ADAM>(a, k, sub, g, p, m, v);
+  else if (ADAM || cw <= 4) sum_piece<VPL, CONSEC, 4, F32>(a, vl, gbase, cnt, sub, g);
+  else sum_piece<VPL, CONSEC, 8, F32>(a, vl, gbase, cnt, sub, g);
+  finish<VPL, CONSEC, ADAM>(a, k, sub, g, p, m, v, cnt > 0);
 }
 
-// Dense mode: the variables no slot hit this step take a zero-gradient step.
+// Dense mode of a step without slots: every variable takes a zero-gradient
+// step (reduce_kernel steps the variables no slot hit along with the others;
+// as a second launch over all of them they cost a fact's step of 14,032
+// variables 5 us of 35).
 template <int VPL, bool CONSEC>
 __global__ __launch_bounds__(256) void dense_kernel(const SegArgs a) {
   const int sub = threadIdx.x & 31;
   const int64_t k = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 5;
   if (k >= a.n_var) return;
-  if (a.stamp[k] == (int32_t)a.step) return;
   float g[VPL], p[VPL], m[VPL], v[VPL];
 #pragma unroll
   for (int t = 0; t < VPL; ++t) g[t] = 0.0f;
@@ -1439,12 +1445,8 @@ int eg_descent_apply(const void* d_out, int32_t d_out_f32, int64_t n_pos, int32_
   a.eps = (float)opt->eps;
   a.neg_step_size = -(float)(opt->lr / bc1);
   a.l2c = opt->l2_coef;
-  if (n > 0) {
-    rc = launch_reduce<true>(a, st);
-    if (rc != EG_OK) return rc;
-  }
-  if (opt->dense) rc = launch_dense(a, st);
-  return rc;
+  if (n > 0) return launch_reduce<true>(a, st);
+  return opt->dense ? launch_dense(a, st) : EG_OK;
 }
 
 int eg_descent_step(const void* d_out, int32_t d_out_f32, const int32_t* rows, int64_t n_pos, int32_t heads,
