@@ -160,6 +160,7 @@ SIGNATURES = {
     "eg_ple_gate_backward": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                        c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int32, c_int32,
                                        c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "eg_ple_gate_backward_kv": (c_int32, [c_void_p] * 11 + [c_int64, c_int32, c_int32] + [c_void_p] * 4),
     "eg_ple_gate_backward_planes": (c_int32, [c_void_p] * 11 + [c_int64, c_int32, c_int32, c_int32, c_int32] +
                                     [c_void_p] * 7),
     "eg_ple_weight_grads_workspace_size": (ctypes.c_size_t, [c_int64, c_int32, c_int32, c_int32]),

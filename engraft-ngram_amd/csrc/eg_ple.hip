@@ -1024,7 +1024,8 @@ __device__ inline void store_planes4(const float* x, __bf16* hi, __bf16* lo, int
 }
 
 // PLANES: d_key and d_value are written as their bf16 hi / lo planes (the
-// operands of eg_gemm_bf16x3), d_key_lo / d_value_lo the lo planes.
+// operands of eg_gemm_bf16x3), d_key_lo / d_value_lo the lo planes.  d_key_ld and
+// d_value_ld: elements from one position's row to the next.
 template <bool PLANES>
 __global__ __launch_bounds__(kGbThreads) void ple_gate_bwd_vec_kernel(
     const float* __restrict__ key, const float* __restrict__ value, const float* __restrict__ hidden,
@@ -1033,7 +1034,7 @@ __global__ __launch_bounds__(kGbThreads) void ple_gate_bwd_vec_kernel(
     const float* __restrict__ d_out, const float* __restrict__ d_normed, int hc, int n, float inv_sqrt_n,
     int detach_value, int detach_gate, float* __restrict__ d_key, float* __restrict__ d_value,
     float* __restrict__ d_hidden, __bf16* __restrict__ d_key_lo, __bf16* __restrict__ d_value_lo,
-    float* __restrict__ d_s) {
+    float* __restrict__ d_s, int64_t d_key_ld, int64_t d_value_ld) {
 #pragma clang fp contract(off)
   __shared__ float red[kGbMaxHc * (kGbThreads / 64)];
   const int64_t t = blockIdx.x;
@@ -1086,8 +1087,9 @@ __global__ __launch_bounds__(kGbThreads) void ple_gate_bwd_vec_kernel(
       for (int j = 0; j < kGbMaxHc; ++j)
         if (j < hc) dv[e] += dg[j][e] * gj[j];
     }
-    if constexpr (PLANES) store_planes4(dv, (__bf16*)d_value, d_value_lo, t * n + i0);
-    else *(float4*)(d_value + t * n + i0) = make_float4(dv[0], dv[1], dv[2], dv[3]);
+    const int64_t o = t * d_value_ld + i0;
+    if constexpr (PLANES) store_planes4(dv, (__bf16*)d_value, d_value_lo, o);
+    else *(float4*)(d_value + o) = make_float4(dv[0], dv[1], dv[2], dv[3]);
   }
   // second reduction: d_gate per stream -> d_s
   float ds[kGbMaxHc];
@@ -1137,8 +1139,9 @@ __global__ __launch_bounds__(kGbThreads) void ple_gate_bwd_vec_kernel(
       dh[e] = dd[e] + ((rq[j] * wq[e]) * (dsn * kn) - h[e] * cq);
     }
     if (d_key != nullptr) {
-      if constexpr (PLANES) store_planes4(dk, (__bf16*)d_key, d_key_lo, row + i0);
-      else *(float4*)(d_key + row + i0) = make_float4(dk[0], dk[1], dk[2], dk[3]);
+      const int64_t o = t * d_key_ld + (int64_t)j * n + i0;
+      if constexpr (PLANES) store_planes4(dk, (__bf16*)d_key, d_key_lo, o);
+      else *(float4*)(d_key + o) = make_float4(dk[0], dk[1], dk[2], dk[3]);
     }
     if (d_hidden != nullptr) *(float4*)(d_hidden + row + i0) = make_float4(dh[0], dh[1], dh[2], dh[3]);
   }
@@ -1410,13 +1413,38 @@ int eg_ple_gate_backward(const float* key, const float* value, const float* hidd
     hipLaunchKernelGGL(ple_gate_bwd_vec_kernel<false>, dim3((unsigned)n_pos), dim3(n_embd / 4), 0, (hipStream_t)stream,
                        key, value, hidden, norm_key, norm_query, norm_conv, s, gate, rstd, d_out, d_normed, hc, n_embd,
                        (float)(1.0 / sqrt((double)n_embd)), detach_value, detach_gate, detach_gate ? nullptr : d_key,
-                       detach_value ? nullptr : d_value, d_hidden, nullptr, nullptr, d_s);
+                       detach_value ? nullptr : d_value, d_hidden, nullptr, nullptr, d_s, (int64_t)hc * n_embd,
+                       (int64_t)n_embd);
   else
     hipLaunchKernelGGL(ple_gate_bwd_kernel, dim3((unsigned)n_pos), dim3(kGbThreads), 0, (hipStream_t)stream, key,
                        value, hidden, norm_key, norm_query, norm_conv, s, gate, rstd, d_out, d_normed, hc, n_embd,
                        (float)(1.0 / sqrt((double)n_embd)), detach_value, detach_gate, detach_gate ? nullptr : d_key,
                        detach_value ? nullptr : d_value, d_hidden, d_s);
   return launch_status("ple_gate_bwd_kernel");
+}
+
+int eg_ple_gate_backward_kv(const float* key, const float* value, const float* hidden, const float* norm_key,
+                            const float* norm_query, const float* norm_conv, const float* s, const float* gate,
+                            const float* rstd, const float* d_out, const float* d_normed, int64_t n_pos, int32_t hc,
+                            int32_t n_embd, float* d_kv, float* d_hidden, float* d_s, void* stream) {
+  EG_CHECK_ARG(n_pos >= 0 && n_pos < (1LL << 31), "n_pos=%lld", (long long)n_pos);
+  if (hc < 1 || hc > kGbMaxHc || n_embd < 256 || n_embd > kGbThreads * 4 || n_embd % 256 != 0)
+    return set_error(EG_ERR_UNSUPPORTED, "gate backward side by side for hc=%d n_embd=%d (built: hc <= %d, n_embd a "
+                     "multiple of 256 up to %d)", hc, n_embd, kGbMaxHc, kGbThreads * 4);
+  EG_CHECK_ARG(n_pos == 0 || (key && value && hidden && norm_key && norm_query && norm_conv && s && gate && rstd &&
+                              d_out && d_normed && d_kv),
+               "NULL argument");
+  EG_CHECK_ARG(((uintptr_t)key | (uintptr_t)value | (uintptr_t)hidden | (uintptr_t)norm_key | (uintptr_t)norm_query |
+                (uintptr_t)norm_conv | (uintptr_t)d_out | (uintptr_t)d_normed | (uintptr_t)d_kv |
+                (uintptr_t)d_hidden) % 16 == 0,
+               "pointers must be 16-byte aligned");
+  if (n_pos == 0) return EG_OK;
+  const int64_t ld = (int64_t)(hc + 1) * n_embd;
+  hipLaunchKernelGGL(ple_gate_bwd_vec_kernel<false>, dim3((unsigned)n_pos), dim3(n_embd / 4), 0, (hipStream_t)stream,
+                     key, value, hidden, norm_key, norm_query, norm_conv, s, gate, rstd, d_out, d_normed, hc, n_embd,
+                     (float)(1.0 / sqrt((double)n_embd)), 0, 0, d_kv, d_kv + (int64_t)hc * n_embd, d_hidden, nullptr,
+                     nullptr, d_s, ld, ld);
+  return launch_status("ple_gate_bwd_vec_kernel");
 }
 
 int eg_ple_gate_backward_planes(const float* key, const float* value, const float* hidden, const float* norm_key,
@@ -1444,7 +1472,7 @@ int eg_ple_gate_backward_planes(const float* key, const float* value, const floa
                      key, value, hidden, norm_key, norm_query, norm_conv, s, gate, rstd, d_out, d_normed, hc, n_embd,
                      (float)(1.0 / sqrt((double)n_embd)), detach_value, detach_gate,
                      detach_gate ? nullptr : (float*)d_key_hi, detach_value ? nullptr : (float*)d_value_hi, d_hidden,
-                     (__bf16*)d_key_lo, (__bf16*)d_value_lo, d_s);
+                     (__bf16*)d_key_lo, (__bf16*)d_value_lo, d_s, (int64_t)hc * n_embd, (int64_t)n_embd);
   return launch_status("ple_gate_bwd_vec_kernel");
 }
 

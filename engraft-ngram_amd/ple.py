@@ -730,13 +730,26 @@ class _PleFn(torch.autograd.Function):
         need = ctx.needs_input_grad
         need_emb, need_hist = need[0], need[8]
         need_wk, need_wv, need_nk, need_nq, need_nc, need_cv = need[2:8]
-        d_key = torch.empty((t_len, c_dim), **f32) if ((need_emb or need_wk) and not detach_gate) else None
-        d_value = torch.empty((t_len, n), **f32) if ((need_emb or need_wv) and not detach_value) else None
+        # both projection weights' gradients: d_key and d_value side by side, so that they
+        # are one product with emb (whole rounds of tiles, emb split once)
+        both = (need_wk and need_wv and not detach_gate and not detach_value and ctx.gemm == "bf16x6"
+                and n % 256 == 0 and t_len > 0 and not (key.data_ptr() | value.data_ptr() | hidden32.data_ptr()
+                                                        | nk32.data_ptr() | nq32.data_ptr() | nc32.data_ptr()
+                                                        | d_out32.data_ptr() | d_full[h0:].data_ptr()) % 16)
         d_s = torch.empty((t_len, hc), **f32)
-        _lib.call("eg_ple_gate_backward", _lib.ptr(key), _lib.ptr(value), _lib.ptr(hidden32), _lib.ptr(nk32),
-                  _lib.ptr(nq32), _lib.ptr(nc32), _lib.ptr(s), _lib.ptr(gate), _lib.ptr(rstd), _lib.ptr(d_out32),
-                  _lib.ptr(d_full[h0:]), t_len, hc, n, int(bool(detach_value)), int(bool(detach_gate)),
-                  _lib.ptr(d_key), _lib.ptr(d_value), _lib.ptr(d_hidden), _lib.ptr(d_s), st)
+        if both:
+            d_kv = torch.empty((t_len, c_dim + n), **f32)
+            d_key, d_value = d_kv[:, :c_dim], d_kv[:, c_dim:]
+            _lib.call("eg_ple_gate_backward_kv", _lib.ptr(key), _lib.ptr(value), _lib.ptr(hidden32), _lib.ptr(nk32),
+                      _lib.ptr(nq32), _lib.ptr(nc32), _lib.ptr(s), _lib.ptr(gate), _lib.ptr(rstd), _lib.ptr(d_out32),
+                      _lib.ptr(d_full[h0:]), t_len, hc, n, _lib.ptr(d_kv), _lib.ptr(d_hidden), _lib.ptr(d_s), st)
+        else:
+            d_key = torch.empty((t_len, c_dim), **f32) if ((need_emb or need_wk) and not detach_gate) else None
+            d_value = torch.empty((t_len, n), **f32) if ((need_emb or need_wv) and not detach_value) else None
+            _lib.call("eg_ple_gate_backward", _lib.ptr(key), _lib.ptr(value), _lib.ptr(hidden32), _lib.ptr(nk32),
+                      _lib.ptr(nq32), _lib.ptr(nc32), _lib.ptr(s), _lib.ptr(gate), _lib.ptr(rstd), _lib.ptr(d_out32),
+                      _lib.ptr(d_full[h0:]), t_len, hc, n, int(bool(detach_value)), int(bool(detach_gate)),
+                      _lib.ptr(d_key), _lib.ptr(d_value), _lib.ptr(d_hidden), _lib.ptr(d_s), st)
         d_emb = None
         if need_emb:
             parts = [(d, w) for d, w in ((d_key, wk32), (d_value, wv32)) if d is not None]
@@ -745,8 +758,12 @@ class _PleFn(torch.autograd.Function):
         wdt = ctx.w_dtypes
         # the projection weights' gradients d_key^T emb and d_value^T emb on eg_gemm_f32
         # (K = the positions); a weight the detached factor cuts off keeps None
-        d_wk = _weight_grad(d_key, emb32, wk32, ctx.gemm).to(wdt[0]) if (need_wk and d_key is not None) else None
-        d_wv = _weight_grad(d_value, emb32, wv32, ctx.gemm).to(wdt[1]) if (need_wv and d_value is not None) else None
+        if both:
+            d_w = _weight_grad(d_kv, emb32, None, ctx.gemm)
+            d_wk, d_wv = d_w[:c_dim].to(wdt[0]), d_w[c_dim:].to(wdt[1])
+        else:
+            d_wk = _weight_grad(d_key, emb32, wk32, ctx.gemm).to(wdt[0]) if (need_wk and d_key is not None) else None
+            d_wv = _weight_grad(d_value, emb32, wv32, ctx.gemm).to(wdt[1]) if (need_wv and d_value is not None) else None
         if detach_gate:  # the gate's whole branch (key, its norm, the query norm) is detached
             need_nk = need_nq = False
         d_nk = d_nq = d_nc = d_cv = None

@@ -477,6 +477,15 @@ int eg_ple_gate_backward(const float* key, const float* value, const float* hidd
                          int32_t hc, int32_t n_embd, int32_t detach_value, int32_t detach_gate,
                          float* d_key, float* d_value, float* d_hidden, float* d_s, void* stream);
 
+/* eg_ple_gate_backward (no factor detached) with d_key and d_value side by side,
+ * d_kv f32 [n_pos, (hc + 1) * n_embd]: one operand of the projection weights'
+ * gradients.  n_embd a multiple of 256, pointers 16-byte aligned. */
+int eg_ple_gate_backward_kv(const float* key, const float* value, const float* hidden, const float* norm_key,
+                            const float* norm_query, const float* norm_conv, const float* s, const float* gate,
+                            const float* rstd, const float* d_out, const float* d_normed, int64_t n_pos,
+                            int32_t hc, int32_t n_embd, float* d_kv, float* d_hidden, float* d_s,
+                            void* stream);
+
 /* eg_ple_gate_backward with d_key and d_value written as their bf16 hi / lo
  * planes (hi = rne(x), lo = rne(x - hi); row strides hc*n_embd and n_embd,
  * the layout of eg_split_bf16's output), ready as eg_gemm_bf16x3 operands:
