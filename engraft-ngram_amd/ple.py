@@ -601,8 +601,11 @@ class _PleFn(torch.autograd.Function):
         if native:
             # emb for the projection weights' gradients
             emb_w = emb32 if any(ctx.needs_input_grad[2:4]) else None
-            # the rows the taps' gradients meet: all of them, or the history alone
-            rows = hist32 if gated else full
+            # the rows the taps' gradients meet: all of them, or the history alone (a copy: the
+            # caller may write the next history over this one before the backward)
+            rows = full
+            if gated:
+                rows = hist32.clone() if any(ctx.needs_input_grad[4:8]) else None
             ctx.save_for_backward(key, value, hidden32, rows, s, gate, rstd, nk32, nq32, nc32, conv32, wk32, wv32, pre,
                                   emb_w)
             ctx.gated = gated

@@ -111,3 +111,30 @@ def test_conv_backward_sums_against_the_separate_kernels(cuda, t, h0, hc, n, tai
     mags.append(torch.stack([(da * pad[3 * k:3 * k + t]).sum(0) for k in range(4)], dim=1))
     for u, v, m in zip(a, b, mags):
         assert bool(((u.double() - v.double()).abs() <= (t + 8) * 2.0 ** -23 * m + 1e-30).all())
+
+
+@pytest.mark.parametrize("weights", [False, True])
+def test_history_written_over_before_the_backward(cuda, weights):
+    """A loop that keeps its history in one buffer overwrites it after the
+    forward; the backward's gradients are those of the history the forward read."""
+    from engraft_ngram_amd import ple
+
+    class HP:
+        hc_mult, n_embd, f_norm_rms_eps, ple_ngram_size = 2, 256, 1e-6, 3
+    g = torch.Generator(device=cuda).manual_seed(4)
+    rnd = lambda *s: torch.randn(s, generator=g, device=cuda)
+    hc, n, t = 2, 256, 70
+    w = ple.PleWeights(rnd(hc * n, n) / 16, rnd(n, n) / 16, *(1 + 0.1 * rnd(hc * n) for _ in range(3)), rnd(hc * n, 4))
+    emb, hidden, hist, r = rnd(t, n), rnd(t, hc, n) + 0.5, rnd(9, hc, n), rnd(t, hc, n)
+    res = []
+    for overwrite in (False, True):
+        leaves = [emb.clone().requires_grad_(True)]
+        ws = {k: v.clone().requires_grad_(weights) for k, v in vars(w).items()}
+        leaves += [v for v in ws.values() if weights]
+        buf = hist.clone()
+        out, new = ple.ple_forward(leaves[0], hidden, ple.PleWeights(**ws), buf, HP)
+        if overwrite:
+            buf.copy_(new.detach())
+        res.append(torch.autograd.grad(out, leaves, r))
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
