@@ -925,8 +925,10 @@ def bench_ple(steps: int, warmup: int, cpu_s: float = 0.0) -> dict:
                 pk, pv = ple.SplitPlanes(w.w_key), ple.SplitPlanes(w.w_value)
                 gemm_ms = timed(lambda: ple.gemm_x3(emb, pk, b_n2=pv), steps)
             else:
-                pk, pv = ple.SplitPlanes(w.w_key, three=True), ple.SplitPlanes(w.w_value, three=True)
-                gemm_ms = timed(lambda: ple.gemm_x6(emb, pk, b_n2=pv), steps)
+                # what this mode's forward runs at this length: fp16 planes, three products
+                pk, pv = ple.HalfPlanes((w.w_key,)), ple.HalfPlanes((w.w_value,))
+                gemm_ms = timed(lambda: ple.gemm_h3((emb,), (w.w_key,), (w.w_value,), planes_b=pk, planes_b2=pv),
+                                steps)
         # forward + backward to emb (the descent's use: the weights stay fixed)
         fb = lambda: torch.autograd.grad(ple.ple_forward(emb_v, hidden, w, hist, HP, gemm=mode)[0], emb_v, d_out)
         fb()
@@ -952,7 +954,7 @@ def bench_ple(steps: int, warmup: int, cpu_s: float = 0.0) -> dict:
         errs = {"fp32": err(ple.gemm_f32(emb, w.w_key, b_n2=w.w_value)),
                 "hipblaslt": err((emb @ w.w_key.T, emb @ w.w_value.T)),
                 "bf16x3": err(ple.gemm_x3(emb, w.w_key, b_n2=w.w_value)),
-                "bf16x6": err(ple.gemm_x6(emb, w.w_key, b_n2=w.w_value))}
+                "bf16x6": err(ple.gemm_h3((emb,), (w.w_key,), (w.w_value,)))}
         torch.backends.cuda.matmul.allow_tf32 = allow
         del refs, e64
     res["fp32"]["gemm_err_vs_fp64"] = errs["fp32"]
@@ -962,8 +964,9 @@ def bench_ple(steps: int, warmup: int, cpu_s: float = 0.0) -> dict:
     out = {"workload": "ple_forward: T 2048, hc 4, n_embd 2560, 4 taps, dilation 3, fp32 activations; key/value "
                        "GEMMs (one launch) either fp32 (eg_gemm_f32 on the fp32 matrix cores; the reference's "
                        "arithmetic; hipBLASLt's time for the same products beside it), bf16x3 (eg_gemm_bf16x3 "
-                       "on the bf16 matrix cores, 16 mantissa bits per operand) or bf16x6 (eg_gemm_bf16x6: three "
-                       "bf16 planes an operand, six products, fp32 accuracy; ple_forward's default); gate/norm "
+                       "on the bf16 matrix cores, 16 mantissa bits per operand) or bf16x6 (fp32 accuracy on the "
+                       "16-bit matrix cores, ple_forward's default: at this length eg_gemm_f16x3, two fp16 planes "
+                       "an operand, three products; the differentiated forward eg_gemm_bf16x6); gate/norm "
                        "and conv in HIP; gemm_err_vs_fp64: the largest |C - C64| / (|emb| |W|^T); the top-level "
                        "figures are the fp32 mode's",
            **res["fp32"], "default_gemm": "bf16x6", "bf16x3": res["bf16x3"], "bf16x6": res["bf16x6"],
