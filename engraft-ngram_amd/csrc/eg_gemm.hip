@@ -895,7 +895,7 @@ __global__ __launch_bounds__(256) void gemm_f32_vec_kernel(const F32Args args) {
 // fp16 matrix cores; 378 us for the PLE key + value of 2,048 positions, its
 // operand's split and the marked rows' check included, against 691 us for the
 // six bf16 products (bound by the matrix cores and their operands' path
-// through LDS, as gemm_x3_kernel).  Every row of an operand is scaled by a power of two that
+// through LDS, as gemm_x3_kernel).  Every row of an operand's source is scaled by a power of two that
 // puts its largest magnitude in [2^14, 2^15) and split into hi = rne16(x) and
 // lo = rne16(x - hi): 22 significand bits where the element is at least
 // 2^-18 of the row's largest, an absolute 2^-40 of it below.  C = hi*hi +
@@ -915,6 +915,14 @@ __global__ __launch_bounds__(256) void gemm_f32_vec_kernel(const F32Args args) {
 // planes gave sixteen half lines), a fragment read is 64 consecutive 16-byte
 // slots (no bank conflicts, no swizzle), and the load addresses are scalar
 // but for the lane's 16 bytes.
+//
+// Two sources have an exponent each: one source's values far below the
+// other's meet products of their own size where B's sources differ the other
+// way, so both keep all their bits (with one exponent a row, sources 2^24 apart
+// left an error of 4e-5).  A tile (or its part of K) that began in source 0 is
+// multiplied by the powers of two that lead to source 1's units when it leaves
+// it, in the accumulators; kApart bounds them.  d_emb of 1,531 positions, K
+// 10,240 + 2,560: 272 us, 15 us of them the second source's own start and the units.
 struct H3Seg {
   const char* a;
   const char* b[2];       // per column group
@@ -927,7 +935,9 @@ struct H3Args {
   H3Seg seg[1];
   int n_seg;
   Plan p;
-  RowScale scale;
+  RowScale scale;         // of the last source: the units sums are kept in
+  RowScale first;         // of source 0, where there are two
+  int64_t kt_first;       // K steps of source 0 where there are two, otherwise all
 };
 
 constexpr int kFragBytes = 1024;  // one operand fragment, 64 lanes x 8 fp16
@@ -935,7 +945,7 @@ constexpr int kStepBytes = 4 * kFragBytes;  // 32 rows x 32 k, both planes
 
 // The steps of x3_tile (its software pipeline and barriers) over
 // fragment-major fp16 planes.
-template <int BM, int BN, int WMW, int WNW>
+template <int BM, int BN, int WMW, int WNW, bool TWO>
 __device__ inline void h3_tile(const H3Args& args, const Work& w, char* lds) {
   constexpr int NW = WMW * WNW, TI = BM / WMW / 32, TJ = BN / WNW / 32;
   constexpr int AB = BM / 32, BB = BN / 32;          // 32-row blocks of a stage
@@ -947,7 +957,6 @@ __device__ inline void h3_tile(const H3Args& args, const Work& w, char* lds) {
   const int uwave = __builtin_amdgcn_readfirstlane(wave);
   const int wm = uwave / WNW, wn = uwave % WNW;
   const H3Seg& sg = args.seg[0];
-  const int64_t lo = w.kv0, hi = w.kv1;
 
   f32x16 acc[TI][TJ];
 #pragma unroll
@@ -957,7 +966,9 @@ __device__ inline void h3_tile(const H3Args& args, const Work& w, char* lds) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-  if (lo < hi) {
+  // K steps [lo, hi), of one source
+  auto steps = [&](int64_t lo, int64_t hi) {
+    if (lo >= hi) return;
     // this wavefront's loads: blocks uwave LB .. + LB - 1 of the stage (A's, then
     // B's), four 1 KB pieces each.  Blocks past the last re-read the last: their
     // products only reach outputs that are not stored.
@@ -1057,14 +1068,54 @@ __device__ inline void h3_tile(const H3Args& args, const Work& w, char* lds) {
 #pragma unroll
     for (int pass = 0; pass < 3; ++pass) mfma(1, pass);
     __builtin_amdgcn_s_barrier();  // the ring is refilled by the next tile
+  };
+  if constexpr (TWO) {
+    const int64_t mid = min(max(w.kv0, args.kt_first), w.kv1);
+    steps(w.kv0, mid);
+    if (w.kv0 < mid) {
+      // into source 1's units, the rows' and columns' powers through the ring
+      // (free between two turns); rows past m or n take the last one's: not stored
+      int* diff = (int*)lds;
+      static_assert(NW * 64 == BM + BN, "a row or a column a thread");
+      const int e = (int)threadIdx.x;
+      if (e < BM) {
+        const int64_t row = min(w.m0 + e, p.m - 1);
+        diff[e] = args.first.a[row] - args.scale.a[row];
+      } else {
+        const int64_t col = min(w.n0 + e - BM, p.n[w.grp] - 1);
+        diff[e] = args.first.b[w.grp][col] - args.scale.b[w.grp][col];
+      }
+      __syncthreads();
+      int lane_o = lane;  // opaque: addresses hoisted out of the walk's loop spill
+      asm volatile("" : "+v"(lane_o));
+      int sb[TJ];
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) sb[j] = diff[BM + (wn * TJ + j) * 32 + (lane_o & 31)];
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          __builtin_amdgcn_sched_barrier(0);
+          const int4 sa = *(const int4*)(diff + (wm * TI + i) * 32 + 8 * q + 4 * (lane_o >> 5));
+          const int sr[4] = {sa.x, sa.y, sa.z, sa.w};
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) acc[i][j][4 * q + r] = ldexpf(acc[i][j][4 * q + r], sr[r] + sb[j]);
+        }
+      __syncthreads();
+    }
+    steps(mid, w.kv1);
+  } else {
+    steps(w.kv0, w.kv1);
   }
   store_acc<BM, BN, TI, TJ>(p, w, acc, wm, wn, lane, args.scale);
 }
 
-template <int BM, int BN, int WMW, int WNW>
+template <int BM, int BN, int WMW, int WNW, bool TWO>
 __global__ __launch_bounds__(WMW * WNW * 64) void gemm_h3_kernel(const H3Args args) {
   extern __shared__ __attribute__((aligned(16))) char ldsh[];
-  EG_GEMM_WALK((h3_tile<BM, BN, WMW, WNW>(args, w, ldsh)))
+  EG_GEMM_WALK((h3_tile<BM, BN, WMW, WNW, TWO>(args, w, ldsh)))
 }
 
 // The split of eg_gemm_f16x3's operands (eg_split_f16): exponents, marks and
@@ -1080,21 +1131,22 @@ struct SplitF16Args {
   int64_t chunks[2];      // 8-value chunks of each source, padding included
   int64_t rows, blk;      // blk: bytes of a 32-row block
   char* planes;
-  int32_t* exps;          // [rows rounded up to 32]
+  int32_t* exps[2];       // per source: [rows rounded up to 32]
   int32_t* wide;          // per 8 rows: any row marked
 };
 
 // A row is marked when more than 1 / kWideShare of its values are nonzero and
 // more than 2^24 below the largest of their source's part of the row (the
-// split's absolute 2^-40 of the row's largest is then 2^-16 of each, and such
-// values count for something: beside them, one huge value), when its largest
-// is not finite, or when that is so small (below 2^-87) that the scale would
-// leave fp32's range.  Fewer small values are left to the planes, since random
-// rows have some near zero; and so is a source far below the other, whose
-// products add less than the rounding of the other's (either rule marked rows
-// of the block's own gradients, and computing those again cost its backward
-// 0.1 to 5 ms).
+// split's absolute 2^-40 of that largest is then 2^-16 of each, and such
+// values count for something: beside them, one huge value), when a source's
+// largest is not finite, or when that is so small (below 2^-87) that the scale
+// would leave fp32's range.  Fewer small values are left to the planes, since
+// random rows have some near zero.
 constexpr int kWideLow = 40, kWideShare = 16;
+// Sources of a row more than 2^kApart apart mark it as well: from source 0's
+// units to source 1's is then 2^72 at most for a pair of rows, and sums of
+// up to 2^44 and products down to 2^-48 stay in fp32's normal range there.
+constexpr int kApart = 36;
 
 // A workgroup of 64 NW threads takes ROWS rows of one 32-row block (ROWS 8:
 // rows contiguous in memory, a wavefront covers 8 rows x 8 chunks, 256 bytes a
@@ -1164,12 +1216,25 @@ __global__ __launch_bounds__(64 * NW) void split_f16_kernel(const SplitF16Args a
     mxs[0] = max(mxs[0], s_max[0][q][r]);
     mxs[1] = max(mxs[1], s_max[1][q][r]);
   }
-  const uint32_t mx = max(mxs[0], mxs[1]);
-  // out of the scale's range: no planes
-  const bool out = mx != 0 && ((mx >> 23) >= 255 || (mx >> 23) < kWideLow);
-  // the row times 2^(14 - e) has its largest magnitude in [2^14, 2^15)
-  const int ex = mx == 0 || out ? 14 : (int)(mx >> 23) - 127;
-  const float scale = __uint_as_float((uint32_t)(127 + 14 - ex) << 23);
+  // out of the scale's range, or the sources too far apart: no planes
+  bool out = false;
+  int ex[2];
+  float scale[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    ex[s] = (int)(mxs[s] >> 23);
+    out |= mxs[s] != 0 && (ex[s] >= 255 || ex[s] < kWideLow);
+  }
+  // a source of zeros takes the other's exponent
+  ex[0] = mxs[0] == 0 ? ex[1] : ex[0];
+  ex[1] = mxs[1] == 0 ? ex[0] : ex[1];
+  out |= abs(ex[0] - ex[1]) > kApart;
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    // the source times 2^(14 - e) has its largest magnitude in [2^14, 2^15)
+    ex[s] = out || ex[s] == 0 ? 14 : ex[s] - 127;
+    scale[s] = __uint_as_float((uint32_t)(127 + 14 - ex[s]) << 23);
+  }
   // the bits of 2^-24 of each source's largest
   const uint32_t low0 = mxs[0] > (24u << 23) ? mxs[0] - (24u << 23) : 0;
   const uint32_t low1 = mxs[1] > (24u << 23) ? mxs[1] - (24u << 23) : 0;
@@ -1181,7 +1246,7 @@ __global__ __launch_bounds__(64 * NW) void split_f16_kernel(const SplitF16Args a
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       n_low += (__float_as_uint(v[e]) & 0x7fffffffu) - 1 < low;  // zero wraps to the largest
-      const float x = out ? 0.0f : v[e] * scale;
+      const float x = out ? 0.0f : v[e] * (c < a.chunks[0] ? scale[0] : scale[1]);
       hi[e] = (_Float16)x;
       lo[e] = (_Float16)(x - (float)hi[e]);
     }
@@ -1211,7 +1276,10 @@ __global__ __launch_bounds__(64 * NW) void split_f16_kernel(const SplitF16Args a
 #pragma unroll
   for (int q = 0; q < NW; ++q) n_low += s_low[q][r];
   const bool wide = out || (int64_t)n_low * kWideShare > a.src[0].cols + a.src[1].cols;
-  if (lane < ROWS && live) a.exps[row] = ex - 14;
+  if (lane < ROWS && live) {
+    a.exps[0][row] = ex[0] - 14;
+    a.exps[1][row] = ex[1] - 14;
+  }
   const uint64_t any = __ballot(wide && lane < ROWS);
   if (lane < ROWS / 8 && r0 + 8 * lane < a.rows) a.wide[r0 / 8 + lane] = (any >> (8 * lane) & 0xff) != 0;
 }
@@ -1861,6 +1929,10 @@ F16Src f16_src(const eg_f16_matrix* x, int s) {
 }
 
 int64_t blocks32(int64_t rows) { return (rows + 31) / 32; }
+
+// exps holds the rows' exponents of source 0, those of source 1, and the marks.
+int32_t* f16_exps(const eg_f16_matrix* x, int s) { return x->exps + blocks32(x->rows) * 32 * s; }
+int32_t* f16_marks(const eg_f16_matrix* x) { return x->exps + blocks32(x->rows) * 64; }
 }  // namespace
 }  // namespace eg
 
@@ -1868,7 +1940,7 @@ extern "C" {
 
 int64_t eg_f16_planes_bytes(int64_t rows, int64_t k) { return rows < 0 || k < 0 ? -1 : eg::blocks32(rows) * ((k + 31) / 32) * eg::kStepBytes; }
 
-int64_t eg_f16_exps_count(int64_t rows) { return rows < 0 ? -1 : eg::blocks32(rows) * 36; }
+int64_t eg_f16_exps_count(int64_t rows) { return rows < 0 ? -1 : eg::blocks32(rows) * 68; }
 
 int eg_split_f16(const eg_f16_matrix* x, void* stream) {
   using namespace eg;
@@ -1886,8 +1958,9 @@ int eg_split_f16(const eg_f16_matrix* x, void* stream) {
   a.rows = x->rows;
   a.blk = steps * kStepBytes;
   a.planes = (char*)x->planes;
-  a.exps = x->exps;
-  a.wide = x->exps + blocks32(x->rows) * 32;
+  a.exps[0] = f16_exps(x, 0);
+  a.exps[1] = f16_exps(x, 1);
+  a.wide = f16_marks(x);
   const int64_t blocks = trans ? blocks32(x->rows) : 4 * blocks32(x->rows);
   EG_CHECK_ARG(blocks < (1LL << 31), "too many rows");
   const int64_t chunks = 4 * steps;
@@ -1937,10 +2010,17 @@ int eg_gemm_f16x3(const eg_f16_matrix* a, const eg_f16_matrix* b, const eg_f16_m
     sg.ktiles = ka;
     g.n_seg = 1;
   }
-  g.scale = RowScale{a->exps, {b->exps, second->exps}};
+  const int last = a->n_src - 1;
+  g.scale = RowScale{f16_exps(a, last), {f16_exps(b, last), f16_exps(second, last)}};
+  g.first = RowScale{f16_exps(a, 0), {f16_exps(b, 0), f16_exps(second, 0)}};
+  g.kt_first = last > 0 ? (a->src[0].cols + 31) / 32 : ka;
   EG_CHECK_ARG(ka > 0, "k must be positive");
-  rc = launch_gemm<kX3BM, kX3BN>(kX3Shape, gemm_h3_kernel<kX3BM, kX3BN, kX3WM, kX3WN>, "gemm_h3_kernel", g, m, n, n2,
-                                 c, ldc, c2, ldc2, 0, 0, workspace, workspace_bytes, stream, g.scale);
+  const bool two = g.kt_first > 0 && g.kt_first < ka;
+  rc = launch_gemm<kX3BM, kX3BN>(kX3Shape,
+                                 two ? gemm_h3_kernel<kX3BM, kX3BN, kX3WM, kX3WN, true>
+                                     : gemm_h3_kernel<kX3BM, kX3BN, kX3WM, kX3WN, false>,
+                                 "gemm_h3_kernel", g, m, n, n2, c, ldc, c2, ldc2, 0, 0, workspace, workspace_bytes,
+                                 stream, g.scale);
   if (rc != EG_OK) return rc;
   WideArgs w{};
   for (int s = 0; s < 2; ++s) {
@@ -1949,9 +2029,9 @@ int eg_gemm_f16x3(const eg_f16_matrix* a, const eg_f16_matrix* b, const eg_f16_m
     w.b[1][s] = f16_src(second, s);
   }
   w.n_src = a->n_src;
-  w.wide[0] = a->exps + blocks32(m) * 32;
-  w.wide[1] = b->exps + blocks32(n) * 32;
-  w.wide[2] = b2 != nullptr ? b2->exps + blocks32(n2) * 32 : nullptr;
+  w.wide[0] = f16_marks(a);
+  w.wide[1] = f16_marks(b);
+  w.wide[2] = b2 != nullptr ? f16_marks(b2) : nullptr;
   w.m = m;
   w.n[0] = n;
   w.n[1] = n2;

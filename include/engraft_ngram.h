@@ -675,12 +675,13 @@ typedef struct eg_f16_matrix {
 int64_t eg_f16_planes_bytes(int64_t rows, int64_t k);
 int64_t eg_f16_exps_count(int64_t rows);
 
-/* Fills x's planes and exps: every row scaled by a power of two (its largest
- * magnitude to [2^14, 2^15), the exponent kept in exps) and split into fp16
- * planes hi = rne(x) and lo = rne(x - hi).  A row is marked when its largest
- * magnitude is not finite or below 2^-87, or when more than 1/16 of its values
- * are nonzero and more than 2^24 below the largest of their source's part.  No counterpart in the reference (part of its fp32
- * matmuls). */
+/* Fills x's planes and exps: each source's part of a row scaled by a power of
+ * two (its largest magnitude to [2^14, 2^15), the exponent kept in exps) and
+ * split into fp16 planes hi = rne(x) and lo = rne(x - hi).  A row is marked when
+ * a source's largest magnitude there is not finite or below 2^-87, when its two
+ * sources' are more than 2^36 apart, or when more than 1/16 of its values are
+ * nonzero and more than 2^24 below the largest of their source's part.  No
+ * counterpart in the reference (part of its fp32 matmuls). */
 int eg_split_f16(const eg_f16_matrix* x, void* stream);
 
 /* C [m, n] = A B^T and, with b2, C2 [m, n2] = A B2^T (m, n, n2 the operands'

@@ -14,6 +14,8 @@ import sys
 import pytest
 import torch
 
+from oracle import ple as P
+
 pytestmark = pytest.mark.gpu
 
 
@@ -97,3 +99,69 @@ def test_gemm_h3_repeats_bitwise_and_in_a_graph(cuda):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, gemm_h3((a,), (b,)))
+
+
+def _rel(got, exp):
+    return float((got.double() - exp).norm() / exp.norm())
+
+
+@pytest.mark.parametrize("layout", ["r", "t"])
+@pytest.mark.parametrize("p", [0, 12, 24, -24, 30, 36, -36, 37, 40, 60])
+def test_gemm_h3_sources_of_different_size(cuda, p, layout):
+    """a1 2^-p of a2 where b1 is 2^p of b2: both products count alike, so both
+    keep an fp32 product's accuracy.  2-norm bar, no K in it but the sums': 3 2^-22
+    for what the split drops of each product, and 2^-24 times the square root
+    of the number of fp32 additions (three products a 16-wide step)."""
+    from engraft_ngram_amd.ple import gemm_h3
+    _say(f"gemm_h3 two sources p={p} {layout}")
+    g = torch.Generator(device=cuda).manual_seed(100 + p)
+    m, n, ks = 300, 270, (320, 96)
+
+    def rnd(rows, k):
+        return torch.randn((rows, k) if layout == "r" else (k, rows), generator=g, device=cuda)
+    a, b = ([rnd(r, k) for k in ks] for r in (m, n))
+    a[0] *= 2.0 ** -p
+    b[0] *= 2.0 ** p
+    if layout == "t":
+        a, b = [x.T for x in a], [x.T for x in b]
+    a[0][5], a[1][7], b[0][9], b[1][11] = 0.0, 0.0, 0.0, 0.0  # rows with one source, of zeros in the other
+    got = gemm_h3(tuple(a), tuple(b))
+    exp = sum(x.double() @ y.double().T for x, y in zip(a, b))
+    bar = 3 * 2.0 ** -22 + (3 * sum(ks) / 16) ** 0.5 * 2.0 ** -24
+    assert _rel(got, exp) <= bar
+    for i in (5, 7):
+        assert _rel(got[i], exp[i]) <= bar
+    for j in (9, 11):
+        assert _rel(got[:, j], exp[:, j]) <= bar
+
+
+@pytest.mark.parametrize("wide", [1e-7, 1e-11])
+def test_ple_backward_with_a_value_projection_near_zero(cuda, wide):
+    """A block added with its value projection near zero: d_emb's two sources
+    (d_key w_key and d_value w_value) differ by its factor each, one up and one
+    down.  Against float64 autograd of the block; the bar allows each of its dozen
+    fp32 stages 2^-20 (the key's rounding enters through the gate's slope)."""
+    from engraft_ngram_amd import ple
+
+    class HP:
+        hc_mult, n_embd, f_norm_rms_eps, ple_ngram_size = 2, 256, 1e-30, 3
+    _say(f"ple backward with w_value times {wide}")
+    g = torch.Generator(device=cuda).manual_seed(8)
+    rnd = lambda *s: torch.randn(s, generator=g, device=cuda)
+    hc, n, t = 2, 256, 96
+    emb = rnd(t, n)
+    hidden = rnd(t, hc, n) * 0.1 + 0.5 * emb.unsqueeze(1)
+    wk, wv = rnd(hc * n, n) / 16, rnd(n, n) / 16 * wide
+    wk.view(hc, n, n).diagonal(dim1=1, dim2=2).add_(0.5)  # scores away from zero
+    w = ple.PleWeights(wk, wv, *(1 + 0.1 * rnd(hc * n) for _ in range(3)), rnd(hc * n, 4) / 2)
+    r = rnd(t, hc, n)
+    e = emb.clone().requires_grad_(True)
+    out, _ = ple.ple_forward(e, hidden, w, hidden.new_zeros((0, hc, n)), HP)
+    got, = torch.autograd.grad(out, e, r)
+    e64 = emb.cpu().double().requires_grad_(True)
+    w64 = {k: v.cpu().double() for k, v in vars(w).items()}
+    out64 = P.ple_forward(e64, hidden.cpu().double(), w64, torch.zeros((0, hc, n), dtype=torch.float64), hc, n,
+                          HP.f_norm_rms_eps, 3)[0]
+    exp, = torch.autograd.grad(out64, e64, r.cpu().double())
+    _say(f"d_emb off by {_rel(got.cpu(), exp):.2e}")
+    assert _rel(got.cpu(), exp) <= 1e-5
