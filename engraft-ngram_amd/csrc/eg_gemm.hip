@@ -1132,17 +1132,19 @@ struct SplitF16Args {
   int64_t rows, blk;      // blk: bytes of a 32-row block
   char* planes;
   int32_t* exps[2];       // per source: [rows rounded up to 32]
-  int32_t* wide;          // per 8 rows: any row marked
+  int32_t* wide;          // per 8 rows: a bit each, marked or not
 };
 
-// A row is marked when more than 1 / kWideShare of its values are nonzero and
-// more than 2^24 below the largest of their source's part of the row (the
-// split's absolute 2^-40 of that largest is then 2^-16 of each, and such
-// values count for something: beside them, one huge value), when a source's
-// largest is not finite, or when that is so small (below 2^-87) that the scale
-// would leave fp32's range.  Fewer small values are left to the planes, since
-// random rows have some near zero.
-constexpr int kWideLow = 40, kWideShare = 16;
+// The planes hold a value to 2^-22 of itself down to 2^-18 of the largest of its
+// source's part of the row, and to 2^-40 of that largest below.  A row is marked
+// when more than 1/16 of its nonzero values are below 2^-18, or more than 1/256
+// below 2^-24 (that many count for something where B is small at the large
+// ones), when a source's largest is not finite, or when that is so small (below
+// 2^-87) that the scale would leave fp32's range.  Fewer small values are left to
+// the planes, since random rows have some near zero: of the operands of the
+// block's own products, one row in 1,531 at most is marked (of the key's
+// gradient, where one stream's score is near zero); any such value would mark half of them.
+constexpr int kWideLow = 40, kShare18 = 16, kShare24 = 256;
 // Sources of a row more than 2^kApart apart mark it as well: from source 0's
 // units to source 1's is then 2^72 at most for a pair of rows, and sums of
 // up to 2^44 and products down to 2^-48 stay in fp32's normal range there.
@@ -1157,7 +1159,7 @@ constexpr int kApart = 36;
 template <int ROWS, int NW, int PER, bool TRANS>
 __global__ __launch_bounds__(64 * NW) void split_f16_kernel(const SplitF16Args a) {
   constexpr int CPW = 64 / ROWS;  // chunks a wavefront covers
-  __shared__ uint32_t s_max[2][NW][ROWS], s_low[NW][ROWS];
+  __shared__ uint32_t s_max[2][NW][ROWS], s_cnt[3][NW][ROWS];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane % ROWS, cl = lane / ROWS;
   const int64_t r0 = (int64_t)blockIdx.x * ROWS, row = r0 + r;
@@ -1235,18 +1237,26 @@ __global__ __launch_bounds__(64 * NW) void split_f16_kernel(const SplitF16Args a
     ex[s] = out || ex[s] == 0 ? 14 : ex[s] - 127;
     scale[s] = __uint_as_float((uint32_t)(127 + 14 - ex[s]) << 23);
   }
-  // the bits of 2^-24 of each source's largest
-  const uint32_t low0 = mxs[0] > (24u << 23) ? mxs[0] - (24u << 23) : 0;
-  const uint32_t low1 = mxs[1] > (24u << 23) ? mxs[1] - (24u << 23) : 0;
-  uint32_t n_low = 0;
+  if (wave == 0 && lane < ROWS && live) {
+    a.exps[0][row] = ex[0] - 14;
+    a.exps[1][row] = ex[1] - 14;
+  }
+  // nonzero values, and those below 2^-18 and 2^-24 of their source's largest
+  uint32_t cnt[3] = {0, 0, 0};
   auto put = [&](int64_t c, const float* v) {
     if (c >= n_chunks) return;
     f16x8 hi, lo;
-    const uint32_t low = c < a.chunks[0] ? low0 : low1;
+    const int s = c < a.chunks[0] ? 0 : 1;
+    const float sc = s ? scale[1] : scale[0];
+    // the bits of 2^-18 of the largest: above 0 unless the row is out or all zeros
+    const uint32_t l18 = (s ? mxs[1] : mxs[0]) - (18u << 23), l24 = l18 - (6u << 23);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      n_low += (__float_as_uint(v[e]) & 0x7fffffffu) - 1 < low;  // zero wraps to the largest
-      const float x = out ? 0.0f : v[e] * (c < a.chunks[0] ? scale[0] : scale[1]);
+      const uint32_t bits = (__float_as_uint(v[e]) & 0x7fffffffu) - 1;  // zero wraps to the largest
+      cnt[0] += bits + 1 != 0;
+      cnt[1] += bits < l18;
+      cnt[2] += bits < l24;
+      const float x = out ? 0.0f : v[e] * sc;
       hi[e] = (_Float16)x;
       lo[e] = (_Float16)(x - (float)hi[e]);
     }
@@ -1268,26 +1278,43 @@ __global__ __launch_bounds__(64 * NW) void split_f16_kernel(const SplitF16Args a
     }
   }
 #pragma unroll
-  for (int o = 32; o >= ROWS; o >>= 1) n_low += (uint32_t)__shfl_xor((int)n_low, o);
-  if (lane < ROWS) s_low[wave][r] = n_low;
+  for (int q = 0; q < 3; ++q) {
+#pragma unroll
+    for (int o = 32; o >= ROWS; o >>= 1) cnt[q] += (uint32_t)__shfl_xor((int)cnt[q], o);
+    if (lane < ROWS) s_cnt[q][wave][r] = cnt[q];
+  }
   __syncthreads();
   if (wave != 0) return;
-  n_low = 0;
 #pragma unroll
-  for (int q = 0; q < NW; ++q) n_low += s_low[q][r];
-  const bool wide = out || (int64_t)n_low * kWideShare > a.src[0].cols + a.src[1].cols;
-  if (lane < ROWS && live) {
-    a.exps[0][row] = ex[0] - 14;
-    a.exps[1][row] = ex[1] - 14;
+  for (int q = 0; q < 3; ++q) {
+    cnt[q] = 0;
+#pragma unroll
+    for (int u = 0; u < NW; ++u) cnt[q] += s_cnt[q][u][r];
   }
+  const bool wide = out || (int64_t)cnt[1] * kShare18 > cnt[0] || (int64_t)cnt[2] * kShare24 > cnt[0];
   const uint64_t any = __ballot(wide && lane < ROWS);
-  if (lane < ROWS / 8 && r0 + 8 * lane < a.rows) a.wide[r0 / 8 + lane] = (any >> (8 * lane) & 0xff) != 0;
+  if (lane < ROWS / 8 && r0 + 8 * lane < a.rows) a.wide[r0 / 8 + lane] = (int32_t)(any >> (8 * lane) & 0xff);
 }
 
-// The outputs of marked rows, in fp32: a 64 x 64 tile with a marked row of A or
-// B is computed again from the fp32 operands (any strides), its K in chunks
-// of 16 whose sums are added up.  Without a marked row a workgroup reads the
-// marks and exits.
+// The outputs of marked rows, in fp32: a 32 x 32 tile that meets a marked row of A
+// or B is computed again from the fp32 operands (any strides) on the fp32
+// matrix cores, and its outputs in those rows and columns are stored: an output
+// depends on its own two rows alone.  Few rows are marked, and then only their
+// strip of tiles is there to do, so the eight wavefronts of a workgroup share a
+// tile, each taking every eighth 32 k of it straight into registers (the next
+// step's while one is multiplied, no barrier), and their sums are added in
+// wavefront order; a step whose part of A is all zeros (positions without a
+// loss, in a weight gradient) is skipped.  Without a marked row a workgroup
+// reads the marks of its tiles and ends (5 us).  One marked row: d_emb of 2,560
+// columns and K 12,800 121 us, bound by its 80 tiles' loads and the fp32 matrix
+// cores of 80 CUs; 12,800 columns, K 2,560 57 us (64 x 64 tiles through LDS 200
+// and 108 us; 4 and 16 wavefronts 148 and 128 us).  Every row marked, 12,800 x
+// 2,560 outputs, K 1,531: 1.7 ms, bound by the 12.5 GB its tiles read from L2
+// (1.3 ms on 64 x 64 tiles, 5.8 ms on the vector units).
+constexpr int kWideGroups = 509;  // two workgroups a CU, and prime, so that a marked row's
+                                  // strip of tiles and a marked column's go over all of them
+constexpr int kWideWaves = 8;
+
 struct WideArgs {
   F16Src a[2], b[2][2];    // sources of A and of B per column group
   const int32_t* wide[3];  // marks of A, B, B2
@@ -1297,59 +1324,107 @@ struct WideArgs {
   int64_t ldc[2];
 };
 
-__global__ __launch_bounds__(256) void gemm_wide_kernel(const WideArgs g) {
-  const int tid = threadIdx.x;
-  int any = 0;
-  const int64_t lens[3] = {g.m, g.n[0], g.n[1]};
-#pragma unroll
-  for (int q = 0; q < 3; ++q)
-    for (int64_t i = tid; i < (lens[q] + 7) / 8; i += 256) any |= g.wide[q][i];
-  if (!__syncthreads_or(any)) return;
-  __shared__ float sa[16][65], sb[16][65];
-  const int64_t tm_n = (g.m + 63) / 64, tn0 = (g.n[0] + 63) / 64, tiles = tm_n * (tn0 + (g.n[1] + 63) / 64);
-  const int ty = tid >> 4, tx = tid & 15;
-  for (int64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
-    const int64_t tn = t / tm_n;
+__global__ __launch_bounds__(64 * kWideWaves, 4) void gemm_wide_kernel(const WideArgs g) {
+  constexpr int NT = 64 * kWideWaves;
+  __shared__ float s_part[kWideWaves][16][64];
+  __shared__ int s_tile[NT], s_mark[2][4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5;
+  const int64_t tm_n = (g.m + 31) / 32, tn0 = (g.n[0] + 31) / 32, tn_n = tn0 + (g.n[1] + 31) / 32;
+  const int64_t pitch = tn_n % kWideGroups == 0 ? tn_n + 1 : tn_n, tiles = tm_n * pitch;
+  auto row_marks = [&](int64_t tm, int q) { return 32 * tm + 8 * q < g.m ? g.wide[0][4 * tm + q] : 0; };
+  auto col_marks = [&](int64_t tn, int q) {
     const int grp = tn < tn0 ? 0 : 1;
-    const int64_t m0 = (t % tm_n) * 64, n0 = (grp ? tn - tn0 : tn) * 64;
+    const int64_t t = grp ? tn - tn0 : tn;
+    return 32 * t + 8 * q < g.n[grp] ? g.wide[1 + grp][4 * t + q] : 0;
+  };
+  // NT of the workgroup's tiles at a time: the marked ones, in order
+  for (int64_t base = blockIdx.x; base < tiles; base += (int64_t)kWideGroups * NT) {
+    const int64_t mine = base + (int64_t)kWideGroups * tid;
     int mark = 0;
-    if (tid < 8 && m0 + 8 * tid < g.m) mark = g.wide[0][m0 / 8 + tid];
-    if (tid >= 8 && tid < 16 && n0 + 8 * (tid - 8) < g.n[grp]) mark = g.wide[1 + grp][n0 / 8 + tid - 8];
+    if (mine < tiles && mine % pitch < tn_n)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) mark |= row_marks(mine / pitch, q) | col_marks(mine % pitch, q);
     if (!__syncthreads_or(mark)) continue;
-    float sum[4][4] = {};
-    for (int s = 0; s < g.n_src; ++s) {
-      const F16Src &xa = g.a[s], &xb = g.b[grp][s];
-      for (int64_t k0 = 0; k0 < xa.cols; k0 += 16) {
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int id = tid + 256 * e, r = id >> 4, k = id & 15;
-          const bool in = k0 + k < xa.cols;
-          sa[k][r] = in && m0 + r < g.m ? xa.x[(m0 + r) * xa.row_stride + (k0 + k) * xa.col_stride] : 0.0f;
-          sb[k][r] = in && n0 + r < g.n[grp] ? xb.x[(n0 + r) * xb.row_stride + (k0 + k) * xb.col_stride] : 0.0f;
-        }
-        __syncthreads();
-        float part[4][4] = {};
-#pragma unroll
-        for (int k = 0; k < 16; ++k)
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) part[i][j] = fmaf(sa[k][ty + 16 * i], sb[k][tx + 16 * j], part[i][j]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) sum[i][j] += part[i][j];
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int64_t row = m0 + ty + 16 * i, col = n0 + tx + 16 * j;
-        if (row < g.m && col < g.n[grp]) g.c[grp][row * g.ldc[grp] + col] = sum[i][j];
-      }
+    s_tile[tid] = mark != 0;
     __syncthreads();
+    for (int64_t i = 0; i < NT && base + kWideGroups * i < tiles; ++i) {
+      if (!s_tile[i]) continue;  // the same for every thread
+      const int64_t tile = base + kWideGroups * i, tm = tile / pitch, tn = tile % pitch;
+      const int grp = tn < tn0 ? 0 : 1;
+      const int64_t m0 = 32 * tm, n0 = 32 * (grp ? tn - tn0 : tn), n_grp = g.n[grp];
+      if (tid < 8) s_mark[tid >> 2][tid & 3] = tid < 4 ? row_marks(tm, tid) : col_marks(tn, tid - 4);
+      f32x16 acc;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+      for (int s = 0; s < g.n_src; ++s) {
+        const F16Src &xa = g.a[s], &xb = g.b[grp][s];
+        const int64_t k_len = xa.cols;
+        // a lane's row (past the end the last one: not stored) and, of 32 k, its half's sixteen
+        const float* pa = xa.x + min(m0 + (lane & 31), g.m - 1) * xa.row_stride + 16 * half * xa.col_stride;
+        const float* pb = xb.x + min(n0 + (lane & 31), n_grp - 1) * xb.row_stride + 16 * half * xb.col_stride;
+        auto load = [&](const F16Src& x, const float* p, int64_t k, float* v) {
+          p += k * x.col_stride;
+          if (k + 32 > k_len) {  // the last step: zeros past the end
+            const int left = (int)(k_len - k) - 16 * half;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+              v[e] = e < left ? *p : 0.0f;
+              p += x.col_stride;
+              asm volatile("" : "+v"(p));  // one address at a time: sixteen of them spill
+            }
+          } else if (x.col_stride == 1 && (x.row_stride & 3) == 0 && ((uintptr_t)x.x & 15) == 0) {
+#pragma unroll
+            for (int e = 0; e < 16; e += 4) {
+              const f32x4 y = *(const f32x4*)(p + e);
+              v[e] = y.x, v[e + 1] = y.y, v[e + 2] = y.z, v[e + 3] = y.w;
+            }
+          } else {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+              v[e] = *p;
+              p += x.col_stride;
+              asm volatile("" : "+v"(p));
+            }
+          }
+        };
+        float na[16], nb[16];
+        int64_t k = 32 * __builtin_amdgcn_readfirstlane(wave);
+        if (k < k_len) {
+          load(xa, pa, k, na);
+          load(xb, pb, k, nb);
+        }
+#pragma unroll 1
+        for (; k < k_len; k += 32 * kWideWaves) {
+          float fa[16], fb[16];
+          bool some = false;  // a value of A, or one of B whose product with zero is not zero
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            fa[e] = na[e], fb[e] = nb[e];
+            some |= fa[e] != 0.0f || (__float_as_uint(fb[e]) & 0x7f800000u) == 0x7f800000u;
+          }
+          if (k + 32 * kWideWaves < k_len) {
+            load(xa, pa, k + 32 * kWideWaves, na);
+            load(xb, pb, k + 32 * kWideWaves, nb);
+          }
+          if (__ballot(some) == 0) continue;
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[e], fb[e], acc, 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s_part[wave][r][lane] = acc[r];
+      __syncthreads();
+#pragma unroll
+      for (int r = wave; r < 16; r += kWideWaves) {
+        const int lr = 8 * (r >> 2) + 4 * half + (r & 3), lc = lane & 31;
+        float v = s_part[0][r][lane];
+#pragma unroll
+        for (int w = 1; w < kWideWaves; ++w) v += s_part[w][r][lane];
+        const bool marked = ((s_mark[0][lr >> 3] >> (lr & 7)) | (s_mark[1][lc >> 3] >> (lc & 7))) & 1;
+        if (marked && m0 + lr < g.m && n0 + lc < n_grp) g.c[grp][(m0 + lr) * g.ldc[grp] + n0 + lc] = v;
+      }
+      __syncthreads();  // the sums and marks are read
+    }
   }
 }
 
@@ -2039,9 +2114,7 @@ int eg_gemm_f16x3(const eg_f16_matrix* a, const eg_f16_matrix* b, const eg_f16_m
   w.c[1] = c2;
   w.ldc[0] = ldc;
   w.ldc[1] = ldc2;
-  const int64_t tiles = ((m + 63) / 64) * ((n + 63) / 64 + (n2 + 63) / 64);
-  hipLaunchKernelGGL(gemm_wide_kernel, dim3((unsigned)(tiles < 512 ? tiles : 512)), dim3(256), 0, (hipStream_t)stream,
-                     w);
+  hipLaunchKernelGGL(gemm_wide_kernel, dim3(kWideGroups), dim3(64 * kWideWaves), 0, (hipStream_t)stream, w);
   return launch_status("gemm_wide_kernel");
 }
 

@@ -679,19 +679,23 @@ int64_t eg_f16_exps_count(int64_t rows);
  * two (its largest magnitude to [2^14, 2^15), the exponent kept in exps) and
  * split into fp16 planes hi = rne(x) and lo = rne(x - hi).  A row is marked when
  * a source's largest magnitude there is not finite or below 2^-87, when its two
- * sources' are more than 2^36 apart, or when more than 1/16 of its values are
- * nonzero and more than 2^24 below the largest of their source's part.  No
- * counterpart in the reference (part of its fp32 matmuls). */
+ * sources' are more than 2^36 apart, or when more than 1/16 of its nonzero values
+ * are below 2^-18 of the largest of their source's part or more than 1/256 below
+ * 2^-24 of it.  No counterpart in the reference (part of its fp32 matmuls). */
 int eg_split_f16(const eg_f16_matrix* x, void* stream);
 
 /* C [m, n] = A B^T and, with b2, C2 [m, n2] = A B2^T (m, n, n2 the operands'
- * rows), with an fp32 matmul's accuracy on the fp16 matrix cores: hi*hi + hi*lo
- * + lo*hi of the operands' eg_split_f16 planes accumulated in fp32; the
- * outputs of marked rows in fp32 from the sources.  a and b with the same
- * sources' cols, at least one column.  Workspace of eg_gemm_workspace_size(m, n,
- * n2, k, 0) bytes, k the sum of the padded cols.  ple_forward's projections
- * and their gradients past a few rows (engraft/replica/layers.py:594-606, torch
- * fp32 matmuls). */
+ * rows) on the fp16 matrix cores: hi*hi + hi*lo + lo*hi of the operands'
+ * eg_split_f16 planes accumulated in fp32; the outputs of marked rows in fp32
+ * from the sources.  The others differ from A B^T by the fp32 sums' rounding and,
+ * per source, at most 3 2^-22 |a| |b| + 2^-40 (max|a| sum|b| + sum|a| max|b|)
+ * over the two rows: below an fp32 matmul's own error in the rows' norms.  Only
+ * an output far below its rows' norms, where few small values of one row meet
+ * the few values of the other that are not near zero, keeps less than there.
+ * a and b with the same sources' cols, at least one column.  Workspace of
+ * eg_gemm_workspace_size(m, n, n2, k, 0) bytes, k the sum of the padded cols.
+ * ple_forward's projections and their gradients past a few rows
+ * (engraft/replica/layers.py:594-606, torch fp32 matmuls). */
 int eg_gemm_f16x3(const eg_f16_matrix* a, const eg_f16_matrix* b, const eg_f16_matrix* b2, float* c, int64_t ldc,
                   float* c2, int64_t ldc2, void* workspace, int64_t workspace_bytes, void* stream);
 

@@ -165,3 +165,68 @@ def test_ple_backward_with_a_value_projection_near_zero(cuda, wide):
     exp, = torch.autograd.grad(out64, e64, r.cpu().double())
     _say(f"d_emb off by {_rel(got.cpu(), exp):.2e}")
     assert _rel(got.cpu(), exp) <= 1e-5
+
+
+def _sums_bar(k: int) -> float:
+    """2-norm: 3 2^-22 for what the split drops, 2^-24 times the root of the fp32 additions of a marked row's
+    output (one a k; the planes' three products take fewer)."""
+    return 3 * 2.0 ** -22 + k ** 0.5 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("layout", ["r", "t"])
+@pytest.mark.parametrize("p", [17, 19, 22, 24, 30, 50, 100])
+def test_gemm_h3_one_column_far_above_the_rest(cuda, p, layout):
+    """Rows of values in [1, 2) with one 2^p above them that meets weights 2^-p, or
+    zeros: most values lie below the planes' 22 bits, on either side."""
+    from engraft_ngram_amd.ple import gemm_h3
+    _say(f"gemm_h3 outlier column p={p} {layout}")
+    g = torch.Generator(device=cuda).manual_seed(p)
+    m, n, k = 150, 140, 1536
+    a = 1 + torch.rand((m, k), generator=g, device=cuda)
+    b = torch.randn((n, k), generator=g, device=cuda)
+    a[:, 700] *= 2.0 ** p
+    b[:, 700] *= 2.0 ** -p
+    b[::3, 700] = 0.0
+    if layout == "t":
+        a, b = (x.T.contiguous().T for x in (a, b))
+    exp = a.double() @ b.double().T
+    for got in (gemm_h3((a,), (b,)), gemm_h3((b,), (a,)).T):
+        assert _rel(got, exp) <= _sums_bar(k)
+        assert _rel(got[::3], exp[::3]) <= _sums_bar(k)
+        assert _rel(got[:, ::3], exp[:, ::3]) <= _sums_bar(k)
+
+
+@pytest.mark.parametrize("k,low,p", [(32, 31, 23), (1536, 90, 30), (1536, 90, 50), (1536, 1500, 20), (160, 2, 30)])
+def test_gemm_h3_low_values_among_zeros(cuda, k, low, p):
+    """One value 1, `low` values around 2^-p and zeros (a gradient over positions of
+    which few have a loss), against columns that are zero at the 1: the low values are
+    counted among the nonzero ones."""
+    from engraft_ngram_amd.ple import gemm_h3
+    _say(f"gemm_h3 low values k={k} low={low} p={p}")
+    g = torch.Generator(device=cuda).manual_seed(k + low + p)
+    m, n = 140, 130
+    a = torch.zeros((m, k), device=cuda)
+    a[:, 0] = 1.0
+    a[:, 1:1 + low] = torch.randn((m, low), generator=g, device=cuda) * 2.0 ** -p
+    a = a[:, torch.randperm(k, generator=g, device=cuda)]
+    b = torch.randn((n, k), generator=g, device=cuda)
+    b[:, (a[0] == 1.0).nonzero()[0, 0]] = 0.0
+    exp = a.double() @ b.double().T
+    for x, y in ((a, b), (a.T.contiguous().T, b.T.contiguous().T)):
+        assert _rel(gemm_h3((x,), (y,)), exp) <= _sums_bar(k)
+        assert _rel(gemm_h3((y,), (x,)).T, exp) <= _sums_bar(k)
+
+
+def test_gemm_h3_outputs_beside_a_marked_row(cuda):
+    """An output takes the fp32 path for its own rows' marks alone: its neighbours' bits stay."""
+    from engraft_ngram_amd.ple import gemm_h3
+    _say("gemm_h3 neighbours of marked rows")
+    g = torch.Generator(device=cuda).manual_seed(12)
+    a, b = _matrix(300, 100, g, cuda, "r"), _matrix(270, 100, g, cuda, "t")
+    first = gemm_h3((a,), (b,))
+    a[129, 3], b[77, 9], b[269, 0] = 1e30, float("inf"), 1e20
+    got = gemm_h3((a,), (b,))
+    _check(got, (a,), (b,))
+    keep = torch.ones_like(first, dtype=torch.bool)
+    keep[129], keep[:, 77], keep[:, 269] = False, False, False
+    assert torch.equal(got[keep], first[keep])
