@@ -41,6 +41,7 @@ from __future__ import annotations
 
 import ctypes
 import dataclasses
+import weakref
 
 import numpy as np
 import torch
@@ -112,29 +113,52 @@ def _block_torch(emb, hidden, w_key, w_value, nk, nq, nc, conv, hist, eps, dil, 
     return out, new_hist.reshape(-1, hc, n)
 
 
-class _TransposedCache:
-    """Row-major copies of the projection weights' transposes, kept between
-    steps: the backward's ``d_emb = d @ w`` is ``gemm_x3(d, w^T)``, whose B
-    operand is K-contiguous.  An entry is used only for the same tensor object
-    (weak reference) at the same version counter, so a weight that is
-    modified in place or freed and replaced is transposed again."""
+class _WeightCache:
+    """What a product takes of its weights (a transpose, split planes), kept
+    between steps: an entry is used only for the same tensor objects (weak
+    references) with the same storage at the same version counters, on the stream
+    that filled it, so a weight that is modified in place or freed and replaced is
+    taken again; entries of freed weights are dropped then.  A
+    call that is captured into a graph neither takes nor leaves an entry: an
+    entry found would be baked in (a replay would not see the weight
+    modified, and would read freed memory once the entry is dropped), and one
+    made is filled only when the graph replays."""
 
-    def __init__(self, size: int = 4):
+    def __init__(self, size: int):
         self._entries: list = []
         self._size = size
 
-    def get(self, w: torch.Tensor) -> torch.Tensor:
-        import weakref
-        for ref, version, wt in self._entries:
-            if ref() is w and version == w._version:
-                return wt
-        wt = w.T.contiguous()
-        self._entries = [e for e in self._entries if e[0]() is not None][-(self._size - 1):]
-        self._entries.append((weakref.ref(w), w._version, wt))
-        return wt
+    def get(self, ws: tuple, make, form=None):
+        """``make()``, or what it made for the same weights and ``form``."""
+        dev = ws[0].device
+        if dev.index is None or dev.index == torch.cuda.current_device():
+            capturing = torch.cuda.is_current_stream_capturing()
+        else:
+            with torch.cuda.device(dev):
+                capturing = torch.cuda.is_current_stream_capturing()
+        if capturing:
+            return make()
+        key = (form, _lib.stream_ptr(dev), *((w.data_ptr(), w.shape, w.stride()) for w in ws))
+        versions = [w._version for w in ws]
+        for refs, v, k, made in self._entries:
+            if k == key and v == versions and all(r() is w for r, w in zip(refs, ws)):
+                return made
+
+        self._entries = [e for e in self._entries if all(r() is not None for r in e[0])][1 - self._size:]
+        made = make()
+        self._entries.append(([weakref.ref(w) for w in ws], versions, key, made))
+        return made
 
 
-_WT = _TransposedCache()
+_WT = _WeightCache(4)
+_PLANES = _WeightCache(8)
+_HALF = _WeightCache(8)
+
+
+def _transposed(w: torch.Tensor) -> torch.Tensor:
+    """A row-major copy of a projection weight's transpose: the backward's ``d_emb =
+    d @ w`` is ``gemm_x3(d, w^T)``, whose B operand is K-contiguous."""
+    return _WT.get((w,), lambda: w.T.contiguous())
 
 
 class SplitPlanes:
@@ -172,34 +196,14 @@ def _empty_planes(rows: int, cols: int, device) -> "SplitPlanes":
     return p
 
 
-class _PlaneCache:
-    """Split planes of weights, kept between steps: an entry is used only for
-    the same tensor object (weak reference) at the same version counter."""
-
-    def __init__(self, size: int = 8):
-        self._entries: list = []
-        self._size = size
-
-    def get(self, w: torch.Tensor, three: bool = False) -> SplitPlanes:
-        import weakref
-        for ref, version, planes in self._entries:
-            if ref() is w and version == w._version and (planes.lo2 is not None) == three:
-                return planes
-        planes = SplitPlanes(w, three=three)
-        self._entries = [e for e in self._entries if e[0]() is not None][-(self._size - 1):]
-        self._entries.append((weakref.ref(w), w._version, planes))
-        return planes
-
-
-_PLANES = _PlaneCache()
-
-
 def _planes(x, cached: bool, three: bool = False) -> SplitPlanes:
     if isinstance(x, SplitPlanes):
         if three and x.lo2 is None:
             raise ValueError("gemm_x6 needs three-plane SplitPlanes (SplitPlanes(x, three=True))")
         return x
-    return _PLANES.get(x, three) if cached else SplitPlanes(x, three=three)
+    if cached:
+        return _PLANES.get((x,), lambda: SplitPlanes(x, three=three), three)
+    return SplitPlanes(x, three=three)
 
 
 def _gemm_workspace(m: int, n: int, n2: int, k: int, k_slices: int | None, dev, size_fn: str):
@@ -350,31 +354,9 @@ class HalfPlanes:
         return m
 
 
-class _HalfPlaneCache:
-    """``HalfPlanes`` of weights, kept between steps: an entry is used only for
-    the same tensor objects (weak references) with the same storage at the same
-    version counters, on the stream that filled it.  Planes made while a graph
-    is captured are not kept: they are filled when the graph replays."""
-
-    def __init__(self, size: int = 8):
-        self._entries: list = []
-        self._size = size
-
-    def get(self, ws: tuple, transposed: bool) -> HalfPlanes:
-        import weakref
-        key = (transposed, _lib.stream_ptr(ws[0].device), *((w.data_ptr(), w._version, w.shape, w.stride())
-                                                            for w in ws))
-        for refs, k, planes in self._entries:
-            if k == key and all(r() is w for r, w in zip(refs, ws)):
-                return planes
-        planes = HalfPlanes(tuple(w.T for w in ws) if transposed else ws)
-        if not torch.cuda.is_current_stream_capturing():
-            live = [e for e in self._entries if all(r() is not None for r in e[0])]
-            self._entries = live[-(self._size - 1):] + [(tuple(weakref.ref(w) for w in ws), key, planes)]
-        return planes
-
-
-_HALF = _HalfPlaneCache()
+def _half_planes(ws: tuple, transposed: bool) -> HalfPlanes:
+    """The ``HalfPlanes`` of weights, or of their transposes."""
+    return _HALF.get(ws, lambda: HalfPlanes(tuple(w.T for w in ws) if transposed else ws), transposed)
 
 
 def gemm_h3(a: tuple, b: tuple, b_n2: tuple | None = None, *, planes_b: HalfPlanes | None = None,
@@ -518,8 +500,8 @@ def _projection_backward(gemm: str, pairs: list) -> torch.Tensor:
     forward's GEMM."""
     if gemm == "bf16x6" and pairs[0][0].shape[0] > H3_MIN_ROWS:
         ds, ws = zip(*pairs)
-        return gemm_h3(ds, tuple(w.T for w in ws), planes_b=_HALF.get(ws, True))
-    flat = [x for d, w in pairs for x in (d, _WT.get(w))]
+        return gemm_h3(ds, tuple(w.T for w in ws), planes_b=_half_planes(ws, True))
+    flat = [x for d, w in pairs for x in (d, _transposed(w))]
     if pairs[0][0].shape[0] <= FEW_ROWS and _f32_in_place(*flat[1::2]):
         return gemm_f32(*flat, few_rows=True)
     if gemm == "bf16x3":
@@ -555,8 +537,8 @@ class _PleFn(torch.autograd.Function):
         elif gemm == "bf16x3":
             key, value = gemm_x3(SplitPlanes(emb32), wk32, cache_b=True, b_n2=wv32)
         elif gemm == "bf16x6" and t_len > H3_MIN_ROWS and not any(ctx.needs_input_grad):
-            key, value = gemm_h3((emb32,), (wk32,), (wv32,), planes_b=_HALF.get((wk32,), False),
-                                 planes_b2=_HALF.get((wv32,), False))
+            key, value = gemm_h3((emb32,), (wk32,), (wv32,), planes_b=_half_planes((wk32,), False),
+                                 planes_b2=_half_planes((wv32,), False))
         elif gemm == "bf16x6":
             key, value = gemm_x6(SplitPlanes(emb32, three=True), wk32, cache_b=True, b_n2=wv32)
         else:
@@ -687,7 +669,7 @@ class _PleFn(torch.autograd.Function):
             d_emb = None
             if need_emb:
                 # with both factors detached emb has no path to the output: None, as autograd gives
-                parts = [(d, _WT.get(w)) for d, w in ((pk, wk32), (pv, wv32)) if d is not None]
+                parts = [(d, _transposed(w)) for d, w in ((pk, wk32), (pv, wv32)) if d is not None]
                 if parts:
                     d_emb = gemm_x3(*[x for part in parts for x in part], cache_b=True).to(emb_dt)
             d_hist_in = d_full[:h0].reshape(h0, hc, n).to(hist_dt) if need_hist else None
