@@ -118,7 +118,7 @@ class _WeightCache:
     between steps: an entry is used only for the same tensor objects (weak
     references) with the same storage at the same version counters, on the stream
     that filled it, so a weight that is modified in place or freed and replaced is
-    taken again; entries of freed weights are dropped then.  A
+    taken again; entries of freed or modified weights are dropped then.  A
     call that is captured into a graph neither takes nor leaves an entry: an
     entry found would be baked in (a replay would not see the weight
     modified, and would read freed memory once the entry is dropped), and one
@@ -144,7 +144,11 @@ class _WeightCache:
             if k == key and v == versions and all(r() is w for r, w in zip(refs, ws)):
                 return made
 
-        self._entries = [e for e in self._entries if all(r() is not None for r in e[0])][1 - self._size:]
+        def current(refs, v):
+            alive = [r() for r in refs]
+            return all(w is not None and w._version == n for w, n in zip(alive, v))
+
+        self._entries = [e for e in self._entries if current(e[0], e[1])][1 - self._size:]
         made = make()
         self._entries.append(([weakref.ref(w) for w in ws], versions, key, made))
         return made

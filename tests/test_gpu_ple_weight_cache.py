@@ -75,6 +75,21 @@ def test_weight_modified_in_place_and_another_stream(cuda, t, gemm, grads):
     _equal(_call(w, *rest), got)
 
 
+@pytest.mark.parametrize("t", [48, 96])
+def test_planes_of_superseded_weights_are_let_go(cuda, t):
+    """Training both projections: what is held does not grow with the steps."""
+    _say(f"planes of superseded weights t={t}")
+    w, *rest = _inputs(cuda, t, 5)
+    held = []
+    for _ in range(12):
+        for grads in (False, True):
+            _call(w, *rest, "bf16x6", grads)
+        w["w_key"].mul_(1.01)
+        w["w_value"].mul_(1.01)
+        held.append(torch.cuda.memory_allocated())
+    assert held[-1] <= held[0], [h - held[0] for h in held]
+
+
 @pytest.mark.parametrize("t,gemm,grads", CASES)
 def test_captured_call_takes_the_weights_of_the_replay(cuda, t, gemm, grads):
     """Warmed up and captured on one stream, the weights modified in place
