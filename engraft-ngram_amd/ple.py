@@ -340,6 +340,11 @@ class HalfPlanes:
     the GEMM reads too; the planes do not keep them."""
 
     def __init__(self, of: tuple):
+        if len(of) not in (1, 2) or any(x.dim() != 2 or x.dtype != torch.float32 for x in of):
+            raise ValueError("HalfPlanes: one or two fp32 matrices expected")
+        if any(x.shape[0] != of[0].shape[0] or x.device != of[0].device for x in of):
+            raise ValueError(f"HalfPlanes: two matrices of the same rows on one device expected, got "
+                             f"{[tuple(x.shape) for x in of]}")
         lib = _lib.load()
         self.shapes = tuple(tuple(x.shape) for x in of)
         self.rows = of[0].shape[0]
@@ -371,10 +376,21 @@ def gemm_h3(a: tuple, b: tuple, b_n2: tuple | None = None, *, planes_b: HalfPlan
     fp16 planes, three products accumulated in fp32; rows beyond the planes'
     range computed in fp32).  ``b_n2``: a second column group over the same
     ``a``; the result is then a pair.  ``planes_b`` / ``planes_b2``: the planes
-    of ``b`` / ``b_n2`` where the caller keeps them."""
-    for name, side in (("b", b), ("b_n2", b_n2)):
-        if side is not None and [x.shape[1] for x in side] != [x.shape[1] for x in a]:
-            raise ValueError(f"gemm_h3: a and {name} must have the same k")
+    of ``b`` / ``b_n2`` where the caller keeps them.  Operands of another dtype are
+    converted, as :func:`gemm_f32`'s."""
+    a, b, b_n2 = (side if side is None else tuple(x.float() for x in side) for side in (a, b, b_n2))
+    for name, side, planes in (("b", b, planes_b), ("b_n2", b_n2, planes_b2)):
+        if side is None:
+            if planes is not None:
+                raise ValueError("gemm_h3: planes_b2 without b_n2")
+            continue
+        if any(x.dim() != 2 for x in a + side) or [x.shape[1] for x in side] != [x.shape[1] for x in a]:
+            raise ValueError(f"gemm_h3: a and {name} must be matrices of the same k")
+        if any(x.device != a[0].device for x in side):
+            raise ValueError(f"gemm_h3: a and {name} must be on one device")
+        if planes is not None and (planes.shapes != tuple(tuple(x.shape) for x in side) or
+                                   planes.planes.device != a[0].device):
+            raise ValueError(f"gemm_h3: the planes given are not those of {name}: {planes.shapes}")
     pa = HalfPlanes(a)
     pb = planes_b if planes_b is not None else HalfPlanes(b)
     pb2 = None if b_n2 is None else planes_b2 if planes_b2 is not None else HalfPlanes(b_n2)

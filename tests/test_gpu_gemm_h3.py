@@ -230,3 +230,12 @@ def test_gemm_h3_outputs_beside_a_marked_row(cuda):
     keep = torch.ones_like(first, dtype=torch.bool)
     keep[129], keep[:, 77], keep[:, 269] = False, False, False
     assert torch.equal(got[keep], first[keep])
+
+
+def test_gemm_h3_converts_other_dtypes(cuda):
+    from engraft_ngram_amd.ple import gemm_h3
+    _say("gemm_h3 of bf16 and float64 operands")
+    g = torch.Generator(device=cuda).manual_seed(13)
+    a, b = (torch.randn((r, 70), generator=g, device=cuda).bfloat16() for r in (40, 33))
+    exp = gemm_h3((a.float(),), (b.float(),))
+    assert torch.equal(gemm_h3((a,), (b.double(),)), exp)
