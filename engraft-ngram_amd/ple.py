@@ -500,6 +500,7 @@ def _f32_in_place(*ws: torch.Tensor) -> bool:
 
 
 WGRAD_MAX_TAPS = 8  # eg_ple_weight_grads' built tap counts (1..8)
+SUMS_MAX_ROWS = 65535 * 63  # eg_ple_conv_backward_sums' rows: one grid row per 63 of them
 
 
 def _weight_grad(d_y: torch.Tensor, x: torch.Tensor, w: torch.Tensor, gemm: str = "fp32") -> torch.Tensor:
@@ -535,6 +536,14 @@ def _native_backward_ok(hc: int, n: int, taps: int, dil: int, weights: bool = Fa
     """The HIP backward's built limits (eg_ple_gate_backward, eg_ple_conv_backward,
     and with ``weights`` eg_ple_weight_grads)."""
     return hc <= 4 and n <= 4096 and (taps - 1) * dil <= 32 and (not weights or taps <= WGRAD_MAX_TAPS)
+
+
+def _gated_ok(rows: int, t_len: int, n: int, taps: int, dil: int, norm_or_conv_grads: bool) -> bool:
+    """Whether the block runs without its normed rows in memory (eg_ple_conv_gated), ``rows``
+    with the history's: the shape that is built and, where norm or convolution weights need
+    gradients, the rows that eg_ple_conv_backward_sums takes."""
+    return (taps == 4 and dil == 3 and n % 256 == 0 and t_len > 0
+            and (not norm_or_conv_grads or rows <= SUMS_MAX_ROWS))
 
 
 class _PleFn(torch.autograd.Function):
@@ -573,8 +582,7 @@ class _PleFn(torch.autograd.Function):
         taps = conv32.shape[1]
         native = any(ctx.needs_input_grad) and _native_backward_ok(hc, n, taps, int(dil),
                                                                    weights=any(ctx.needs_input_grad[2:8]))
-        # without the normed rows in memory where the gated convolution is built
-        gated = (taps == 4 and int(dil) == 3 and n % 256 == 0 and t_len > 0
+        gated = (_gated_ok(h0 + t_len, t_len, n, taps, int(dil), any(ctx.needs_input_grad[4:8]))
                  and not (hidden32.data_ptr() | hist.data_ptr() | nc32.data_ptr() | conv32.data_ptr()) % 16)
         rstd = torch.empty((t_len, hc, 3), **f32) if native or gated else None
         full = None if gated else torch.empty((h0 + t_len, hc * n), **f32)

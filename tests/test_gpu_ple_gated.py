@@ -138,3 +138,32 @@ def test_history_written_over_before_the_backward(cuda, weights):
         res.append(torch.autograd.grad(out, leaves, r))
     for a, b in zip(*res):
         assert torch.equal(a, b)
+
+
+def test_gradients_past_the_weight_sums_rows(cuda, monkeypatch):
+    """A call of more rows than eg_ple_conv_backward_sums takes keeps its normed rows (the limit set
+    to the call's own here): outputs and history as within the limit bit for bit, every
+    gradient within T 2^-20 of its largest entry (other orders of the sums over T positions)."""
+    from engraft_ngram_amd import _lib, ple
+    print("[gpu-test] gradients past the weight sums' rows", file=sys.stderr, flush=True)
+
+    class HP:
+        hc_mult, n_embd, f_norm_rms_eps, ple_ngram_size = 2, 256, 1e-6, 3
+    g = torch.Generator(device=cuda).manual_seed(9)
+    rnd = lambda *s: torch.randn(s, generator=g, device=cuda)
+    hc, n, t = 2, 256, 70
+    w = ple.PleWeights(rnd(hc * n, n) / 16, rnd(n, n) / 16, *(1 + 0.1 * rnd(hc * n) for _ in range(3)), rnd(hc * n, 4))
+    emb, hidden, hist, r = rnd(t, n), rnd(t, hc, n) + 0.5, rnd(9, hc, n), rnd(t, hc, n)
+    real, res = _lib.call, []
+    for limit in (ple.SUMS_MAX_ROWS, t + 8):
+        monkeypatch.setattr(ple, "SUMS_MAX_ROWS", limit)
+        called = []
+        monkeypatch.setattr(_lib, "call", lambda name, *a: (called.append(name), real(name, *a))[1])
+        leaves = [x.clone().requires_grad_(True) for x in (emb, hidden, hist, *vars(w).values())]
+        out, new = ple.ple_forward(leaves[0], leaves[1], ple.PleWeights(*leaves[3:]), leaves[2], HP)
+        res.append((out, new, *torch.autograd.grad(out, leaves, r)))
+        past = limit < t + 9
+        assert ("eg_ple_weight_grads" in called) is past and ("eg_ple_conv_backward_sums" in called) is not past
+    assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
+    for a, b in zip(res[0][2:], res[1][2:]):
+        assert float((a - b).abs().max()) <= t * 2.0 ** -20 * float(a.abs().max())
