@@ -47,8 +47,7 @@ def _matrix(rows, k, g, dev, layout):
     return val(rows, k)
 
 
-# edges of the 256 x 256 tiles, 32-row blocks and 32-wide K steps; the register and the
-# re-reading forms of the split (rows of 2560 / columns of 2048 values); K ranges of the last round
+# edges of the 256 x 256 tiles, 32-row blocks and 32-wide K steps; K ranges of the last round
 @pytest.mark.parametrize("m,n,n2,ks,layout", [
     (1, 1, 0, (1,), "r"), (65, 33, 31, (31,), "r"), (256, 256, 256, (32,), "slice"), (257, 255, 0, (33, 65), "r"),
     (300, 513, 1, (2560,), "r"), (31, 260, 40, (2561,), "slice"), (130, 200, 0, (2048,), "t"),
@@ -62,6 +61,19 @@ def test_gemm_h3_against_float64(cuda, m, n, n2, ks, layout):
     got = gemm_h3(a, b, b2)
     for o, y in zip(got if n2 else (got,), (b, b2)):
         _check(o, a, y)
+
+
+# the split keeps a row's values in registers up to 2,560 of them (80 steps of 32), a column's up
+# to 1,536 (48 steps), and reads longer ones again: the last of each form and the first past it
+@pytest.mark.parametrize("layout,ks", [("r", (2529,)), ("r", (2560,)), ("r", (2561,)), ("slice", (2560,)),
+                                       ("r", (2500, 40)), ("r", (2530, 40)), ("t", (1505,)), ("t", (1536,)),
+                                       ("t", (1537,)), ("t", (1568,)), ("t", (1500, 20)), ("t", (1500, 40))])
+def test_gemm_h3_split_in_registers_and_read_again(cuda, layout, ks):
+    from engraft_ngram_amd.ple import gemm_h3
+    _say(f"gemm_h3 split forms {layout} k={ks}")
+    g = torch.Generator(device=cuda).manual_seed(sum(ks))
+    a, b = (tuple(_matrix(r, k, g, cuda, layout) for k in ks) for r in (41, 67))
+    _check(gemm_h3(a, b), a, b)
 
 
 @pytest.mark.parametrize("layout", ["r", "t"])

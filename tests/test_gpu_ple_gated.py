@@ -1,7 +1,7 @@
 """eg_ple_conv_gated (the convolution over normed rows it computes from the
 gate's factors) against eg_ple_gate + eg_ple_conv with those rows in memory:
 output, pre-activation and new history bit for bit, at the edges of its
-32-position runs, its 256-channel blocks and the history's 9 rows."""
+16-position runs, its 256-channel blocks and the history's 9 rows."""
 from __future__ import annotations
 
 import sys
@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("t,h0,hc,n", [(1, 0, 4, 2560), (1, 9, 4, 2560), (8, 1, 1, 256), (9, 0, 3, 512),
-                                       (31, 4, 4, 256), (32, 9, 2, 768), (33, 12, 4, 512), (100, 9, 4, 2560)])
+                                       (15, 9, 2, 256), (16, 9, 4, 256), (17, 3, 2, 512), (31, 4, 4, 256), (32, 9, 2, 768), (33, 12, 4, 512), (100, 9, 4, 2560)])
 def test_conv_gated_is_the_convolution_of_the_normed_rows(cuda, t, h0, hc, n):
     from engraft_ngram_amd import _lib
     print(f"[gpu-test] conv_gated t={t} h0={h0} hc={hc} n={n}", file=sys.stderr, flush=True)

@@ -312,3 +312,13 @@ def test_rowstore_padded_iq4nl_rows():
         T.RowStore("iq4_nl", 160, torch.zeros((6, 88), dtype=torch.uint8))
     with pytest.raises(ValueError):
         T.RowStore.empty("q8_0", 6, 128, "cpu", row_stride=256)
+
+
+@pytest.mark.parametrize("n", [0, 1, (1 << 18) - 1, 1 << 18, (1 << 18) + 1, 700_001, 8_000_000])
+def test_scan_pieces_cover_a_block(n):
+    """The pieces of a block follow each other and cover it; the first is at most 2^18 tokens."""
+    *_, damage = _pkg()
+    pieces = damage._pieces(n)
+    assert [a for a, _ in pieces] == [0, *(b for _, b in pieces)][:len(pieces)]
+    assert (pieces[-1][1] if pieces else 0) == n and all(0 < b - a <= 1 << 20 for a, b in pieces)
+    assert not pieces or pieces[0][1] <= 1 << 18
