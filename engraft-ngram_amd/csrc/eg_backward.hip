@@ -591,7 +591,7 @@ struct SegArgs {
   TableDev base;          // for the pull term (rows0 at the variables' ids)
   const float* anchor;    // or rows0 per variable [n_var, dim]
   int64_t step;
-  int32_t dense;          // stamp the rows hit (the dense pass skips them)
+  int32_t dense;          // every variable is stepped; the rows hit are stamped (the caller's record)
   float w1, b2, w2, bc2s, eps, neg_step_size, l2c;
   int32_t overwrite;      // gradient mode: grad_out = the sum (0 for a variable no slot hits), not +=
 };

@@ -71,6 +71,7 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -695,6 +696,8 @@ __global__ __launch_bounds__(BM * BN / 64) void gemm_f32_kernel(const F32Args ar
 // cost the address path a request a lane (42 us).  131 MB of the PLE key and
 // value weights, 5 to 8 rows: 36 us, 32 rows: 44 us; 115 us for gemm_x6_kernel's 256-row tiles
 // (196 MB of planes, its parts' sum included).
+// The 128 registers of four wavefronts a SIMD are 6 (MR 8) and 16 (MR 32) too few: the
+// compiler keeps 28 and 68 bytes a lane in scratch.
 constexpr int kFewRows = 32;  // SETS: 2 or 3
 
 template <int NW, int MR, int SETS>
@@ -893,20 +896,20 @@ __global__ __launch_bounds__(256) void gemm_f32_vec_kernel(const F32Args args) {
 
 // gemm_h3_kernel (eg_gemm_f16x3): fp32 accuracy from three products on the
 // fp16 matrix cores; 378 us for the PLE key + value of 2,048 positions, its
-// operand's split and the marked rows' check included, against 691 us for the
+// operand's split and gemm_wide_kernel's check included, against 691 us for the
 // six bf16 products (bound by the matrix cores and their operands' path
 // through LDS, as gemm_x3_kernel).  Every row of an operand's source is scaled by a power of two that
 // puts its largest magnitude in [2^14, 2^15) and split into hi = rne16(x) and
 // lo = rne16(x - hi): 22 significand bits where the element is at least
-// 2^-18 of the row's largest, an absolute 2^-40 of it below.  C = hi*hi +
+// 2^-18 of the row's largest, an absolute 2^-39 of it below.  C = hi*hi +
 // hi*lo + lo*hi in fp32, scaled back when it is stored (RowScale); the dropped
 // lo*lo is at most 2^-22 of |a||b|.  Half the matrix work of the six bf16
 // products (gemm_x6_kernel) and four planes loaded in place of its eight, and
 // fewer fp32 additions: its error against float64 is no larger (2048 x 10240 x
 // 2560 of N(0, 1): 5.3e-7 in the 2-norm, against 8.3e-7 for the six products
-// and for gemm_f32_kernel).  Rows the planes do not hold (one value far above
-// the rest, an infinity, a NaN) are marked by the split and their outputs
-// computed by gemm_wide_kernel instead.
+// and for gemm_f32_kernel).  What the planes
+// do not hold (values far below their row's largest, an infinity, a NaN) the split
+// marks, and gemm_wide_kernel computes the outputs for which it counts.
 //
 // Planes are fragment-major: 32 rows x 32 k are one 4 KB run, [k half of 16]
 // [hi, lo][lane][8 values], lane l holding row l % 32 and k 8 (l / 32) .. + 7 of
@@ -1132,19 +1135,30 @@ struct SplitF16Args {
   int64_t rows, blk;      // blk: bytes of a 32-row block
   char* planes;
   int32_t* exps[2];       // per source: [rows rounded up to 32]
-  int32_t* wide;          // per 8 rows: a bit each, marked or not
+  int32_t* info[2];       // per source and row: kHard, kLossy and the values near the largest
+  int32_t* sum8;          // per 8 rows three: a bit a row hard, lossy in source 0, in source 1; the fewest near values
 };
 
 // The planes hold a value to 2^-22 of itself down to 2^-18 of the largest of its
-// source's part of the row, and to 2^-40 of that largest below.  A row is marked
-// when more than 1/16 of its nonzero values are below 2^-18, or more than 1/256
-// below 2^-24 (that many count for something where B is small at the large
-// ones), when a source's largest is not finite, or when that is so small (below
-// 2^-87) that the scale would leave fp32's range.  Fewer small values are left to
-// the planes, since random rows have some near zero: of the operands of the
-// block's own products, one row in 1,531 at most is marked (of the key's
-// gradient, where one stream's score is near zero); any such value would mark half of them.
-constexpr int kWideLow = 40, kShare18 = 16, kShare24 = 256;
+// source's part of the row, and to 2^-39 of that largest below.  A row is hard (all
+// its outputs computed in fp32) when a source's largest is not finite or so small
+// (below 2^-87) that the scale would leave fp32's range.  It is lossy in a source
+// when the octaves that its values there lie below 2^-18, and eight times those below
+// 2^-24, come to more than 12/128 of one per nonzero value (one in 16 an octave and a half
+// below 2^-18, one in 256 below 2^-26).  Rows with fewer small values are not
+// lossy, since random rows have some near zero.
+// What a lossy row loses counts where the other row is small at its large
+// values and only there: an output of it is computed in fp32 unless enough products are
+// of two near values, of 2^-6 of their rows' largest at least.  Of K products n_a +
+// n_b - K are, n the near values of either row; from K / 16 on sum |a b| is
+// at least K 2^-16 of the largest's product and the loss at most 2^-38 K of it, 2^-22
+// of sum |a b|.  (A position where one stream's score is near zero is lossy in the
+// key's gradient; its near values are that stream's, and no weight is small at
+// all of them.  Computing such rows again, one or two of 1,531, cost the block's
+// d_emb 121 us.)
+constexpr int kWideLow = 40, kNearShare = 16;
+constexpr float kLost = 12.0f;  // in 1/128 octaves
+constexpr int kHard = 1 << 30, kLossy = 1 << 29, kNear = kLossy - 1;  // kNear: a row of zeros, all near
 // Sources of a row more than 2^kApart apart mark it as well: from source 0's
 // units to source 1's is then 2^72 at most for a pair of rows, and sums of
 // up to 2^44 and products down to 2^-48 stay in fp32's normal range there.
@@ -1159,16 +1173,20 @@ constexpr int kApart = 36;
 template <int ROWS, int NW, int PER, bool TRANS>
 __global__ __launch_bounds__(64 * NW) void split_f16_kernel(const SplitF16Args a) {
   constexpr int CPW = 64 / ROWS;  // chunks a wavefront covers
-  __shared__ uint32_t s_max[2][NW][ROWS], s_cnt[3][NW][ROWS];
+  __shared__ uint32_t s_max[2][NW][ROWS];
+  __shared__ float s_tally[2][3][NW][ROWS];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane % ROWS, cl = lane / ROWS;
   const int64_t r0 = (int64_t)blockIdx.x * ROWS, row = r0 + r;
   const bool live = row < a.rows;
   const int64_t n_chunks = a.chunks[0] + a.chunks[1];
 
+  // both read once: indexed by a lane's source they are loaded before each of its chunks
+  const F16Src src0 = a.src[0], src1 = a.src[1];
   auto load = [&](int64_t c, float* v) {
     const int s = c < a.chunks[0] ? 0 : 1;
-    const F16Src& src = a.src[s];
+    const F16Src src = {s ? src1.x : src0.x, s ? src1.cols : src0.cols, s ? src1.row_stride : src0.row_stride,
+                        s ? src1.col_stride : src0.col_stride};
     const int64_t k = (s ? c - a.chunks[0] : c) * 8;
     const float* x = src.x + row * src.row_stride + k * src.col_stride;
     if (!live || c >= n_chunks) {
@@ -1241,24 +1259,43 @@ __global__ __launch_bounds__(64 * NW) void split_f16_kernel(const SplitF16Args a
     a.exps[0][row] = ex[0] - 14;
     a.exps[1][row] = ex[1] - 14;
   }
-  // nonzero values, and those below 2^-18 and 2^-24 of their source's largest
-  uint32_t cnt[3] = {0, 0, 0};
+  // per source: nonzero values, near values, and 1/128 octaves lost, from the upper
+  // halves of two values a word at a time (8 bits of exponent, 7 of the significand).
+  // 1,531 rows of 12,800 values: 69 us, 64 us with the planes and one count alone
+  float tally[2][3] = {};
+  u16x2 one = 1;
+  asm("" : "+v"(one));  // min(h, 1) stays that: two compares and selects a word otherwise
   auto put = [&](int64_t c, const float* v) {
     if (c >= n_chunks) return;
     f16x8 hi, lo;
     const int s = c < a.chunks[0] ? 0 : 1;
     const float sc = s ? scale[1] : scale[0];
-    // the bits of 2^-18 of the largest: above 0 unless the row is out or all zeros
-    const uint32_t l18 = (s ? mxs[1] : mxs[0]) - (18u << 23), l24 = l18 - (6u << 23);
+    const uint16_t t18 = (uint16_t)(((s ? mxs[1] : mxs[0]) >> 16) - 18 * 128);  // above 24 octaves' unless out or zero
+    const u16x2 v18 = t18, v24 = (uint16_t)(t18 - 6 * 128), v6 = (uint16_t)(t18 + 12 * 128 - 1);
+    uint32_t seen = 0, lost = 0, pair = 0;  // seen: nonzero + 256 near
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const uint32_t bits = (__float_as_uint(v[e]) & 0x7fffffffu) - 1;  // zero wraps to the largest
-      cnt[0] += bits + 1 != 0;
-      cnt[1] += bits < l18;
-      cnt[2] += bits < l24;
-      const float x = out ? 0.0f : v[e] * sc;
+      float y = v[e];
+      asm("" : "+v"(y));  // nothing of the maximum's pass is kept in registers for this one
+      if (e & 1) {
+        const uint32_t tops = __builtin_amdgcn_perm(__float_as_uint(y), pair, 0x07060302) & 0x7fff7fffu;
+        const u16x2 h = __builtin_bit_cast(u16x2, tops), z = h - one;  // zero wraps to the largest
+        lost = __builtin_amdgcn_udot2(__builtin_elementwise_sub_sat(v18, z), one, lost, false);
+        lost = __builtin_amdgcn_udot2(__builtin_elementwise_sub_sat(v24, z), (u16x2)8, lost, false);
+        seen = __builtin_amdgcn_udot2(__builtin_elementwise_min(h, one), one, seen, false);
+        seen = __builtin_amdgcn_udot2(__builtin_elementwise_min(__builtin_elementwise_sub_sat(h, v6), one),
+                                      (u16x2)256, seen, false);
+      }
+      pair = __float_as_uint(y);
+      const float x = out ? 0.0f : y * sc;
       hi[e] = (_Float16)x;
       lo[e] = (_Float16)(x - (float)hi[e]);
+    }
+    const float got[3] = {(float)(seen & 0xff), (float)(seen >> 8), (float)lost};
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      tally[0][q] += s ? 0.0f : got[q];
+      tally[1][q] += s ? got[q] : 0.0f;
     }
     char* o = a.planes + (row >> 5) * a.blk + (c >> 2) * kStepBytes + ((c >> 1) & 1) * 2 * kFragBytes +
               ((row & 31) + 32 * (c & 1)) * 16;
@@ -1267,7 +1304,10 @@ __global__ __launch_bounds__(64 * NW) void split_f16_kernel(const SplitF16Args a
   };
   if constexpr (PER > 0) {
 #pragma unroll
-    for (int i = 0; i < PER; ++i) put((int64_t)(i * NW + wave) * CPW + cl, kept[i]);
+    for (int i = 0; i < PER; ++i) {
+      put((int64_t)(i * NW + wave) * CPW + cl, kept[i]);
+      __builtin_amdgcn_sched_barrier(0);  // one chunk's values at a time: several at once take 80 registers more
+    }
   } else {
     for (int64_t c = wave * CPW + cl; c < n_chunks; c += 2 * NW * CPW) {
       float v[2][8];
@@ -1278,46 +1318,68 @@ __global__ __launch_bounds__(64 * NW) void split_f16_kernel(const SplitF16Args a
     }
   }
 #pragma unroll
-  for (int q = 0; q < 3; ++q) {
+  for (int s = 0; s < 2; ++s)
 #pragma unroll
-    for (int o = 32; o >= ROWS; o >>= 1) cnt[q] += (uint32_t)__shfl_xor((int)cnt[q], o);
-    if (lane < ROWS) s_cnt[q][wave][r] = cnt[q];
-  }
+    for (int q = 0; q < 3; ++q) {
+#pragma unroll
+      for (int o = 32; o >= ROWS; o >>= 1) tally[s][q] += __shfl_xor(tally[s][q], o);
+      if (lane < ROWS) s_tally[s][q][wave][r] = tally[s][q];
+    }
   __syncthreads();
   if (wave != 0) return;
+  // lanes of the same row hold the same
+  int fewest[2];
+  uint64_t lossy[2];
 #pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    cnt[q] = 0;
+  for (int s = 0; s < 2; ++s) {
 #pragma unroll
-    for (int u = 0; u < NW; ++u) cnt[q] += s_cnt[q][u][r];
+    for (int q = 0; q < 3; ++q) {
+      tally[s][q] = 0.0f;
+#pragma unroll
+      for (int u = 0; u < NW; ++u) tally[s][q] += s_tally[s][q][u][r];
+    }
+    const bool is = tally[s][2] > kLost * tally[s][0];
+    fewest[s] = tally[s][0] == 0.0f || !live ? kNear : (int)fminf(tally[s][1], (float)(kNear / 2));
+    if (lane < ROWS && live) a.info[s][row] = fewest[s] | (is ? kLossy : 0) | (out ? kHard : 0);
+    lossy[s] = __ballot(is);
+#pragma unroll
+    for (int o = 4; o >= 1; o >>= 1) fewest[s] = min(fewest[s], __shfl_xor(fewest[s], o));
+    fewest[s] = __shfl(fewest[s], 8 * lane & 63);  // of rows 8 lane .. 8 lane + 7
   }
-  const bool wide = out || (int64_t)cnt[1] * kShare18 > cnt[0] || (int64_t)cnt[2] * kShare24 > cnt[0];
-  const uint64_t any = __ballot(wide && lane < ROWS);
-  if (lane < ROWS / 8 && r0 + 8 * lane < a.rows) a.wide[r0 / 8 + lane] = (int32_t)(any >> (8 * lane) & 0xff);
+  const uint64_t hard = __ballot(out);
+  if (lane < ROWS / 8 && r0 + 8 * lane < a.rows) {
+    int32_t* o = a.sum8 + 3 * (r0 / 8 + lane);
+    o[0] = (int32_t)((hard >> 8 * lane & 0xff) | (lossy[0] >> 8 * lane & 0xff) << 8 |
+                     (lossy[1] >> 8 * lane & 0xff) << 16);
+    o[1] = fewest[0];
+    o[2] = fewest[1];
+  }
 }
 
-// The outputs of marked rows, in fp32: a 32 x 32 tile that meets a marked row of A
-// or B is computed again from the fp32 operands (any strides) on the fp32
-// matrix cores, and its outputs in those rows and columns are stored: an output
-// depends on its own two rows alone.  Few rows are marked, and then only their
+// The outputs that the planes do not give (hard rows; lossy rows against rows with too few near
+// values), in fp32: a 32 x 32 tile that has one is computed again from the fp32 operands
+// (any strides) on the fp32 matrix cores, and those outputs are stored: an output
+// depends on its own two rows alone.  There are few such rows, and then only their
 // strip of tiles is there to do, so the eight wavefronts of a workgroup share a
 // tile, each taking every eighth 32 k of it straight into registers (the next
 // step's while one is multiplied, no barrier), and their sums are added in
 // wavefront order; a step whose part of A is all zeros (positions without a
-// loss, in a weight gradient) is skipped.  Without a marked row a workgroup
-// reads the marks of its tiles and ends (5 us).  One marked row: d_emb of 2,560
+// loss, in a weight gradient) is skipped.  Without such a row a workgroup
+// reads the marks of its tiles and ends (5 us).  One hard row: d_emb of 2,560
 // columns and K 12,800 121 us, bound by its 80 tiles' loads and the fp32 matrix
 // cores of 80 CUs; 12,800 columns, K 2,560 57 us (64 x 64 tiles through LDS 200
-// and 108 us; 4 and 16 wavefronts 148 and 128 us).  Every row marked, 12,800 x
+// and 108 us; 4 and 16 wavefronts 148 and 128 us).  Every row, 12,800 x
 // 2,560 outputs, K 1,531: 1.7 ms, bound by the 12.5 GB its tiles read from L2
 // (1.3 ms on 64 x 64 tiles, 5.8 ms on the vector units).
-constexpr int kWideGroups = 509;  // two workgroups a CU, and prime, so that a marked row's
-                                  // strip of tiles and a marked column's go over all of them
+constexpr int kWideGroups = 509;  // two workgroups a CU, and prime, so that a row's strip of
+                                  // tiles and a column's go over all of them
 constexpr int kWideWaves = 8;
 
 struct WideArgs {
   F16Src a[2], b[2][2];    // sources of A and of B per column group
-  const int32_t* wide[3];  // marks of A, B, B2
+  const int32_t* info[3][2];  // of A, B, B2
+  const int32_t* sum8[3];
+  int near[2];             // near values of two rows together from which their output stays, per source
   int n_src;
   int64_t m, n[2];
   float* c[2];
@@ -1327,23 +1389,36 @@ struct WideArgs {
 __global__ __launch_bounds__(64 * kWideWaves, 4) void gemm_wide_kernel(const WideArgs g) {
   constexpr int NT = 64 * kWideWaves;
   __shared__ float s_part[kWideWaves][16][64];
-  __shared__ int s_tile[NT], s_mark[2][4];
+  __shared__ int s_tile[NT], s_info[2][2][32];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5;
   const int64_t tm_n = (g.m + 31) / 32, tn0 = (g.n[0] + 31) / 32, tn_n = tn0 + (g.n[1] + 31) / 32;
   const int64_t pitch = tn_n % kWideGroups == 0 ? tn_n + 1 : tn_n, tiles = tm_n * pitch;
-  auto row_marks = [&](int64_t tm, int q) { return 32 * tm + 8 * q < g.m ? g.wide[0][4 * tm + q] : 0; };
-  auto col_marks = [&](int64_t tn, int q) {
-    const int grp = tn < tn0 ? 0 : 1;
-    const int64_t t = grp ? tn - tn0 : tn;
-    return 32 * t + 8 * q < g.n[grp] ? g.wide[1 + grp][4 * t + q] : 0;
+  // of an output's row and column, or of a tile's two sides: their marks, and near values together
+  auto needed = [&](int hard, int lossy0, int lossy1, int n0, int n1) {
+    return hard != 0 || (lossy0 != 0 && n0 < g.near[0]) || (lossy1 != 0 && n1 < g.near[1]);
   };
-  // NT of the workgroup's tiles at a time: the marked ones, in order
+  // of the 32 rows of a side's tile: their marks, and the fewest near values
+  auto side = [&](int x, int64_t t, int64_t rows, int* n) {
+    int mark = 0;
+    n[0] = n[1] = kNear;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int32_t* o = g.sum8[x] + 3 * (4 * t + q);
+      if (32 * t + 8 * q < rows) mark |= o[0], n[0] = min(n[0], o[1]), n[1] = min(n[1], o[2]);
+    }
+    return mark;
+  };
+  // NT of the workgroup's tiles at a time: those with outputs to compute, in order
   for (int64_t base = blockIdx.x; base < tiles; base += (int64_t)kWideGroups * NT) {
     const int64_t mine = base + (int64_t)kWideGroups * tid;
     int mark = 0;
-    if (mine < tiles && mine % pitch < tn_n)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) mark |= row_marks(mine / pitch, q) | col_marks(mine % pitch, q);
+    if (mine < tiles && mine % pitch < tn_n) {
+      const int64_t tn = mine % pitch;
+      const int grp = tn < tn0 ? 0 : 1;
+      int na[2], nb[2];
+      const int both = side(0, mine / pitch, g.m, na) | side(1 + grp, grp ? tn - tn0 : tn, g.n[grp], nb);
+      mark = needed(both & 0xff, both >> 8 & 0xff, both >> 16 & 0xff, na[0] + nb[0], na[1] + nb[1]);
+    }
     if (!__syncthreads_or(mark)) continue;
     s_tile[tid] = mark != 0;
     __syncthreads();
@@ -1352,7 +1427,10 @@ __global__ __launch_bounds__(64 * kWideWaves, 4) void gemm_wide_kernel(const Wid
       const int64_t tile = base + kWideGroups * i, tm = tile / pitch, tn = tile % pitch;
       const int grp = tn < tn0 ? 0 : 1;
       const int64_t m0 = 32 * tm, n0 = 32 * (grp ? tn - tn0 : tn), n_grp = g.n[grp];
-      if (tid < 8) s_mark[tid >> 2][tid & 3] = tid < 4 ? row_marks(tm, tid) : col_marks(tn, tid - 4);
+      if (tid < 128) {  // rows past the end take the last one's: not stored
+        const int x = tid >> 6 ? 1 + grp : 0, s = tid >> 5 & 1;
+        s_info[tid >> 6][s][tid & 31] = g.info[x][s][min((x ? n0 : m0) + (tid & 31), (x ? n_grp : g.m) - 1)];
+      }
       f32x16 acc;
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
@@ -1420,7 +1498,9 @@ __global__ __launch_bounds__(64 * kWideWaves, 4) void gemm_wide_kernel(const Wid
         float v = s_part[0][r][lane];
 #pragma unroll
         for (int w = 1; w < kWideWaves; ++w) v += s_part[w][r][lane];
-        const bool marked = ((s_mark[0][lr >> 3] >> (lr & 7)) | (s_mark[1][lc >> 3] >> (lc & 7))) & 1;
+        const int a0 = s_info[0][0][lr], a1 = s_info[0][1][lr], b0 = s_info[1][0][lc], b1 = s_info[1][1][lc];
+        const bool marked = needed((a0 | b0) & kHard, (a0 | b0) & kLossy, (a1 | b1) & kLossy,
+                                   (a0 & kNear) + (b0 & kNear), (a1 & kNear) + (b1 & kNear));
         if (marked && m0 + lr < g.m && n0 + lc < n_grp) g.c[grp][(m0 + lr) * g.ldc[grp] + n0 + lc] = v;
       }
       __syncthreads();  // the sums and marks are read
@@ -2005,9 +2085,11 @@ F16Src f16_src(const eg_f16_matrix* x, int s) {
 
 int64_t blocks32(int64_t rows) { return (rows + 31) / 32; }
 
-// exps holds the rows' exponents of source 0, those of source 1, and the marks.
+// exps holds the rows' exponents of source 0, those of source 1, the rows' info of
+// either, and the summaries of 8 rows.
 int32_t* f16_exps(const eg_f16_matrix* x, int s) { return x->exps + blocks32(x->rows) * 32 * s; }
-int32_t* f16_marks(const eg_f16_matrix* x) { return x->exps + blocks32(x->rows) * 64; }
+int32_t* f16_info(const eg_f16_matrix* x, int s) { return x->exps + blocks32(x->rows) * 32 * (2 + s); }
+int32_t* f16_sum8(const eg_f16_matrix* x) { return x->exps + blocks32(x->rows) * 128; }
 }  // namespace
 }  // namespace eg
 
@@ -2015,7 +2097,7 @@ extern "C" {
 
 int64_t eg_f16_planes_bytes(int64_t rows, int64_t k) { return rows < 0 || k < 0 ? -1 : eg::blocks32(rows) * ((k + 31) / 32) * eg::kStepBytes; }
 
-int64_t eg_f16_exps_count(int64_t rows) { return rows < 0 ? -1 : eg::blocks32(rows) * 68; }
+int64_t eg_f16_exps_count(int64_t rows) { return rows < 0 ? -1 : eg::blocks32(rows) * 140; }
 
 int eg_split_f16(const eg_f16_matrix* x, void* stream) {
   using namespace eg;
@@ -2035,7 +2117,9 @@ int eg_split_f16(const eg_f16_matrix* x, void* stream) {
   a.planes = (char*)x->planes;
   a.exps[0] = f16_exps(x, 0);
   a.exps[1] = f16_exps(x, 1);
-  a.wide = f16_marks(x);
+  a.info[0] = f16_info(x, 0);
+  a.info[1] = f16_info(x, 1);
+  a.sum8 = f16_sum8(x);
   const int64_t blocks = trans ? blocks32(x->rows) : 4 * blocks32(x->rows);
   EG_CHECK_ARG(blocks < (1LL << 31), "too many rows");
   const int64_t chunks = 4 * steps;
@@ -2104,9 +2188,16 @@ int eg_gemm_f16x3(const eg_f16_matrix* a, const eg_f16_matrix* b, const eg_f16_m
     w.b[1][s] = f16_src(second, s);
   }
   w.n_src = a->n_src;
-  w.wide[0] = f16_marks(a);
-  w.wide[1] = f16_marks(b);
-  w.wide[2] = b2 != nullptr ? f16_marks(b2) : nullptr;
+  const eg_f16_matrix* of[3] = {a, b, second};
+  for (int x = 0; x < (b2 != nullptr ? 3 : 2); ++x) {
+    w.info[x][0] = f16_info(of[x], 0);
+    w.info[x][1] = f16_info(of[x], 1);
+    w.sum8[x] = f16_sum8(of[x]);
+  }
+  for (int s = 0; s < 2; ++s) {
+    const int64_t k = w.a[s].cols;
+    w.near[s] = (int)std::min<int64_t>(k + (k + kNearShare - 1) / kNearShare, INT32_MAX);
+  }
   w.m = m;
   w.n[0] = n;
   w.n[1] = n2;

@@ -373,8 +373,8 @@ def gemm_h3(a: tuple, b: tuple, b_n2: tuple | None = None, *, planes_b: HalfPlan
     """``sum_s a[s] @ b[s].T`` over one or two pairs of fp32 matrices (any
     strides) with an fp32 matmul's accuracy on the fp16 matrix cores
     (``eg_gemm_f16x3``: every row scaled by a power of two and split into two
-    fp16 planes, three products accumulated in fp32; rows beyond the planes'
-    range computed in fp32).  ``b_n2``: a second column group over the same
+    fp16 planes, three products accumulated in fp32; outputs for which it counts
+    what their rows' planes lose are computed in fp32).  ``b_n2``: a second column group over the same
     ``a``; the result is then a pair.  ``planes_b`` / ``planes_b2``: the planes
     of ``b`` / ``b_n2`` where the caller keeps them.  Operands of another dtype are
     converted, as :func:`gemm_f32`'s."""
@@ -483,7 +483,11 @@ def gemm_f32(a, b, a2=None, b2=None, out: torch.Tensor | None = None, accumulate
 # launches.  The forward of a call that is differentiated keeps gemm_x6: the
 # score's gradient goes as 1/sqrt|s|, so at a score near zero any other rounding
 # of the key moves the hidden, key and norm gradients by far more than its own
-# size (1e-4 at |s| 0.03).
+# size (1e-4 at |s| 0.03).  "Differentiated" is any input with requires_grad, under
+# no_grad too: the first pass of a re-entrant checkpoint runs so, and its output has to
+# be the recomputation's bit for bit.  Past H3_MIN_ROWS positions the outputs of a call with
+# and of one without such inputs therefore differ in their rounding, and evaluating a
+# block whose weights are being trained takes gemm_x6 unless it is given detached weights.
 H3_MIN_ROWS = 64
 
 # Up to this many positions every gemm= runs eg_gemm_f32_rows: reading the weights
@@ -769,8 +773,9 @@ class _PleFn(torch.autograd.Function):
             if parts:  # none: both factors detached, emb has no path to the output
                 d_emb = _projection_backward(ctx.gemm, parts).to(emb_dt)
         wdt = ctx.w_dtypes
-        # the projection weights' gradients d_key^T emb and d_value^T emb on eg_gemm_f32
-        # (K = the positions); a weight the detached factor cuts off keeps None
+        # the projection weights' gradients d_key^T emb and d_value^T emb (K = the positions); a
+        # weight the detached factor cuts off keeps None.  Side by side they are views of one
+        # buffer: either gradient keeps the other's memory
         if both:
             d_w = _weight_grad(d_kv, emb32, None, ctx.gemm)
             d_wk, d_wv = d_w[:c_dim].to(wdt[0]), d_w[c_dim:].to(wdt[1])
@@ -813,12 +818,14 @@ def ple_forward(emb: torch.Tensor, hidden: torch.Tensor, w: PleWeights, hist: to
     ``[rows, hc, n_embd]`` (at most ``(K-1)*ple_ngram_size`` rows, empty at a
     sequence start); all on the device.  ``gemm`` picks the projections' GEMM:
     ``"bf16x6"``, the default (``gemm_x6`` or, past ``H3_MIN_ROWS`` positions of a
-    call without gradients and in the backward, ``gemm_h3``: the 16-bit matrix
-    cores with fp32 accuracy, both errors against float64 below the fp32
-    path's, and the fastest at that accuracy), ``"fp32"`` (``gemm_f32``: fp32
+    call none of whose inputs requires gradients and in the backward, and for the
+    weights' gradients, ``gemm_h3``: the 16-bit matrix cores with fp32 accuracy,
+    both errors against float64 below the fp32 path's, and the fastest at that
+    accuracy), ``"fp32"`` (``gemm_f32``: fp32
     products on the fp32 matrix cores, the reference's torch matmul
     arithmetic) or ``"bf16x3"`` (``gemm_x3``: 16 mantissa bits per operand,
-    about 1e-5 relative per projection)."""
+    about 1e-5 relative per projection).  Up to ``FEW_ROWS`` positions every
+    choice runs ``eg_gemm_f32_rows``."""
     if gemm not in ("fp32", "bf16x3", "bf16x6"):
         raise ValueError(f"gemm must be 'fp32', 'bf16x3' or 'bf16x6', got {gemm!r}")
     hc = hparams.hc_mult

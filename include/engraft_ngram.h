@@ -677,21 +677,23 @@ int64_t eg_f16_exps_count(int64_t rows);
 
 /* Fills x's planes and exps: each source's part of a row scaled by a power of
  * two (its largest magnitude to [2^14, 2^15), the exponent kept in exps) and
- * split into fp16 planes hi = rne(x) and lo = rne(x - hi).  A row is marked when
- * a source's largest magnitude there is not finite or below 2^-87, when its two
- * sources' are more than 2^36 apart, or when more than 1/16 of its nonzero values
- * are below 2^-18 of the largest of their source's part or more than 1/256 below
- * 2^-24 of it.  No counterpart in the reference (part of its fp32 matmuls). */
+ * split into fp16 planes hi = rne(x) and lo = rne(x - hi).  A row is hard when a
+ * source's largest magnitude there is not finite or below 2^-87, or when its two
+ * sources' are more than 2^36 apart.  It is lossy in a source when the octaves that
+ * its values there lie below 2^-18 of its largest, and eight times those below 2^-24,
+ * come to more than 12/128 of an octave per nonzero value.  exps also keeps these marks and the
+ * number of values near each largest (within 2^-6 of it).  No counterpart in the
+ * reference (part of its fp32 matmuls). */
 int eg_split_f16(const eg_f16_matrix* x, void* stream);
 
 /* C [m, n] = A B^T and, with b2, C2 [m, n2] = A B2^T (m, n, n2 the operands'
  * rows) on the fp16 matrix cores: hi*hi + hi*lo + lo*hi of the operands'
- * eg_split_f16 planes accumulated in fp32; the outputs of marked rows in fp32
- * from the sources.  The others differ from A B^T by the fp32 sums' rounding and,
- * per source, at most 3 2^-22 |a| |b| + 2^-40 (max|a| sum|b| + sum|a| max|b|)
- * over the two rows: below an fp32 matmul's own error in the rows' norms.  Only
- * an output far below its rows' norms, where few small values of one row meet
- * the few values of the other that are not near zero, keeps less than there.
+ * eg_split_f16 planes accumulated in fp32; in fp32 from the sources the outputs
+ * of hard rows and, where a row is lossy in a source of k columns, those whose two
+ * rows have fewer than k + k / 16 near values there together.  The others differ
+ * from A B^T by the fp32 sums' rounding and, per source, at most 3 2^-22 sum |a b|
+ * and 2^-39 (max|a| sum|b| + sum|a| max|b|) over the two rows; where either is lossy
+ * the latter is below 2^-21 sum |a b|.
  * a and b with the same sources' cols, at least one column.  Workspace of
  * eg_gemm_workspace_size(m, n, n2, k, 0) bytes, k the sum of the padded cols.
  * ple_forward's projections and their gradients past a few rows

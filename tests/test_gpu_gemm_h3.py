@@ -4,9 +4,9 @@ matrix cores) against float64 products of the same fp32 operands.
 Bar: |C - C64| <= ((k + 2) 2^-24 + 3 2^-22) (|A| |B|^T): an fp32 sum of k
 products in any order, plus what the split drops of each product (lo*lo and
 the two lo planes' rounding, 2^-22 each at most).  Rows spread over less than
-2^18 are within the planes' 22 bits everywhere; marked rows (most values 2^24
-below the largest, tiny, infinite, NaN) are computed in fp32 and held to the
-same bar."""
+2^18 are within the planes' 22 bits everywhere; marked rows (a share of the values far
+below the largest, tiny, infinite, NaN) are computed in fp32, where the other row
+does not make up for it, and held to the same bar."""
 from __future__ import annotations
 
 import sys
@@ -251,3 +251,45 @@ def test_gemm_h3_converts_other_dtypes(cuda):
     a, b = (torch.randn((r, 70), generator=g, device=cuda).bfloat16() for r in (40, 33))
     exp = gemm_h3((a.float(),), (b.float(),))
     assert torch.equal(gemm_h3((a,), (b.double(),)), exp)
+
+
+@pytest.mark.parametrize("ks", [(1024,), (512, 160), (2624,), (96,)])
+@pytest.mark.parametrize("p", [15, 22, 30, 60])
+def test_gemm_h3_rows_small_outside_a_part(cuda, ks, p):
+    """Rows of which a quarter is 2^p above the rest (a stream with a steep gradient): what their
+    planes lose counts for columns that are small there, alone.  Those are computed in fp32; the
+    columns that are not keep the planes' bits (those of the rows without what is lost: at
+    p 60 nothing is left of it).  At the rule's line too: of K / 4 large values, K / 16 of a column's
+    are large as well, or one fewer."""
+    from engraft_ngram_amd.ple import gemm_h3
+    _say(f"gemm_h3 rows small outside a part k={ks} p={p}")
+    g = torch.Generator(device=cuda).manual_seed(sum(ks) + p)
+    m, n = 70, 96
+
+    def near(*shape):  # within 2^-6 of the largest, which is below 2: all of them near
+        x = torch.rand(shape, generator=g, device=cuda) * 1.9 - 0.95
+        return x + 0.05 * x.sign()
+    a, b, a0 = [], [], []
+    for k in ks:
+        x, y = near(m, k), near(n, k)
+        q = k // 4
+        x[:, q:] *= 2.0 ** -p
+        x[:35, 0], y[:, 0] = 1.0, 1.0  # the largest of each row in the part
+        y[0::4, :q] = 0.0                     # nothing of the part
+        y[1::4, (k + 15) // 16:q] = 0.0        # exactly enough of it
+        y[2::4, (k + 15) // 16 - 1:q] = 0.0     # one too few
+        x[40] = 0.0                           # a row of zeros
+        a.append(x), b.append(y)
+        a0.append(torch.where(torch.arange(k, device=cuda) < q, x, 0.0))
+    k = sum(ks)
+    exp = sum(x.double() @ y.double().T for x, y in zip(a, b))
+    for flip in (False, True):
+        got = gemm_h3(tuple(b), tuple(a)).T if flip else gemm_h3(tuple(a), tuple(b))
+        without = gemm_h3(tuple(b), tuple(a0)).T if flip else gemm_h3(tuple(a0), tuple(b))
+        for c in range(4):
+            assert _rel(got[:, c::4], exp[:, c::4]) <= _sums_bar(k), (c, flip)
+        assert not got[40].any()
+        if p == 60:
+            for c in (1, 3):
+                assert torch.equal(got[:, c::4], without[:, c::4]), (c, flip)
+            assert _rel(got[:, 0::4], exp[:, 0::4]) <= _sums_bar(k) and not without[:, 0::4].any()
