@@ -924,8 +924,9 @@ __global__ __launch_bounds__(256) void gemm_f32_vec_kernel(const F32Args args) {
 // way, so both keep all their bits (with one exponent a row, sources 2^24 apart
 // left an error of 4e-5).  A tile (or its part of K) that began in source 0 is
 // multiplied by the powers of two that lead to source 1's units when it leaves
-// it, in the accumulators; kApart bounds them.  d_emb of 1,531 positions, K
-// 10,240 + 2,560: 272 us, 15 us of them the second source's own start and the units.
+// it, in the accumulators, between two steps of the pipeline; kApart bounds them.
+// d_emb of 1,531 positions, K 10,240 + 2,560: 247 us (257 us with the pipeline started
+// again for source 1).
 struct H3Seg {
   const char* a;
   const char* b[2];       // per column group
@@ -961,6 +962,8 @@ __device__ inline void h3_tile(const H3Args& args, const Work& w, char* lds) {
   const int wm = uwave / WNW, wn = uwave % WNW;
   const H3Seg& sg = args.seg[0];
 
+  int* diff = (int*)(lds + 2 * STAGE);  // two sources: the powers between them, of rows and columns
+
   f32x16 acc[TI][TJ];
 #pragma unroll
   for (int i = 0; i < TI; ++i)
@@ -969,9 +972,11 @@ __device__ inline void h3_tile(const H3Args& args, const Work& w, char* lds) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-  // K steps [lo, hi), of one source
-  auto steps = [&](int64_t lo, int64_t hi) {
-    if (lo >= hi) return;
+  const int64_t lo = w.kv0, hi = w.kv1;
+  // two sources: the step before which the sums so far go into source 1's units
+  // (past the last one where the tile's part ends in source 0), if it began in source 0
+  const int64_t mid = TWO && lo < args.kt_first ? min(args.kt_first, hi) : -1;
+  if (lo < hi) {
     // this wavefront's loads: blocks uwave LB .. + LB - 1 of the stage (A's, then
     // B's), four 1 KB pieces each.  Blocks past the last re-read the last: their
     // products only reach outputs that are not stored.
@@ -1027,7 +1032,42 @@ __device__ inline void h3_tile(const H3Args& args, const Work& w, char* lds) {
 #pragma unroll
         for (int j = 0; j < TJ; ++j) one(f, pass, i, j);
     };
+    // the sums into source 1's units: times the rows' and columns' powers
+    auto into_second = [&] {
+      int lane_o = lane;  // opaque: addresses hoisted out of the walk's loop spill
+      asm volatile("" : "+v"(lane_o));
+      int sb[TJ];
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) sb[j] = diff[BM + (wn * TJ + j) * 32 + (lane_o & 31)];
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          __builtin_amdgcn_sched_barrier(0);
+          const int4 sa = *(const int4*)(diff + (wm * TI + i) * 32 + 8 * q + 4 * (lane_o >> 5));
+          const int sr[4] = {sa.x, sa.y, sa.z, sa.w};
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) acc[i][j][4 * q + r] = ldexpf(acc[i][j][4 * q + r], sr[r] + sb[j]);
+        }
+      // the powers are read before the barrier that lets the next tile's in
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+    };
     issue(lo);
+    if (TWO && mid > 0) {  // rows past m or n take the last one's: not stored
+      const int e = (int)threadIdx.x;
+      static_assert(NW * 64 == BM + BN, "a row or a column a thread");
+      if (e < BM) {
+        const int64_t row = min(w.m0 + e, p.m - 1);
+        diff[e] = args.first.a[row] - args.scale.a[row];
+      } else {
+        const int64_t col = min(w.n0 + e - BM, p.n[w.grp] - 1);
+        diff[e] = args.first.b[w.grp][col] - args.scale.b[w.grp][col];
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // in LDS for the others after the barrier below
+    }
     if (lo + 1 < hi) {
       issue(lo + 1);
       wait_vm<LPW>();  // this wavefront's part of the first step is in LDS
@@ -1037,6 +1077,7 @@ __device__ inline void h3_tile(const H3Args& args, const Work& w, char* lds) {
     __builtin_amdgcn_s_barrier();
     read(0, lo, 0);
     for (int64_t kt = lo; kt + 1 < hi; ++kt) {
+      if (TWO && kt == mid) into_second();
       mfma(0, 0);
       __builtin_amdgcn_sched_barrier(0);  // the reads stay between the passes
       read(1, kt, 1);
@@ -1064,53 +1105,15 @@ __device__ inline void h3_tile(const H3Args& args, const Work& w, char* lds) {
         }
       }
     }
+    if (TWO && mid == hi - 1) into_second();
     mfma(0, 0);
     read(1, hi - 1, 1);
     mfma(0, 1);
     mfma(0, 2);
 #pragma unroll
     for (int pass = 0; pass < 3; ++pass) mfma(1, pass);
-    __builtin_amdgcn_s_barrier();  // the ring is refilled by the next tile
-  };
-  if constexpr (TWO) {
-    const int64_t mid = min(max(w.kv0, args.kt_first), w.kv1);
-    steps(w.kv0, mid);
-    if (w.kv0 < mid) {
-      // into source 1's units, the rows' and columns' powers through the ring
-      // (free between two turns); rows past m or n take the last one's: not stored
-      int* diff = (int*)lds;
-      static_assert(NW * 64 == BM + BN, "a row or a column a thread");
-      const int e = (int)threadIdx.x;
-      if (e < BM) {
-        const int64_t row = min(w.m0 + e, p.m - 1);
-        diff[e] = args.first.a[row] - args.scale.a[row];
-      } else {
-        const int64_t col = min(w.n0 + e - BM, p.n[w.grp] - 1);
-        diff[e] = args.first.b[w.grp][col] - args.scale.b[w.grp][col];
-      }
-      __syncthreads();
-      int lane_o = lane;  // opaque: addresses hoisted out of the walk's loop spill
-      asm volatile("" : "+v"(lane_o));
-      int sb[TJ];
-#pragma unroll
-      for (int j = 0; j < TJ; ++j) sb[j] = diff[BM + (wn * TJ + j) * 32 + (lane_o & 31)];
-#pragma unroll
-      for (int i = 0; i < TI; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          __builtin_amdgcn_sched_barrier(0);
-          const int4 sa = *(const int4*)(diff + (wm * TI + i) * 32 + 8 * q + 4 * (lane_o >> 5));
-          const int sr[4] = {sa.x, sa.y, sa.z, sa.w};
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int j = 0; j < TJ; ++j) acc[i][j][4 * q + r] = ldexpf(acc[i][j][4 * q + r], sr[r] + sb[j]);
-        }
-      __syncthreads();
-    }
-    steps(mid, w.kv1);
-  } else {
-    steps(w.kv0, w.kv1);
+    if (TWO && mid == hi) into_second();
+    __builtin_amdgcn_s_barrier();  // the ring (and powers) are refilled by the next tile
   }
   store_acc<BM, BN, TI, TJ>(p, w, acc, wm, wn, lane, args.scale);
 }
@@ -1636,6 +1639,7 @@ struct Shape {
 
 constexpr Shape kX3Shape{kX3BM, kX3BN, kX3WM * kX3WN * 64, 1, (size_t)kStages * 2 * (kX3BM + kX3BN) * kBK * 2, 4.2,
                          true};
+constexpr Shape kH3TwoShape{kX3BM, kX3BN, kX3WM * kX3WN * 64, 1, kX3Shape.lds + (kX3BM + kX3BN) * 4, 4.2, true};
 constexpr int kF32BM = 256, kF32BN = 256;
 constexpr Shape kF32Shape{kF32BM, kF32BN, kF32BM * kF32BN / 64, 1,
                           (size_t)kStages * (kF32BM + kF32BN) * kBK * 4, 1.6, true};
@@ -2175,7 +2179,7 @@ int eg_gemm_f16x3(const eg_f16_matrix* a, const eg_f16_matrix* b, const eg_f16_m
   g.kt_first = last > 0 ? (a->src[0].cols + 31) / 32 : ka;
   EG_CHECK_ARG(ka > 0, "k must be positive");
   const bool two = g.kt_first > 0 && g.kt_first < ka;
-  rc = launch_gemm<kX3BM, kX3BN>(kX3Shape,
+  rc = launch_gemm<kX3BM, kX3BN>(two ? kH3TwoShape : kX3Shape,
                                  two ? gemm_h3_kernel<kX3BM, kX3BN, kX3WM, kX3WN, true>
                                      : gemm_h3_kernel<kX3BM, kX3BN, kX3WM, kX3WN, false>,
                                  "gemm_h3_kernel", g, m, n, n2, c, ldc, c2, ldc2, 0, 0, workspace, workspace_bytes,

@@ -293,3 +293,19 @@ def test_gemm_h3_rows_small_outside_a_part(cuda, ks, p):
             for c in (1, 3):
                 assert torch.equal(got[:, c::4], without[:, c::4]), (c, flip)
             assert _rel(got[:, 0::4], exp[:, 0::4]) <= _sums_bar(k) and not without[:, 0::4].any()
+
+
+@pytest.mark.parametrize("steps", [9, 32])
+def test_gemm_h3_second_source_from_every_step_on(cuda, steps):
+    """A tile's K is cut into ranges; the second source begins at every step of them (the first,
+    inside, the last, past the last), 2^24 from the first in size."""
+    from engraft_ngram_amd.ple import gemm_h3
+    _say(f"gemm_h3 second source from every of {steps} steps")
+    g = torch.Generator(device=cuda).manual_seed(steps)
+    m, n, k = 70, 260, 32 * steps
+    a, b = (torch.randn((r, k), generator=g, device=cuda) for r in (m, n))
+    for q in range(32, k, 32):
+        x, y = (a[:, :q] * 2.0 ** -24, a[:, q:]), (b[:, :q] * 2.0 ** 24, b[:, q:])
+        got = gemm_h3(x, y)
+        exp = a.double() @ b.double().T
+        assert _rel(got, exp) <= 3 * 2.0 ** -22 + (3 * k / 16) ** 0.5 * 2.0 ** -24, q
