@@ -1152,9 +1152,9 @@ struct SplitF16Args {
 // lossy, since random rows have some near zero.
 // What a lossy row loses counts where the other row is small at its large
 // values and only there: an output of it is computed in fp32 unless enough products are
-// of two near values, of 2^-6 of their rows' largest at least.  Of K products n_a +
+// of two near values, of 2^-7 of their rows' largest at least.  Of K products n_a +
 // n_b - K are, n the near values of either row; from K / 16 on sum |a b| is
-// at least K 2^-16 of the largest's product and the loss at most 2^-38 K of it, 2^-22
+// at least K 2^-18 of the largest's product and the loss at most 2^-38 K of it, 2^-20
 // of sum |a b|.  (A position where one stream's score is near zero is lossy in the
 // key's gradient; its near values are that stream's, and no weight is small at
 // all of them.  Computing such rows again, one or two of 1,531, cost the block's
@@ -1274,7 +1274,7 @@ __global__ __launch_bounds__(64 * NW) void split_f16_kernel(const SplitF16Args a
     const int s = c < a.chunks[0] ? 0 : 1;
     const float sc = s ? scale[1] : scale[0];
     const uint16_t t18 = (uint16_t)(((s ? mxs[1] : mxs[0]) >> 16) - 18 * 128);  // above 24 octaves' unless out or zero
-    const u16x2 v18 = t18, v24 = (uint16_t)(t18 - 6 * 128), v6 = (uint16_t)(t18 + 12 * 128 - 1);
+    const u16x2 v18 = t18, v24 = (uint16_t)(t18 - 6 * 128), v7 = (uint16_t)(t18 + 11 * 128 - 1);
     uint32_t seen = 0, lost = 0, pair = 0;  // seen: nonzero + 256 near
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -1286,7 +1286,7 @@ __global__ __launch_bounds__(64 * NW) void split_f16_kernel(const SplitF16Args a
         lost = __builtin_amdgcn_udot2(__builtin_elementwise_sub_sat(v18, z), one, lost, false);
         lost = __builtin_amdgcn_udot2(__builtin_elementwise_sub_sat(v24, z), (u16x2)8, lost, false);
         seen = __builtin_amdgcn_udot2(__builtin_elementwise_min(h, one), one, seen, false);
-        seen = __builtin_amdgcn_udot2(__builtin_elementwise_min(__builtin_elementwise_sub_sat(h, v6), one),
+        seen = __builtin_amdgcn_udot2(__builtin_elementwise_min(__builtin_elementwise_sub_sat(h, v7), one),
                                       (u16x2)256, seen, false);
       }
       pair = __float_as_uint(y);

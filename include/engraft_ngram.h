@@ -682,7 +682,7 @@ int64_t eg_f16_exps_count(int64_t rows);
  * sources' are more than 2^36 apart.  It is lossy in a source when the octaves that
  * its values there lie below 2^-18 of its largest, and eight times those below 2^-24,
  * come to more than 12/128 of an octave per nonzero value.  exps also keeps these marks and the
- * number of values near each largest (within 2^-6 of it).  No counterpart in the
+ * number of values near each largest (within 2^-7 of it).  No counterpart in the
  * reference (part of its fp32 matmuls). */
 int eg_split_f16(const eg_f16_matrix* x, void* stream);
 
@@ -693,7 +693,7 @@ int eg_split_f16(const eg_f16_matrix* x, void* stream);
  * rows have fewer than k + k / 16 near values there together.  The others differ
  * from A B^T by the fp32 sums' rounding and, per source, at most 3 2^-22 sum |a b|
  * and 2^-39 (max|a| sum|b| + sum|a| max|b|) over the two rows; where either is lossy
- * the latter is below 2^-21 sum |a b|.
+ * the latter is below 2^-19 sum |a b|.
  * a and b with the same sources' cols, at least one column.  Workspace of
  * eg_gemm_workspace_size(m, n, n2, k, 0) bytes, k the sum of the padded cols.
  * ple_forward's projections and their gradients past a few rows
