@@ -131,27 +131,31 @@ class _WeightCache:
     def get(self, ws: tuple, make, form=None):
         """``make()``, or what it made for the same weights and ``form``."""
         dev = ws[0].device
-        if dev.index is None or dev.index == torch.cuda.current_device():
+        if dev.index == torch.cuda.current_device():
             capturing = torch.cuda.is_current_stream_capturing()
         else:
             with torch.cuda.device(dev):
                 capturing = torch.cuda.is_current_stream_capturing()
         if capturing:
             return make()
-        key = (form, _lib.stream_ptr(dev), *((w.data_ptr(), w.shape, w.stride()) for w in ws))
-        versions = [w._version for w in ws]
-        for refs, v, k, made in self._entries:
-            if k == key and v == versions and all(r() is w for r, w in zip(refs, ws)):
-                return made
-
-        def current(refs, v):
-            alive = [r() for r in refs]
-            return all(w is not None and w._version == n for w, n in zip(alive, v))
-
-        self._entries = [e for e in self._entries if current(e[0], e[1])][1 - self._size:]
+        key = (form, _lib.stream_ptr(dev), len(ws))
+        for of, k, made in self._entries:
+            if k == key:
+                for w, (ref, place) in zip(ws, of):
+                    if ref() is not w or place != (w._version, w.data_ptr(), w.shape, w.stride()):
+                        break
+                else:
+                    return made
+        self._entries = [e for e in self._entries if self._current(e[0])][1 - self._size:]
         made = make()
-        self._entries.append(([weakref.ref(w) for w in ws], versions, key, made))
+        self._entries.append((tuple((weakref.ref(w), (w._version, w.data_ptr(), w.shape, w.stride())) for w in ws),
+                              key, made))
         return made
+
+    @staticmethod
+    def _current(of) -> bool:
+        alive = [(ref(), place[0]) for ref, place in of]
+        return all(w is not None and w._version == version for w, version in alive)
 
 
 _WT = _WeightCache(4)
@@ -340,11 +344,14 @@ class HalfPlanes:
     the GEMM reads too; the planes do not keep them."""
 
     def __init__(self, of: tuple):
-        if len(of) not in (1, 2) or any(x.dim() != 2 or x.dtype != torch.float32 for x in of):
+        if len(of) not in (1, 2):
             raise ValueError("HalfPlanes: one or two fp32 matrices expected")
-        if any(x.shape[0] != of[0].shape[0] or x.device != of[0].device for x in of):
-            raise ValueError(f"HalfPlanes: two matrices of the same rows on one device expected, got "
-                             f"{[tuple(x.shape) for x in of]}")
+        for x in of:
+            if x.dim() != 2 or x.dtype != torch.float32:
+                raise ValueError("HalfPlanes: one or two fp32 matrices expected")
+            if x.shape[0] != of[0].shape[0] or x.device != of[0].device:
+                raise ValueError(f"HalfPlanes: two matrices of the same rows on one device expected, got "
+                                 f"{[tuple(x.shape) for x in of]}")
         lib = _lib.load()
         self.shapes = tuple(tuple(x.shape) for x in of)
         self.rows = of[0].shape[0]
@@ -391,6 +398,13 @@ def gemm_h3(a: tuple, b: tuple, b_n2: tuple | None = None, *, planes_b: HalfPlan
         if planes is not None and (planes.shapes != tuple(tuple(x.shape) for x in side) or
                                    planes.planes.device != a[0].device):
             raise ValueError(f"gemm_h3: the planes given are not those of {name}: {planes.shapes}")
+    return _gemm_h3(a, b, b_n2, planes_b, planes_b2)
+
+
+def _gemm_h3(a: tuple, b: tuple, b_n2: tuple | None = None, planes_b: HalfPlanes | None = None,
+             planes_b2: HalfPlanes | None = None):
+    """:func:`gemm_h3` of operands that are known to fit, as the block's own are (its checks
+    took 10 us of a short call's host time)."""
     pa = HalfPlanes(a)
     pb = planes_b if planes_b is not None else HalfPlanes(b)
     pb2 = None if b_n2 is None else planes_b2 if planes_b2 is not None else HalfPlanes(b_n2)
@@ -516,7 +530,7 @@ def _weight_grad(d_y: torch.Tensor, x: torch.Tensor, w: torch.Tensor, gemm: str 
     if d_y.shape[0] == 0:
         return torch.zeros_like(w)
     if gemm == "bf16x6":
-        return gemm_h3((d_y.T,), (x.T,))
+        return _gemm_h3((d_y.T,), (x.T,))
     return gemm_f32(d_y.T, x.T)
 
 
@@ -525,7 +539,7 @@ def _projection_backward(gemm: str, pairs: list) -> torch.Tensor:
     forward's GEMM."""
     if gemm == "bf16x6" and pairs[0][0].shape[0] > H3_MIN_ROWS:
         ds, ws = zip(*pairs)
-        return gemm_h3(ds, tuple(w.T for w in ws), planes_b=_half_planes(ws, True))
+        return _gemm_h3(ds, tuple(w.T for w in ws), planes_b=_half_planes(ws, True))
     flat = [x for d, w in pairs for x in (d, _transposed(w))]
     if pairs[0][0].shape[0] <= FEW_ROWS and _f32_in_place(*flat[1::2]):
         return gemm_f32(*flat, few_rows=True)
@@ -570,8 +584,8 @@ class _PleFn(torch.autograd.Function):
         elif gemm == "bf16x3":
             key, value = gemm_x3(SplitPlanes(emb32), wk32, cache_b=True, b_n2=wv32)
         elif gemm == "bf16x6" and t_len > H3_MIN_ROWS and not any(ctx.needs_input_grad):
-            key, value = gemm_h3((emb32,), (wk32,), (wv32,), planes_b=_half_planes((wk32,), False),
-                                 planes_b2=_half_planes((wv32,), False))
+            key, value = _gemm_h3((emb32,), (wk32,), (wv32,), planes_b=_half_planes((wk32,), False),
+                                  planes_b2=_half_planes((wv32,), False))
         elif gemm == "bf16x6":
             key, value = gemm_x6(SplitPlanes(emb32, three=True), wk32, cache_b=True, b_n2=wv32)
         else:
